@@ -155,10 +155,13 @@ int lower_score_mods(const pjx_score_mods* mods, FlashArgs& a, const char* who) 
   m.softcap = mods->softcap;
   m.head_scale = mods->head_scales;
   m.constant = mods->constant;
-  const bool full = m.seg_q || m.alibi || m.softcap > 0.f || m.head_scale || m.constant != 0.f;
+  const bool full = m.seg_lt || m.softcap > 0.f || m.head_scale || m.constant != 0.f;
   const bool intervals = m.causal_shift != 0 || m.win_left != kNoBound || m.win_right != kNoBound ||
                          m.prefix || m.seqlen;
-  a.ext = full ? 2 : intervals ? 1 : 0;
+  // 2: segment ids and slopes alone have kernels that skip and trim by segment
+  // and add the slope in two operations (times at ext_segments); whatever
+  // needs a modifier of the score itself, or a key count per row, takes 3.
+  a.ext = full ? 3 : (m.seg_q || m.alibi) ? 2 : intervals ? 1 : 0;
   return PJX_OK;
 }
 

@@ -53,13 +53,14 @@ static int run_bwd_h16(const FlashBwdArgs& a, bool hb, hipStream_t s) {
 
 template <int D, int EXT>
 static int run_bwd_t(const FlashBwdArgs& a, int dtype, bool hb, hipStream_t s) {
-  if (dtype == PJX_DTYPE_F32) return run_bwd_f32<D, EXT>(a, hb, s);
+  if (dtype == PJX_DTYPE_F32) return run_bwd_f32<D, EXT == 2 ? 3 : EXT>(a, hb, s);
   if (dtype == PJX_DTYPE_F16) return run_bwd_h16<F16Fmt, D, EXT>(a, hb, s);
   return run_bwd_h16<Bf16Fmt, D, EXT>(a, hb, s);
 }
 
 template <int D>
 static int run_bwd(const FlashBwdArgs& a, int dtype, bool hb, hipStream_t s) {
+  if (a.f.ext == 3) return run_bwd_t<D, 3>(a, dtype, hb, s);
   if (a.f.ext == 2) return run_bwd_t<D, 2>(a, dtype, hb, s);
   return a.f.ext == 1 ? run_bwd_t<D, 1>(a, dtype, hb, s) : run_bwd_t<D, 0>(a, dtype, hb, s);
 }

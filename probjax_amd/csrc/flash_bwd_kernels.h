@@ -228,9 +228,11 @@ __global__ __launch_bounds__(NG * kThreads, (D <= 128 ? 2 : 1)) void flash_bwd_d
            (size_t)(row_in ? g.qi : 0) * a.Lk;
   }
   const bool bias_vec = (a.Lk & 3) == 0;
-  const float cx = (HB || EXT == 2) ? kLog2e : a.scale * kLog2e;
+  const bool natural = HB || EXT == 3 || (EXT == 2 && a.m.alibi != nullptr);
+  const float cx = natural ? kLog2e : a.scale * kLog2e;
   ExtRows er;
   if constexpr (EXT > 0) er = ext_rows(a, g);
+  if constexpr (EXT == 2) ext_segments(a, g, er, BK, (int*)smem0);
 
   uint32_t voff[T::NLD];
 #pragma unroll
@@ -263,12 +265,26 @@ __global__ __launch_bounds__(NG * kThreads, (D <= 128 ? 2 : 1)) void flash_bwd_d
     }
   };
 
-  auto compute = [&](int t, const unsigned char* ks) {
+  // Level 2: the segment id of key k0 + lane of the tile loaded next.
+  int seg_next = 0;
+  auto fetch_seg = [&](int t) {
+    if constexpr (EXT == 2) {
+      const int kk = (t_begin + t) * BK + lane;
+      if (a.m.seg_k && kk < g.kv_end) seg_next = a.m.seg_k[(size_t)g.b * a.Lk + kk];
+    }
+  };
+
+  auto compute = [&](int t, const unsigned char* ks, int seg_id) {
     const int k0 = (t_begin + t) * BK;
     if constexpr (EXT > 0) {
       if (!er.any || k0 > er.hi_last || k0 + BK - 1 < er.lo_first) return;
     } else {
       if (a.causal && k0 > q_last_w) return;  // tile above this wave's diagonal
+    }
+    SegTile seg = kSegWhole;
+    if constexpr (EXT == 2) {
+      if (a.m.seg_k) seg = seg_tile(seg_id, k0 + lane < g.kv_end, er.seg_lo, er.seg_hi);
+      if (seg == kSegSkip) return;
     }
     const unsigned char* vs = ks + TILE_B;
 
@@ -292,7 +308,7 @@ __global__ __launch_bounds__(NG * kThreads, (D <= 128 ? 2 : 1)) void flash_bwd_d
     }
     PJX_SCHED_LDS_READS_AHEAD(2 * (D / 16) * (BK / 32), 3, 1);  // K / V fragments 3 MFMAs ahead
     f32x16 dbv[DB ? BK / 32 : 1];  // dL/d(bias) = P (dP - delta), kept for the store
-    if constexpr (EXT == 2) {
+    if constexpr (EXT == 3) {
       // modified scores, masks, P and dS = P (dP - delta) * scale * f'(s)
       ext_scores_sT<BK / 32, HB>(a, g, er, s, k0, half, brow, row_in,
                                  [&](int kb, int r, float x, float gg) {
@@ -314,7 +330,11 @@ __global__ __launch_bounds__(NG * kThreads, (D <= 128 ? 2 : 1)) void flash_bwd_d
           for (int j = 0; j < 4; ++j) s[kb][4 * gq + j] = fmaf(s[kb][4 * gq + j], a.scale, bv[j]);
         }
     }
-    if constexpr (EXT == 1) ext_mask_sT<BK / 32>(g, er, s, k0, half);
+    if constexpr (EXT == 2) {
+      if (a.m.alibi) ext_slope_sT<BK / 32, HB>(a, g, er, s, k0, half);
+      if (seg == kSegMixed) ext_seg_mask_sT<BK / 32>(a, g, er, s, k0, half);
+    }
+    if constexpr (EXT == 1 || EXT == 2) ext_mask_sT<BK / 32>(g, er, s, k0, half);
     const bool need_mask = EXT == 0 && ((k0 + BK > g.kv_end) || (a.causal && k0 + BK - 1 > g.qw) ||
                                         (g.qw + 31 >= g.q_hi));
     if (need_mask) {
@@ -359,17 +379,23 @@ __global__ __launch_bounds__(NG * kThreads, (D <= 128 ? 2 : 1)) void flash_bwd_d
   // group) keeps the barriers in step
   const int n_loc = (n_tiles - gi + NG - 1) / NG;
   const int n_steps = (n_tiles + NG - 1) / NG;
-  if (n_loc > 0) issue(gi, st0);
+  auto load = [&](int s, unsigned char* st) {
+    issue(NG * s + gi, st);
+    fetch_seg(NG * s + gi);
+  };
+  if (n_loc > 0) load(0, st0);
   for (int s = 0; s < n_steps; s += 2) {
     __builtin_amdgcn_s_waitcnt(0);
     __syncthreads();
-    if (s + 1 < n_loc) issue(NG * (s + 1) + gi, st1);
-    if (s < n_loc) compute(NG * s + gi, smem0);
+    const int seg0 = seg_next;
+    if (s + 1 < n_loc) load(s + 1, st1);
+    if (s < n_loc) compute(NG * s + gi, smem0, seg0);
     if (s + 1 >= n_steps) break;
     __builtin_amdgcn_s_waitcnt(0);
     __syncthreads();
-    if (s + 2 < n_loc) issue(NG * (s + 2) + gi, st0);
-    if (s + 1 < n_loc) compute(NG * (s + 1) + gi, smem1);
+    const int seg1 = seg_next;
+    if (s + 2 < n_loc) load(s + 2, st0);
+    if (s + 1 < n_loc) compute(NG * (s + 1) + gi, smem1, seg1);
   }
   if constexpr (NG > 1) {
     // Group 1 hands its dQ^T sums to group 0 through LDS, lane by lane in the
@@ -470,6 +496,17 @@ __global__ __launch_bounds__(NG * kThreads, (D <= 128 ? 2 : 1)) void flash_bwd_d
     }
     if (a.m.seg_k && key < a.Lk) segk = a.m.seg_k[(size_t)b * a.Lk + key];
   }
+  // Level 2: the wave's id range, and the workgroup's query range narrowed to
+  // the documents its keys belong to.
+  int seg_lo = 0, seg_hi = 0;
+  if constexpr (EXT == 2) {
+    if (a.m.seg_k && k0 < kv_end) {
+      seg_range(a.m.seg_k, b, a.Lk, kw, 32, kv_end, seg_lo, seg_hi);
+      int lo, hi;
+      seg_range(a.m.seg_k, b, a.Lk, k0, kBKV, kv_end, lo, hi);
+      seg_narrow(a.m.seg_q, b, a.Lq, lo, hi, (int*)smem0, q_begin, q_end);
+    }
+  }
   const int n_qt = (k0 < kv_end && q_end > q_begin) ? (q_end - q_begin + kBQs - 1) / kBQs : 0;
   const int n_tiles = G * n_qt;
 
@@ -491,7 +528,8 @@ __global__ __launch_bounds__(NG * kThreads, (D <= 128 ? 2 : 1)) void flash_bwd_d
       vf[s] = E::as8(rv);
     }
   }
-  const float cx = (BIAS || EXT == 2) ? kLog2e : a.scale * kLog2e;
+  const bool natural = BIAS || EXT == 3 || (EXT == 2 && a.m.alibi != nullptr);
+  const float cx = natural ? kLog2e : a.scale * kLog2e;
   const uint32_t rowstride = (uint32_t)a.Hq * D * 2;
 
   uint32_t voff[T::NLD];
@@ -538,7 +576,16 @@ __global__ __launch_bounds__(NG * kThreads, (D <= 128 ? 2 : 1)) void flash_bwd_d
     buffer_load_lds4(rdl, small + kBQs * 4, 4 * lane);
   };
 
-  auto compute = [&](int t, const unsigned char* st) {
+  // Level 2: the segment id of query q0 + lane of the stage loaded next.
+  int seg_next = 0;
+  auto fetch_seg = [&](int t) {
+    if constexpr (EXT == 2) {
+      const int qq = tile_q0(t) + lane;
+      if (a.m.seg_k && qq < q_hi) seg_next = a.m.seg_q[(size_t)b * a.Lq + qq];
+    }
+  };
+
+  auto compute = [&](int t, const unsigned char* st, int seg_id) {
     const int h = tile_head(t), q0 = tile_q0(t);
     const unsigned char* qs = st;
     const unsigned char* dos = st + TILE_B;
@@ -553,7 +600,7 @@ __global__ __launch_bounds__(NG * kThreads, (D <= 128 ? 2 : 1)) void flash_bwd_d
       if constexpr (EXT > 0) {
         if (qs0 > wq_last || qs0 + 31 < wq_first) continue;  // no row of this step sees the wave's keys
       }
-      if constexpr (EXT == 2) {
+      if constexpr (EXT == 3) {
         // S = Q K^T and dP = dO V^T first, then one pass: modified score,
         // mask, P and dS = P (dP - delta) * scale * f'(s).
         f32x16 sx = f32x16{}, dpx = f32x16{};
@@ -587,6 +634,12 @@ __global__ __launch_bounds__(NG * kThreads, (D <= 128 ? 2 : 1)) void flash_bwd_d
         }
         continue;
       }
+      SegTile seg = kSegWhole;
+      if constexpr (EXT == 2) {
+        if (a.m.seg_k)
+          seg = seg_tile(seg_id, (lane >> 5) == qb && q0 + lane < q_hi, seg_lo, seg_hi);
+        if (seg == kSegSkip) continue;
+      }
       if (EXT == 0 && a.causal && qs0 + 31 < kw) continue;  // every query before this wave's first key
 
       // S[query][key] = Q K^T: register r holds query qs0 + 8*(r/4) + 4*half + r%4
@@ -605,7 +658,11 @@ __global__ __launch_bounds__(NG * kThreads, (D <= 128 ? 2 : 1)) void flash_bwd_d
           s[r] = fmaf(s[r], a.scale, bv);
         }
       }
-      if constexpr (EXT == 1)
+      if constexpr (EXT == 2) {
+        if (a.m.alibi) ext_slope_S<BIAS>(a, a.m.alibi[h], s, key, kw + 31, qs0, half);
+        if (seg == kSegMixed) ext_seg_mask_S(a, b, segk, s, qs0, half);
+      }
+      if constexpr (EXT == 1 || EXT == 2)
         ext_mask_S(s, qs0, half, qlo, qhi, !(kw + 31 < kv_end && qs0 >= qlo_last && qs0 + 31 <= qhi_first));
       const bool need_mask = EXT == 0 && ((a.causal && qs0 < kw + 31) || (kw + 32 > kv_end) || (qs0 + 32 > q_hi));
       if (need_mask) {
@@ -657,17 +714,23 @@ __global__ __launch_bounds__(NG * kThreads, (D <= 128 ? 2 : 1)) void flash_bwd_d
   // group) keeps the barriers in step
   const int n_loc = (n_tiles - gi + NG - 1) / NG;
   const int n_steps = (n_tiles + NG - 1) / NG;
-  if (n_loc > 0) issue(gi, st0);
+  auto load = [&](int s, unsigned char* st) {
+    issue(NG * s + gi, st);
+    fetch_seg(NG * s + gi);
+  };
+  if (n_loc > 0) load(0, st0);
   for (int s = 0; s < n_steps; s += 2) {
     __builtin_amdgcn_s_waitcnt(0);
     __syncthreads();
-    if (s + 1 < n_loc) issue(NG * (s + 1) + gi, st1);
-    if (s < n_loc) compute(NG * s + gi, smem0);
+    const int seg0 = seg_next;
+    if (s + 1 < n_loc) load(s + 1, st1);
+    if (s < n_loc) compute(NG * s + gi, smem0, seg0);
     if (s + 1 >= n_steps) break;
     __builtin_amdgcn_s_waitcnt(0);
     __syncthreads();
-    if (s + 2 < n_loc) issue(NG * (s + 2) + gi, st0);
-    if (s + 1 < n_loc) compute(NG * (s + 1) + gi, smem1);
+    const int seg1 = seg_next;
+    if (s + 2 < n_loc) load(s + 2, st0);
+    if (s + 1 < n_loc) compute(NG * (s + 1) + gi, smem1, seg1);
   }
   if constexpr (NG > 1) {
     // Group 1 hands its dK^T / dV^T sums to group 0 through LDS, lane by lane
@@ -794,7 +857,7 @@ __global__ __launch_bounds__(kThreads, 1) void flash_bwd_dq_f32_kernel(FlashBwdA
            (size_t)(row_in ? g.qi : 0) * a.Lk;
   }
   const bool bias_vec = (a.Lk & 3) == 0;
-  const float cx = (HB || EXT == 2) ? kLog2e : a.scale * kLog2e;
+  const float cx = (HB || EXT == 3) ? kLog2e : a.scale * kLog2e;
   ExtRows er;
   if constexpr (EXT > 0) er = ext_rows(a, g);
 
@@ -858,7 +921,7 @@ __global__ __launch_bounds__(kThreads, 1) void flash_bwd_dq_f32_kernel(FlashBwdA
       }
     }
     f32x16 dbv[DB ? BK / 32 : 1];
-    if constexpr (EXT == 2) {
+    if constexpr (EXT == 3) {
       ext_scores_sT<BK / 32, HB>(a, g, er, s, k0, half, brow, row_in,
                                  [&](int kb, int r, float x, float gg) {
                                    const float p = fast_exp2(fmaf(x, cx, -lse2));
@@ -1013,7 +1076,7 @@ __global__ __launch_bounds__(kThreads, 1) void flash_bwd_dkdv_f32_kernel(FlashBw
       }
     }
   }
-  const float cx = (BIAS || EXT == 2) ? kLog2e : a.scale * kLog2e;
+  const float cx = (BIAS || EXT == 3) ? kLog2e : a.scale * kLog2e;
   const size_t q_row = (size_t)a.Hq * D;
 
   f32x16 acck[D / 32], accv[D / 32];
@@ -1090,7 +1153,7 @@ __global__ __launch_bounds__(kThreads, 1) void flash_bwd_dkdv_f32_kernel(FlashBw
       }
     }
     f32x16 ds;
-    if constexpr (EXT == 2) {
+    if constexpr (EXT == 3) {
       const float* bbase = nullptr;
       if constexpr (BIAS) bbase = a.bias + (size_t)b * a.bias_bstride + (size_t)h * a.bias_hstride;
       const HeadMods hm = head_mods(a.m, h);

@@ -24,7 +24,7 @@ struct FlashArgs {
   float scale;
   int n_qtiles;
   int dv;       // output row width (elements per head); the wide kernels' V width
-  int ext;      // 0: none; 1: interval masks in `m`; 2: also segment ids / score modifiers
+  int ext;      // 0: none; 1: interval masks in `m`; 2: also segment ids / distance slopes; 3: all of `m`
   int f16;      // 16-bit inputs are fp16 (else bf16); read by the host-side launchers only
   ScoreMods m;
 };
@@ -100,8 +100,77 @@ struct ExtRows {
   int lo_last, hi_last;    // interval of the wave's last existing row
   bool any;            // the wave has a row < q_hi
   int segq;            // this row's segment id
+  int seg_lo, seg_hi;  // smallest and largest id of the wave's rows (segment ids, level 2)
   HeadMods hm;
 };
+
+// Smallest and largest value over a wave's lanes, the same in every lane.
+__device__ __forceinline__ int wave_min(int x) {
+#pragma unroll
+  for (int m = 1; m < 64; m <<= 1) x = min(x, __shfl_xor(x, m, 64));
+  return __builtin_amdgcn_readfirstlane(x);
+}
+__device__ __forceinline__ int wave_max(int x) {
+#pragma unroll
+  for (int m = 1; m < 64; m <<= 1) x = max(x, __shfl_xor(x, m, 64));
+  return __builtin_amdgcn_readfirstlane(x);
+}
+
+// Smallest and largest segment id of positions [p0, min(p0 + n, end)) of batch
+// b in ids [B, L], the same in every lane (lo > hi: no position).
+__device__ __forceinline__ void seg_range(const int32_t* ids, int b, int L, int p0, int n, int end, int& lo,
+                                          int& hi) {
+  lo = 0x7fffffff;
+  hi = -0x7fffffff - 1;
+  const int lane = threadIdx.x & 63;
+  for (int p = p0 + lane; p < min(p0 + n, end); p += 64) {
+    const int id = ids[(size_t)b * L + p];
+    lo = min(lo, id);
+    hi = max(hi, id);
+  }
+  lo = wave_min(lo);
+  hi = wave_max(hi);
+}
+
+// Narrows [begin, end) of batch b's positions to the first and last one whose
+// id lies in [lo, hi] (empty: begin == end).  Rows of packed documents see
+// only their own document's keys, so a workgroup whose rows hold documents
+// lo .. hi need not load any key outside the range found here; it stays exact
+// for ids in any order, since keys between are still compared one by one.
+// Every thread of the workgroup calls it; `sm` holds 2 ints.
+__device__ __forceinline__ void seg_narrow(const int32_t* ids, int b, int L, int lo, int hi, int* sm, int& begin,
+                                           int& end) {
+  if (threadIdx.x == 0) {
+    sm[0] = 0x7fffffff;
+    sm[1] = -1;
+  }
+  __syncthreads();
+  int first = 0x7fffffff, last = -1;
+#pragma unroll 4
+  for (int p = begin + (int)threadIdx.x; p < end; p += (int)blockDim.x) {
+    const int id = ids[(size_t)b * L + p];
+    if (id >= lo && id <= hi) {
+      first = min(first, p);
+      last = p;
+    }
+  }
+  first = wave_min(first);
+  last = wave_max(last);
+  if ((threadIdx.x & 63) == 0) {
+    atomicMin(&sm[0], first);
+    atomicMax(&sm[1], last);
+  }
+  __syncthreads();
+  first = __builtin_amdgcn_readfirstlane(sm[0]);
+  last = __builtin_amdgcn_readfirstlane(sm[1]);
+  __syncthreads();
+  if (last < 0) {
+    end = begin;
+  } else {
+    begin = first;
+    end = last + 1;
+  }
+}
 
 __device__ __forceinline__ ExtRows ext_rows(const FlashArgs& a, const BlockGeom& g) {
   ExtRows e;
@@ -111,8 +180,29 @@ __device__ __forceinline__ ExtRows ext_rows(const FlashArgs& a, const BlockGeom&
   row_bounds(a.m, a.causal, g.b, g.kv_end, g.q_hi, g.qw, e.lo_first, e.hi_first);
   row_bounds(a.m, a.causal, g.b, g.kv_end, g.q_hi, ql, e.lo_last, e.hi_last);
   e.segq = (a.m.seg_q && g.qi < a.Lq) ? a.m.seg_q[(size_t)g.b * a.Lq + g.qi] : 0;
+  e.seg_lo = e.seg_hi = 0;
   e.hm = head_mods(a.m, g.h);
   return e;
+}
+
+// Level 2 (segment ids compared for equality, distance slopes): the wave's id
+// range in `er`, and the workgroup's key range narrowed to the documents its
+// rows belong to.  The general level (3) visits every tile of the interval,
+// compares ids per score and spends ~14 vector operations a score on modifiers
+// that are absent; with packed documents most of its tiles are masked whole.
+// Finding the range costs one 4-byte read per key (K and V take 256 or more).
+// Measured, forward + backward: 6 packed documents, bf16 B=2 H=16 L=2048
+// D=128, 707 -> 193 us; causal slopes, bf16 B=2 H=12 L=1024 D=64, the three
+// kernels 168 -> 91 us.
+__device__ __forceinline__ void ext_segments(const FlashArgs& a, BlockGeom& g, ExtRows& er, int tile, int* sm) {
+  if (!a.m.seg_k) return;
+  seg_range(a.m.seg_q, g.b, a.Lq, g.qw, 32, g.q_hi, er.seg_lo, er.seg_hi);
+  int lo, hi;
+  seg_range(a.m.seg_q, g.b, a.Lq, g.q0, kBQ, g.q_hi, lo, hi);
+  int begin = g.kv_begin, end = g.kv_stop;
+  seg_narrow(a.m.seg_k, g.b, a.Lk, lo, hi, sm, begin, end);
+  g.kv_begin = (begin / tile) * tile;
+  g.kv_stop = end;
 }
 
 // Segment ids of 4 consecutive positions kk .. kk+3 (kk a multiple of 4) of
@@ -310,6 +400,92 @@ __device__ __forceinline__ void ext_scores_S_t(const FlashArgs& a, int b, const 
       emit(r, keep ? x : -INFINITY, gg);
     }
     __builtin_amdgcn_sched_barrier(0);
+  }
+}
+
+// Level 2 in the S^T layout.  Distance slopes: s (already sm_scale * q.k
+// [+ bias] when SCALED) becomes sm_scale * q.k [+ bias] - slope * f(q - k),
+// f = max(., 0) or |.|.  Where every row of the wave is at or past the tile's
+// last key, f(q - k) = q - k: two fused multiply-adds per score.
+template <int NKB, bool SCALED>
+__device__ __forceinline__ void ext_slope_sT(const FlashArgs& a, const BlockGeom& g, const ExtRows& er, f32x16* s,
+                                             int k0, int half) {
+  const float sc = SCALED ? 1.f : a.scale;
+  const float d0 = (float)(g.qi - (k0 + 4 * half));
+  if (g.qw >= k0 + NKB * 32 - 1) {
+    const float t0 = -er.hm.slope * d0;
+#pragma unroll
+    for (int kb = 0; kb < NKB; ++kb)
+#pragma unroll
+      for (int r = 0; r < 16; ++r)
+        s[kb][r] = fmaf(s[kb][r], sc, fmaf(er.hm.slope, (float)(kb * 32 + 8 * (r >> 2) + (r & 3)), t0));
+  } else {
+    const float neg = a.m.alibi_sym ? -1.f : 0.f;
+#pragma unroll
+    for (int kb = 0; kb < NKB; ++kb)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        const float d = d0 - (float)(kb * 32 + 8 * (r >> 2) + (r & 3));
+        s[kb][r] = fmaf(s[kb][r], sc, -er.hm.slope * fmaxf(d, neg * d));
+      }
+  }
+}
+
+// Segment ids of a tile that may hold keys of another segment: scores of keys
+// whose id differs from the row's become -inf.
+template <int NKB>
+__device__ __forceinline__ void ext_seg_mask_sT(const FlashArgs& a, const BlockGeom& g, const ExtRows& er, f32x16* s,
+                                                int k0, int half) {
+#pragma unroll
+  for (int kb = 0; kb < NKB; ++kb)
+#pragma unroll
+    for (int gq = 0; gq < 4; ++gq) {
+      const int4 sg = seg4(a.m.seg_k, g.b, k0 + kb * 32 + 8 * gq + 4 * half, a.Lk);
+      const int sgv[4] = {sg.x, sg.y, sg.z, sg.w};
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        if (sgv[j] != er.segq) s[kb][4 * gq + j] = -INFINITY;
+    }
+}
+
+// What a wave does with a 64-key tile whose id of key k0 + lane is `id`:
+// skip it (no key of its rows' segments), take it without comparing ids (one
+// segment on both sides), or compare.
+enum SegTile { kSegSkip, kSegWhole, kSegMixed };
+__device__ __forceinline__ SegTile seg_tile(int id, bool in, int lo, int hi) {
+  if (!wave_any(in && id >= lo && id <= hi)) return kSegSkip;
+  return lo == hi && !wave_any(in && id != lo) ? kSegWhole : kSegMixed;
+}
+
+// The same two in the S layout (lane = key, register r = query qs0 +
+// 8*(r/4) + 4*half + r%4).
+template <bool SCALED>
+__device__ __forceinline__ void ext_slope_S(const FlashArgs& a, float slope, f32x16& s, int key, int key_last, int qs0,
+                                            int half) {
+  const float sc = SCALED ? 1.f : a.scale;
+  const float d0 = (float)(qs0 + 4 * half - key);
+  if (qs0 >= key_last) {
+    const float t0 = -slope * d0;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) s[r] = fmaf(s[r], sc, fmaf(-slope, (float)(8 * (r >> 2) + (r & 3)), t0));
+  } else {
+    const float neg = a.m.alibi_sym ? -1.f : 0.f;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+      const float d = d0 + (float)(8 * (r >> 2) + (r & 3));
+      s[r] = fmaf(s[r], sc, -slope * fmaxf(d, neg * d));
+    }
+  }
+}
+
+__device__ __forceinline__ void ext_seg_mask_S(const FlashArgs& a, int b, int segk, f32x16& s, int qs0, int half) {
+#pragma unroll
+  for (int gq = 0; gq < 4; ++gq) {
+    const int4 sg = seg4(a.m.seg_q, b, qs0 + 8 * gq + 4 * half, a.Lq);
+    const int sgv[4] = {sg.x, sg.y, sg.z, sg.w};
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      if (sgv[j] != segk) s[4 * gq + j] = -INFINITY;
   }
 }
 

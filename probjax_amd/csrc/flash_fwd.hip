@@ -105,9 +105,11 @@ __global__ __launch_bounds__(kThreads, 2) void flash_fwd_bf16_kernel(FlashArgs a
   const bool bias_vec = (a.Lk & 3) == 0;
   // score units -> log2 units (the scale is applied to the score itself when
   // a bias or modifier is added to it)
-  const float cx = (BIAS || EXT == 2) ? kLog2e : a.scale * kLog2e;
+  const bool natural = BIAS || EXT == 3 || (EXT == 2 && a.m.alibi != nullptr);
+  const float cx = natural ? kLog2e : a.scale * kLog2e;
   ExtRows er;
   if constexpr (EXT > 0) er = ext_rows(a, g);
+  if constexpr (EXT == 2) ext_segments(a, g, er, BK, (int*)smem0);
 
   // Per-lane byte offsets, fixed for the whole key loop.
   uint32_t voffK[T::NLD], voffV[T::NLD];
@@ -154,13 +156,28 @@ __global__ __launch_bounds__(kThreads, 2) void flash_fwd_bf16_kernel(FlashArgs a
     }
   };
 
-  auto compute = [&](int t, const unsigned char* ks) {
+  // Level 2: the segment id of key k0 + lane of the tile loaded next, fetched
+  // with it.
+  int seg_next = 0;
+  auto fetch_seg = [&](int t) {
+    if constexpr (EXT == 2) {
+      const int kk = (t_begin + t) * BK + lane;
+      if (a.m.seg_k && kk < g.kv_end) seg_next = a.m.seg_k[(size_t)g.b * a.Lk + kk];
+    }
+  };
+
+  auto compute = [&](int t, const unsigned char* ks, int seg_id) {
     const int k0 = (t_begin + t) * BK;
     if constexpr (EXT > 0) {
       // tile outside every row of this wave
       if (!er.any || k0 > er.hi_last || k0 + BK - 1 < er.lo_first) return;
     } else {
       if (a.causal && k0 > q_last_w) return;  // tile above this wave's diagonal
+    }
+    SegTile seg = kSegWhole;
+    if constexpr (EXT == 2) {
+      if (a.m.seg_k) seg = seg_tile(seg_id, k0 + lane < g.kv_end, er.seg_lo, er.seg_hi);
+      if (seg == kSegSkip) return;
     }
     const unsigned char* vs = ks + TILE_B;
 
@@ -177,7 +194,7 @@ __global__ __launch_bounds__(kThreads, 2) void flash_fwd_bf16_kernel(FlashArgs a
     }
 
     // Register r of block kb holds key k0 + kb*32 + 8*(r/4) + 4*half + r%4.
-    if constexpr (EXT == 2) {
+    if constexpr (EXT == 3) {
       ext_scores_sT<BK / 32, BIAS>(a, g, er, s, k0, half, brow, row_in,
                                    [&](int kb, int r, float x, float) { s[kb][r] = x; });
     } else if constexpr (BIAS) {
@@ -193,7 +210,11 @@ __global__ __launch_bounds__(kThreads, 2) void flash_fwd_bf16_kernel(FlashArgs a
         }
       }
     }
-    if constexpr (EXT == 1) ext_mask_sT<BK / 32>(g, er, s, k0, half);
+    if constexpr (EXT == 2) {
+      if (a.m.alibi) ext_slope_sT<BK / 32, BIAS>(a, g, er, s, k0, half);
+      if (seg == kSegMixed) ext_seg_mask_sT<BK / 32>(a, g, er, s, k0, half);
+    }
+    if constexpr (EXT == 1 || EXT == 2) ext_mask_sT<BK / 32>(g, er, s, k0, half);
     const bool need_mask = EXT == 0 && ((k0 + BK > g.kv_end) || (a.causal && k0 + BK - 1 > g.qw) ||
                                         (g.qw + 31 >= g.q_hi));
     if (need_mask) {
@@ -265,17 +286,28 @@ __global__ __launch_bounds__(kThreads, 2) void flash_fwd_bf16_kernel(FlashArgs a
   // tile t have landed (waitcnt), then every wave's have and every wave is done
   // reading the other stage (barrier), so tile t+1's loads can go there while
   // tile t is computed.
-  if (n_tiles > 0) issue(0, smem0);
+  if (n_tiles > 0) {
+    issue(0, smem0);
+    fetch_seg(0);
+  }
   for (int t = 0; t < n_tiles; t += 2) {
     __builtin_amdgcn_s_waitcnt(0);
     __syncthreads();
-    if (t + 1 < n_tiles) issue(t + 1, smem1);
-    compute(t, smem0);
+    const int seg0 = seg_next;
+    if (t + 1 < n_tiles) {
+      issue(t + 1, smem1);
+      fetch_seg(t + 1);
+    }
+    compute(t, smem0, seg0);
     if (t + 1 >= n_tiles) break;
     __builtin_amdgcn_s_waitcnt(0);
     __syncthreads();
-    if (t + 2 < n_tiles) issue(t + 2, smem0);
-    compute(t + 1, smem1);
+    const int seg1 = seg_next;
+    if (t + 2 < n_tiles) {
+      issue(t + 2, smem0);
+      fetch_seg(t + 2);
+    }
+    compute(t + 1, smem1, seg1);
   }
 
   const float l_tot = xor32_sum(l_run);
@@ -636,7 +668,7 @@ __global__ __launch_bounds__(kThreads, 1) void flash_fwd_f32_kernel(FlashArgs a)
            (size_t)(row_in ? g.qi : 0) * a.Lk;
   }
   const bool bias_vec = (a.Lk & 3) == 0;
-  const float cx = (BIAS || EXT == 2) ? kLog2e : a.scale * kLog2e;
+  const float cx = (BIAS || EXT == 3) ? kLog2e : a.scale * kLog2e;
   ExtRows er;
   if constexpr (EXT > 0) er = ext_rows(a, g);
 
@@ -694,7 +726,7 @@ __global__ __launch_bounds__(kThreads, 1) void flash_fwd_f32_kernel(FlashArgs a)
         for (int j = 0; j < 4; ++j) s[kb] = mfma32x32x2f32(kf[j], qf[4 * st4 + j], s[kb]);
       }
     }
-    if constexpr (EXT == 2) {
+    if constexpr (EXT == 3) {
       ext_scores_sT<BK / 32, BIAS>(a, g, er, s, k0, half, brow, row_in,
                                    [&](int kb, int r, float x, float) { s[kb][r] = x; });
     } else if constexpr (BIAS) {
@@ -1003,20 +1035,24 @@ static int launch_pipe128(const FlashArgs& a, hipStream_t stream) {
   return launch<flash_fwd_bf16_pipe_kernel<E, 128, 32, 3>>(a, stream);
 }
 
+// The one-pass kernel with extended masks.
+template <typename E, int EXT>
+static int launch_ext(const FlashArgs& a, int head_dim, hipStream_t s) {
+  const bool hb = a.bias != nullptr;
+  if (head_dim == 128)
+    return hb ? launch<flash_fwd_bf16_kernel<E, 128, true, EXT>>(a, s) : launch<flash_fwd_bf16_kernel<E, 128, false, EXT>>(a, s);
+  return hb ? launch<flash_fwd_bf16_kernel<E, 64, true, EXT>>(a, s) : launch<flash_fwd_bf16_kernel<E, 64, false, EXT>>(a, s);
+}
+
 // The 16-bit kernels (bf16 or fp16 operands, format E) for head_dim 64 / 128.
 template <typename E>
 static int launch_h16(const FlashArgs& a, int head_dim, hipStream_t s) {
   const bool hb = a.bias != nullptr;
   if (a.ext) {
     // Extended masks / score modifiers: the one-pass kernel's EXT variants
-    // (1: interval masks, 2: segment ids / score modifiers as well).
-    const bool full = a.ext == 2;
-    if (head_dim == 128) {
-      if (full) return hb ? launch<flash_fwd_bf16_kernel<E, 128, true, 2>>(a, s) : launch<flash_fwd_bf16_kernel<E, 128, false, 2>>(a, s);
-      return hb ? launch<flash_fwd_bf16_kernel<E, 128, true, 1>>(a, s) : launch<flash_fwd_bf16_kernel<E, 128, false, 1>>(a, s);
-    }
-    if (full) return hb ? launch<flash_fwd_bf16_kernel<E, 64, true, 2>>(a, s) : launch<flash_fwd_bf16_kernel<E, 64, false, 2>>(a, s);
-    return hb ? launch<flash_fwd_bf16_kernel<E, 64, true, 1>>(a, s) : launch<flash_fwd_bf16_kernel<E, 64, false, 1>>(a, s);
+    // (1: interval masks, 2: segment ids and distance slopes as well, 3: all).
+    if (a.ext == 1) return launch_ext<E, 1>(a, head_dim, s);
+    return a.ext == 2 ? launch_ext<E, 2>(a, head_dim, s) : launch_ext<E, 3>(a, head_dim, s);
   }
   // Dense bias with 16-byte aligned rows and 32-bit slice offsets: the LDS
   // ring that streams the bias; otherwise bias loads into registers.
@@ -1138,12 +1174,12 @@ extern "C" int pjx_flash_fwd(int dtype, const void* q, const void* k, const void
   if (dtype == PJX_DTYPE_BF16) return launch_h16<Bf16Fmt>(a, (int)head_dim, s);
   if (dtype == PJX_DTYPE_F16) return launch_h16<F16Fmt>(a, (int)head_dim, s);
   if (a.ext) {
-    const bool full = a.ext == 2;
+    const bool full = a.ext >= 2;
     if (head_dim == 128) {
-      if (full) return hb ? launch<flash_fwd_f32_kernel<128, true, 2>>(a, s) : launch<flash_fwd_f32_kernel<128, false, 2>>(a, s);
+      if (full) return hb ? launch<flash_fwd_f32_kernel<128, true, 3>>(a, s) : launch<flash_fwd_f32_kernel<128, false, 3>>(a, s);
       return hb ? launch<flash_fwd_f32_kernel<128, true, 1>>(a, s) : launch<flash_fwd_f32_kernel<128, false, 1>>(a, s);
     }
-    if (full) return hb ? launch<flash_fwd_f32_kernel<64, true, 2>>(a, s) : launch<flash_fwd_f32_kernel<64, false, 2>>(a, s);
+    if (full) return hb ? launch<flash_fwd_f32_kernel<64, true, 3>>(a, s) : launch<flash_fwd_f32_kernel<64, false, 3>>(a, s);
     return hb ? launch<flash_fwd_f32_kernel<64, true, 1>>(a, s) : launch<flash_fwd_f32_kernel<64, false, 1>>(a, s);
   }
   // fp32 with fewer 128-row workgroups than CUs: split each query block's
