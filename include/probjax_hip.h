@@ -175,6 +175,18 @@ size_t pjx_flash_bwd_ds_workspace_size(int dtype, int64_t batch, int64_t q_heads
                                        int64_t kv_len, int64_t head_dim);
 
 /*
+ * Bytes of workspace with which pjx_flash_bwd spreads each key block's part of
+ * dK and dV over several workgroups, or 0 where it does not: 16-bit inputs at
+ * head_dim 64 or 128 whose key blocks are too few to keep the device busy.
+ * Size: pjx_flash_bwd_workspace_size() rounded up to 256 bytes, plus one fp32
+ * dK and dV per split (a power of two up to 8, a function of the sizes only).
+ * The partials are added in split order, so results are deterministic; they
+ * differ from the smaller workspace's by the order of an fp32 sum.
+ */
+size_t pjx_flash_bwd_split_workspace_size(int dtype, int64_t batch, int64_t q_heads, int64_t kv_heads,
+                                          int64_t q_len, int64_t kv_len, int64_t head_dim, int causal);
+
+/*
  * Flash-attention backward: dq, dk, dv of pjx_flash_fwd's output.  Replaces
  * the Pallas backward of `mha` (probjax/nn/pallas_kernels/kernels/
  * attention.py: _preprocess_backward_kernel 853-867, mha_backward_kernel
@@ -199,7 +211,8 @@ size_t pjx_flash_bwd_ds_workspace_size(int dtype, int64_t batch, int64_t q_heads
  * (fully written, zeros where no valid score reaches).  workspace: at least
  * pjx_flash_bwd_workspace_size(batch, q_heads, q_len) bytes.  mods: the
  * forward's (pjx_score_mods) or NULL.  A workspace of at least
- * pjx_flash_bwd_ds_workspace_size() bytes selects the dS route where it applies.
+ * pjx_flash_bwd_ds_workspace_size() bytes selects the dS route where it applies,
+ * one of pjx_flash_bwd_split_workspace_size() bytes the split key blocks.
  * dtype: PJX_DTYPE_BF16, PJX_DTYPE_F16 or PJX_DTYPE_F32 (all fp32 products, no
  * roundings).  head_dim in {64, 128, 256}.
  */

@@ -22,6 +22,43 @@ static int run_bwd_f32(const FlashBwdArgs& a, bool hb, hipStream_t s) {
             : launch_dkdv<flash_bwd_dkdv_f32_kernel<D, false, EXT>>(a, s);
 }
 
+// out = the sum over splits of dK (blockIdx.y 0) or dV (1), in split order,
+// rounded to 16 bits; n elements of each (a multiple of 4).  Bound by the
+// partials' traffic.
+template <typename E>
+__global__ __launch_bounds__(kThreads) void bwd_split_reduce_kernel(const float* part, int nsplit, size_t n,
+                                                                    uint16_t* dk, uint16_t* dv) {
+  const size_t e = 4 * ((size_t)blockIdx.x * kThreads + threadIdx.x);
+  if (e >= n) return;
+  const float* p = part + (size_t)blockIdx.y * nsplit * n + e;
+  f32x4 acc = *(const f32x4*)p;
+  for (int s = 1; s < nsplit; ++s) acc += *(const f32x4*)(p + s * n);
+  *(u32x2*)((blockIdx.y ? dv : dk) + e) = u32x2{E::pack2(acc[0], acc[1]), E::pack2(acc[2], acc[3])};
+}
+
+// Splits of a key block's steps (64 queries x 128 keys of one head) for the
+// 16-bit dK/dV kernel at these sizes: a function of the shapes, so that the
+// workspace is known without a device; the lines are for 256 CUs.  One 8-wave
+// workgroup fits a CU, so up to 128 blocks leave half the CUs idle, and about
+// one causal block per CU lasts as long as the heaviest, twice the mean: twice
+// as many halves, heaviest first, fill both gaps.  A split costs 16 bytes
+// written and read per element of dK and dV, and its own start and end: worth
+// 16 steps where CUs are idle, 32 where only the balance is gained.
+// Backward, bf16, us at 1 / 2 / 4 / 8 splits (B, Hq, Hkv, L, D; the rule's choice in []):
+//   causal (2,16,4,4096,128), 256 blocks: 665 [522] 548 618
+//   causal (1,16,2,4096,128), 64 blocks:  976 559 354 [293]
+//   causal (1,32,8,2048,128), 128 blocks: 294 204 [177] 208
+//   causal (1,8,8,4096,64), 256 blocks:   123 [108] 123 156
+//   causal (1,16,16,2048,128), 256 blocks of 32 steps: [115] 120 154 231
+//   full   (2,8,2,2048,128), 64 blocks:   283 182 [145] 161
+static int bwd_nsplit(int64_t batch, int64_t q_heads, int64_t kv_heads, int64_t q_len, int64_t kv_len, bool causal) {
+  const int64_t blocks = (kv_len + kBKV - 1) / kBKV * batch * kv_heads;
+  const int64_t steps = (q_len + kBQs - 1) / kBQs * (q_heads / kv_heads);
+  int ns = 1;
+  while (ns < 8 && blocks * ns <= (causal ? 256 : 128) && steps >= 2 * ns * (blocks * ns <= 128 ? 16 : 32)) ns *= 2;
+  return ns;
+}
+
 template <typename E, int D, int EXT>
 static int run_bwd_h16(const FlashBwdArgs& a, bool hb, hipStream_t s) {
   // Small grids (at most one workgroup per CU, or two with a causal mask,
@@ -44,11 +81,18 @@ static int run_bwd_h16(const FlashBwdArgs& a, bool hb, hipStream_t s) {
     if (rc != PJX_OK) return rc;
   }
   if (a.f.Lk == 0) return PJX_OK;
+  int rc;
   if (small((long)((a.f.Lk + kBKV - 1) / kBKV) * a.f.B * a.f.Hkv))
-    return hb ? launch_dkdv<flash_bwd_dkdv_kernel<E, D, true, 0, 2>>(a, s, 2 * kThreads)
-              : launch_dkdv<flash_bwd_dkdv_kernel<E, D, false, 0, 2>>(a, s, 2 * kThreads);
-  return hb ? launch_dkdv<flash_bwd_dkdv_kernel<E, D, true, EXT>>(a, s)
+    rc = hb ? launch_dkdv<flash_bwd_dkdv_kernel<E, D, true, 0, 2>>(a, s, 2 * kThreads)
+            : launch_dkdv<flash_bwd_dkdv_kernel<E, D, false, 0, 2>>(a, s, 2 * kThreads);
+  else
+    rc = hb ? launch_dkdv<flash_bwd_dkdv_kernel<E, D, true, EXT>>(a, s)
             : launch_dkdv<flash_bwd_dkdv_kernel<E, D, false, EXT>>(a, s);
+  if (rc != PJX_OK || a.nsplit == 1) return rc;
+  const size_t n = (size_t)a.f.B * a.f.Lk * a.f.Hkv * D;
+  launch_kernel<bwd_split_reduce_kernel<E>>(dim3((unsigned)((n / 4 + kThreads - 1) / kThreads), 2), dim3(kThreads), 0, s,
+                                            (const float*)a.part, a.nsplit, n, (uint16_t*)a.dk, (uint16_t*)a.dv);
+  return check_launch("pjx_flash_bwd (split sum)");
 }
 
 template <int D, int EXT>
@@ -72,6 +116,18 @@ using namespace pjx;
 extern "C" size_t pjx_flash_bwd_workspace_size(int64_t batch, int64_t q_heads, int64_t q_len) {
   if (batch <= 0 || q_heads <= 0 || q_len <= 0) return 0;
   return (size_t)(2 * batch * q_heads * q_len) * sizeof(float);
+}
+
+extern "C" size_t pjx_flash_bwd_split_workspace_size(int dtype, int64_t batch, int64_t q_heads, int64_t kv_heads,
+                                                     int64_t q_len, int64_t kv_len, int64_t head_dim, int causal) {
+  if (dtype != PJX_DTYPE_BF16 && dtype != PJX_DTYPE_F16) return 0;
+  if (head_dim != 64 && head_dim != 128) return 0;
+  if (batch <= 0 || q_heads <= 0 || kv_heads <= 0 || q_heads % kv_heads || q_len <= 0 || kv_len <= 0) return 0;
+  if (q_len > (1 << 30) || kv_len > (1 << 30)) return 0;
+  const int ns = bwd_nsplit(batch, q_heads, kv_heads, q_len, kv_len, causal != 0);
+  if (ns == 1) return 0;
+  return wide_bwd_ds_offset(pjx_flash_bwd_workspace_size(batch, q_heads, q_len)) +
+         (size_t)ns * 2 * batch * kv_len * kv_heads * head_dim * sizeof(float);
 }
 
 extern "C" size_t pjx_flash_bwd_ds_workspace_size(int dtype, int64_t batch, int64_t q_heads, int64_t q_len,
@@ -152,6 +208,16 @@ extern "C" int pjx_flash_bwd(int dtype, const void* q, const void* k, const void
   ba.lse2 = ba.delta + batch * q_heads * q_len;
   ba.dq = dq; ba.dk = dk; ba.dv = dv;
   ba.dbias = dbias;
+  ba.part = nullptr;
+  ba.nsplit = 1;
+  const size_t split_need =
+      pjx_flash_bwd_split_workspace_size(dtype, batch, q_heads, kv_heads, q_len, kv_len, head_dim, causal);
+  // a window or segment ids leave each key block few of the steps counted
+  const bool local = a.m.win_left != kNoBound || a.m.win_right != kNoBound || a.m.seqlen || a.m.seg_k;
+  if (split_need > 0 && workspace_bytes >= split_need && !local) {
+    ba.part = (float*)((unsigned char*)workspace + wide_bwd_ds_offset(need));
+    ba.nsplit = bwd_nsplit(batch, q_heads, kv_heads, q_len, kv_len, causal != 0);
+  }
   hipStream_t s = (hipStream_t)stream;
   if (head_dim == 256 && f32) return run_flash_f32_wide_bwd(ba, s);
   if (head_dim == 256) {

@@ -55,6 +55,11 @@ struct FlashBwdArgs {
   void* dk;
   void* dv;
   float* dbias;       // [B, Hq, Lq, Lk] fp32 dL/d(bias): P (dP - delta) per score, or null
+  // The 16-bit dK/dV kernel's steps of one key block spread over nsplit
+  // workgroups (1: none): fp32 sums [2 (dK, dV)][nsplit][B, Lk, Hkv, D], added
+  // and rounded by bwd_split_reduce_kernel.
+  float* part;
+  int nsplit;
 };
 
 constexpr int kBKV = 128;  // keys per dK/dV workgroup (32 per wave)
@@ -466,7 +471,8 @@ __global__ __launch_bounds__(NG * kThreads, (D <= 128 ? 2 : 1)) void flash_bwd_d
   const int col = lane & 31, half = lane >> 5;
   const int BH = a.B * a.Hkv;
   const int bh = blockIdx.x % BH;
-  const int k0 = (blockIdx.x / BH) * kBKV;
+  const int split = (blockIdx.x / BH) % ba.nsplit;
+  const int k0 = (blockIdx.x / (BH * ba.nsplit)) * kBKV;
   const int b = bh / a.Hkv, hkv = bh % a.Hkv;
   const int G = a.Hq / a.Hkv;
   const int kw = k0 + 32 * w;
@@ -508,7 +514,9 @@ __global__ __launch_bounds__(NG * kThreads, (D <= 128 ? 2 : 1)) void flash_bwd_d
     }
   }
   const int n_qt = (k0 < kv_end && q_end > q_begin) ? (q_end - q_begin + kBQs - 1) / kBQs : 0;
-  const int n_tiles = G * n_qt;
+  // This split's share [t_first, t_first + n_tiles) of the block's steps.
+  const int t_first = (int)((long)G * n_qt * split / ba.nsplit);
+  const int n_tiles = (int)((long)G * n_qt * (split + 1) / ba.nsplit) - t_first;
 
   // K^T and V^T as B operands: lane holds key `key`, dims 16*s + 8*half + [0,8).
   typename E::v8 kf[D / 16], vf[D / 16];
@@ -552,8 +560,8 @@ __global__ __launch_bounds__(NG * kThreads, (D <= 128 ? 2 : 1)) void flash_bwd_d
   // one KV head's key blocks (same XCD, running together) then stream the same
   // Q / dO tile at the same time, so all but the first read it from L2
   // (causal: each starts at the sequence's end and stops at its own keys).
-  auto tile_head = [&](int t) { return hkv * G + t % G; };
-  auto tile_q0 = [&](int t) { return q_begin + (n_qt - 1 - t / G) * kBQs; };
+  auto tile_head = [&](int t) { return hkv * G + (t_first + t) % G; };
+  auto tile_q0 = [&](int t) { return q_begin + (n_qt - 1 - (t_first + t) / G) * kBQs; };
 
   auto issue = [&](int t, unsigned char* st) {
     const int h = tile_head(t), q0 = tile_q0(t);
@@ -765,6 +773,22 @@ __global__ __launch_bounds__(NG * kThreads, (D <= 128 ? 2 : 1)) void flash_bwd_d
       }
   }
 
+  if (ba.nsplit > 1) {
+    if (key < a.Lk) {
+      const size_t n = (size_t)a.B * a.Lk * a.Hkv * D;
+      float* pk = ba.part + split * n + ((size_t)(b * a.Lk + key) * a.Hkv + hkv) * D;
+      float* pv = pk + ba.nsplit * n;
+#pragma unroll
+      for (int db = 0; db < D / 32; ++db)
+#pragma unroll
+        for (int gq = 0; gq < 4; ++gq) {
+          const int d = db * 32 + 8 * gq + 4 * half;
+          *(f32x4*)(pk + d) = f32x4{acck[db][4 * gq], acck[db][4 * gq + 1], acck[db][4 * gq + 2], acck[db][4 * gq + 3]};
+          *(f32x4*)(pv + d) = f32x4{accv[db][4 * gq], accv[db][4 * gq + 1], accv[db][4 * gq + 2], accv[db][4 * gq + 3]};
+        }
+    }
+    return;
+  }
   // dK, dV rows of this lane's key (zeros for keys past the valid length).
   if (key < a.Lk) {
     const size_t koff = ((size_t)(b * a.Lk + key) * a.Hkv + hkv) * D;
@@ -1246,7 +1270,7 @@ static int launch_dq(const FlashBwdArgs& a, hipStream_t stream, int threads = kT
 
 template <auto K>
 static int launch_dkdv(const FlashBwdArgs& a, hipStream_t stream, int threads = kThreads) {
-  const long blocks = (long)((a.f.Lk + kBKV - 1) / kBKV) * a.f.B * a.f.Hkv;
+  const long blocks = (long)((a.f.Lk + kBKV - 1) / kBKV) * a.f.B * a.f.Hkv * a.nsplit;
   launch_kernel<K>(dim3((unsigned)blocks), dim3(threads), 0, stream, a);
   return check_launch("pjx_flash_bwd (dk, dv)");
 }

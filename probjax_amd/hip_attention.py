@@ -236,6 +236,10 @@ def flash_attention_bwd(
             ds_bytes = int(lib.pjx_flash_bwd_ds_workspace_size(code, B, Hq, Lq, Lk, D))
         nbytes = _ds_route_bytes(nbytes, ds_bytes, ds_route, dev,
                                  "the dS route takes 16-bit inputs at head dim 256 without bias or score modifiers")
+        if mods is None or (mods.window_left < 0 and mods.window_right < 0 and mods.seq_lengths is None
+                            and mods.segment_k is None):
+            split = lib.pjx_flash_bwd_split_workspace_size(code, B, Hq, Hkv, Lq, Lk, D, int(bool(causal)))
+            nbytes = max(nbytes, int(split))
     ws = _workspace(nbytes, dev, workspace)
     rc = lib.pjx_flash_bwd(
         code, _ptr(q), _ptr(k), _ptr(v), _ptr(o), _ptr(do), _ptr(lse), _ptr(dq),
