@@ -3,24 +3,9 @@
 // flash_bwd_kernels.h; this unit is built in the VGPR MFMA register form, the
 // D = 256 dK/dV kernel in flash_bwd256.hip in the default form.
 #include "flash_bwd_kernels.h"
+#include "flash_f32_bwd.h"
 
 namespace pjx {
-
-// dQ first (it writes the delta * sm_scale and lse*log2e the dK/dV kernel reads), then
-// dK/dV.  Without keys only dQ (= 0) runs; without queries only dK/dV (= 0).
-template <int D, int EXT>
-static int run_bwd_f32(const FlashBwdArgs& a, bool hb, hipStream_t s) {
-  if (a.f.Lq > 0) {
-    const bool db = a.dbias != nullptr;
-    const int rc = db ? launch_dq<flash_bwd_dq_f32_kernel<D, 2, EXT>>(a, s)
-                 : hb ? launch_dq<flash_bwd_dq_f32_kernel<D, 1, EXT>>(a, s)
-                      : launch_dq<flash_bwd_dq_f32_kernel<D, 0, EXT>>(a, s);
-    if (rc != PJX_OK) return rc;
-  }
-  if (a.f.Lk == 0) return PJX_OK;
-  return hb ? launch_dkdv<flash_bwd_dkdv_f32_kernel<D, true, EXT>>(a, s)
-            : launch_dkdv<flash_bwd_dkdv_f32_kernel<D, false, EXT>>(a, s);
-}
 
 // out = the sum over splits of dK (blockIdx.y 0) or dV (1), in split order,
 // rounded to 16 bits; n elements of each (a multiple of 4).  Bound by the
@@ -59,6 +44,8 @@ static int bwd_nsplit(int64_t batch, int64_t q_heads, int64_t kv_heads, int64_t 
   return ns;
 }
 
+// dQ first (it writes the delta * sm_scale and lse*log2e the dK/dV kernel reads), then
+// dK/dV.  Without keys only dQ (= 0) runs; without queries only dK/dV (= 0).
 template <typename E, int D, int EXT>
 static int run_bwd_h16(const FlashBwdArgs& a, bool hb, hipStream_t s) {
   // Small grids (at most one workgroup per CU, or two with a causal mask,
@@ -97,7 +84,6 @@ static int run_bwd_h16(const FlashBwdArgs& a, bool hb, hipStream_t s) {
 
 template <int D, int EXT>
 static int run_bwd_t(const FlashBwdArgs& a, int dtype, bool hb, hipStream_t s) {
-  if (dtype == PJX_DTYPE_F32) return run_bwd_f32<D, EXT == 2 ? 3 : EXT>(a, hb, s);
   if (dtype == PJX_DTYPE_F16) return run_bwd_h16<F16Fmt, D, EXT>(a, hb, s);
   return run_bwd_h16<Bf16Fmt, D, EXT>(a, hb, s);
 }
@@ -253,5 +239,10 @@ extern "C" int pjx_flash_bwd(int dtype, const void* q, const void* k, const void
     return launch_dkdv256(ba, dtype == PJX_DTYPE_F16, hb256, s);
   }
   const bool hb = bias != nullptr;
+  if (f32) {
+    const int rc = head_dim == 128 ? run_dq_f32_128(ba, s) : run_dq_f32_64(ba, s);
+    if (rc != PJX_OK) return rc;
+    return head_dim == 128 ? run_dkdv_f32_128(ba, s) : run_dkdv_f32_64(ba, s);
+  }
   return head_dim == 128 ? run_bwd<128>(ba, dtype, hb, s) : run_bwd<64>(ba, dtype, hb, s);
 }

@@ -809,458 +809,6 @@ __global__ __launch_bounds__(NG * kThreads, (D <= 128 ? 2 : 1)) void flash_bwd_d
   }
 }
 
-// ---------------------------------------------------------------------------
-// fp32 path: v_mfma_f32_32x32x2f32 (full fp32 products) for every product.
-// One MFMA step contracts two indices, one per wave half.  Products whose
-// contraction runs over the head dim take half rows (half 0: dims s, half 1:
-// dims D/2 + s) as in the fp32 forward; products whose contraction runs over
-// keys or queries take the pair (register r, half 0), (r, half 1) of a 32x32
-// C block as the two indices, so their A operand is one float of a row-major
-// tile.  Tiles are staged through registers into LDS rows padded to D + 4
-// floats (16-byte reads of 16 consecutive rows hit distinct banks).
-// ---------------------------------------------------------------------------
-template <int D, int BIAS, int EXT>
-__global__ __launch_bounds__(kThreads, 1) void flash_bwd_dq_f32_kernel(FlashBwdArgs ba) {
-  constexpr bool HB = BIAS != 0, DB = BIAS == 2;  // as in flash_bwd_dq_kernel
-  const FlashArgs& a = ba.f;
-  constexpr int BK = (D == 128) ? 32 : 64;
-  constexpr int KS = D + 4;
-  constexpr int DC = D / 4;
-  constexpr int PER_T = BK * DC / kThreads;
-  static_assert(PER_T >= 1, "tile shape");
-  __shared__ __attribute__((aligned(16))) float k_lds[2][BK * KS];
-  __shared__ __attribute__((aligned(16))) float v_lds[2][BK * KS];
-
-  BlockGeom g = block_geom(a);
-  if constexpr (EXT > 0) ext_block_range(a, g, BK);
-  const int tid = threadIdx.x, lane = tid & 63;
-  const int col = lane & 31, half = lane >> 5;
-  const size_t kv_row = (size_t)a.Hkv * D;
-  const float* Kb = (const float*)a.k + ((size_t)g.b * a.Lk * a.Hkv + g.hkv) * D;
-  const float* Vb = (const float*)a.v + ((size_t)g.b * a.Lk * a.Hkv + g.hkv) * D;
-  const bool row_in = g.qi < a.Lq;
-  const bool row_ok = g.qi < g.q_hi;
-
-  float qf[D / 2], dof[D / 2];
-  float dsum = 0.f;
-  {
-    const size_t roff = ((size_t)(g.b * a.Lq + (row_in ? g.qi : 0)) * a.Hq + g.h) * D + half * (D / 2);
-    const float* qrow = (const float*)a.q + roff;
-    const float* drow = (const float*)ba.dout + roff;
-    const float* orow = (const float*)a.o + roff;
-#pragma unroll
-    for (int s = 0; s < D / 8; ++s) {
-      f32x4 rq = {0.f, 0.f, 0.f, 0.f}, rd = rq, ro = rq;
-      if (row_in) {
-        rq = *(const f32x4*)(qrow + 4 * s);
-        rd = *(const f32x4*)(drow + 4 * s);
-        ro = *(const f32x4*)(orow + 4 * s);
-      }
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        qf[4 * s + j] = rq[j];
-        dof[4 * s + j] = rd[j];
-        dsum = fmaf(ro[j], rd[j], dsum);
-      }
-    }
-  }
-  const float delta = xor32_sum(dsum);
-  const float dsc = delta * a.scale;  // the workspace holds delta * sm_scale
-  float lse2 = 0.f;
-  const size_t lidx = ((size_t)g.b * a.Hq + g.h) * a.Lq + g.qi;
-  if (row_in) {
-    lse2 = a.lse[lidx] * kLog2e;
-    if (half == 0) {
-      ba.delta[lidx] = dsc;
-      ba.lse2[lidx] = lse2;
-    }
-  }
-  const float* brow = nullptr;
-  if constexpr (HB) {
-    brow = a.bias + (size_t)g.b * a.bias_bstride + (size_t)g.h * a.bias_hstride +
-           (size_t)(row_in ? g.qi : 0) * a.Lk;
-  }
-  const bool bias_vec = (a.Lk & 3) == 0;
-  const float cx = (HB || EXT == 3) ? kLog2e : a.scale * kLog2e;
-  ExtRows er;
-  if constexpr (EXT > 0) er = ext_rows(a, g);
-
-  f32x16 acc[D / 32];
-#pragma unroll
-  for (int i = 0; i < D / 32; ++i) acc[i] = f32x16{};
-  const int t_begin = g.kv_begin / BK;
-  const int n_tiles = max((g.kv_stop + BK - 1) / BK - t_begin, 0);
-  const int q_last_w = g.qw + 31;
-
-  f32x4 kreg[PER_T], vreg[PER_T];
-  auto load_tile = [&](int t) {
-    const int k0 = (t_begin + t) * BK;
-#pragma unroll
-    for (int i = 0; i < PER_T; ++i) {
-      const int u = tid + kThreads * i;
-      const int kk = k0 + u / DC, dc = u % DC;
-      f32x4 rk = {0.f, 0.f, 0.f, 0.f}, rv = rk;
-      if (kk < g.kv_stop) {
-        rk = *(const f32x4*)(Kb + (size_t)kk * kv_row + dc * 4);
-        rv = *(const f32x4*)(Vb + (size_t)kk * kv_row + dc * 4);
-      }
-      kreg[i] = rk;
-      vreg[i] = rv;
-    }
-  };
-  auto store_tile = [&](int buf) {
-#pragma unroll
-    for (int i = 0; i < PER_T; ++i) {
-      const int u = tid + kThreads * i;
-      *(f32x4*)(&k_lds[buf][(u / DC) * KS + (u % DC) * 4]) = kreg[i];
-      *(f32x4*)(&v_lds[buf][(u / DC) * KS + (u % DC) * 4]) = vreg[i];
-    }
-  };
-
-  auto compute = [&](int t, int buf) {
-    const int k0 = (t_begin + t) * BK;
-    if constexpr (EXT > 0) {
-      if (!er.any || k0 > er.hi_last || k0 + BK - 1 < er.lo_first) return;
-    } else {
-      if (a.causal && k0 > q_last_w) return;
-    }
-    const float* kl = k_lds[buf];
-    const float* vl = v_lds[buf];
-    f32x16 s[BK / 32], dp[BK / 32];
-#pragma unroll
-    for (int kb = 0; kb < BK / 32; ++kb) {
-      s[kb] = f32x16{};
-      dp[kb] = f32x16{};
-      const float* kp = kl + (kb * 32 + col) * KS + half * (D / 2);
-      const float* vp = vl + (kb * 32 + col) * KS + half * (D / 2);
-#pragma unroll
-      for (int st4 = 0; st4 < D / 8; ++st4) {
-        const f32x4 kf = *(const f32x4*)(kp + 4 * st4);
-        const f32x4 vf = *(const f32x4*)(vp + 4 * st4);
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          s[kb] = mfma32x32x2f32(kf[j], qf[4 * st4 + j], s[kb]);
-          dp[kb] = mfma32x32x2f32(vf[j], dof[4 * st4 + j], dp[kb]);
-        }
-      }
-    }
-    f32x16 dbv[DB ? BK / 32 : 1];
-    if constexpr (EXT == 3) {
-      ext_scores_sT<BK / 32, HB>(a, g, er, s, k0, half, brow, row_in,
-                                 [&](int kb, int r, float x, float gg) {
-                                   const float p = fast_exp2(fmaf(x, cx, -lse2));
-                                   const float t = p * (dp[kb][r] - delta);
-                                   if constexpr (DB) dbv[kb][r] = t;
-                                   s[kb][r] = t * a.scale * gg;
-                                 });
-    } else {
-    if constexpr (HB) {
-#pragma unroll
-      for (int kb = 0; kb < BK / 32; ++kb)
-#pragma unroll
-        for (int gq = 0; gq < 4; ++gq) {
-          const int kk = k0 + kb * 32 + 8 * gq + 4 * half;
-          f32x4 bv = {0.f, 0.f, 0.f, 0.f};
-          if (row_in) bv = bias_vec ? load_bias4<true>(brow, kk, a.Lk) : load_bias4<false>(brow, kk, a.Lk);
-#pragma unroll
-          for (int j = 0; j < 4; ++j) s[kb][4 * gq + j] = fmaf(s[kb][4 * gq + j], a.scale, bv[j]);
-        }
-    }
-    if constexpr (EXT == 1) ext_mask_sT<BK / 32>(g, er, s, k0, half);
-    const bool need_mask = EXT == 0 && ((k0 + BK > g.kv_end) || (a.causal && k0 + BK - 1 > g.qw) ||
-                                        (g.qw + 31 >= g.q_hi));
-    if (need_mask) {
-#pragma unroll
-      for (int kb = 0; kb < BK / 32; ++kb)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          const int kk = k0 + kb * 32 + 8 * (r >> 2) + 4 * half + (r & 3);
-          const bool keep = row_ok && kk < g.kv_end && (!a.causal || kk <= g.qi);
-          if (!keep) s[kb][r] = -INFINITY;
-        }
-    }
-#pragma unroll
-    for (int kb = 0; kb < BK / 32; ++kb)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const float p = fast_exp2(fmaf(s[kb][r], cx, -lse2));
-        if constexpr (DB) {
-          const float t = p * (dp[kb][r] - delta);
-          dbv[kb][r] = t;
-          s[kb][r] = t * a.scale;
-        } else {
-          s[kb][r] = p * fmaf(dp[kb][r], a.scale, -dsc);  // p (dp - delta) scale
-        }
-      }
-    }
-    if constexpr (DB) store_dbias<BK / 32>(ba, g, dbv, k0, half, row_in);
-    // dQ^T[d][query] += K^T dS^T: step (kb, r) contracts keys (r, half 0/1).
-#pragma unroll
-    for (int db = 0; db < D / 32; ++db)
-#pragma unroll
-      for (int kb = 0; kb < BK / 32; ++kb)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          const int key = kb * 32 + 8 * (r >> 2) + 4 * half + (r & 3);
-          acc[db] = mfma32x32x2f32(kl[key * KS + db * 32 + col], s[kb][r], acc[db]);
-        }
-  };
-
-  if (n_tiles > 0) {
-    load_tile(0);
-    store_tile(0);
-  }
-  __syncthreads();
-  for (int t = 0; t < n_tiles; ++t) {
-    if (t + 1 < n_tiles) load_tile(t + 1);
-    compute(t, t & 1);
-    if (t + 1 < n_tiles) store_tile((t + 1) & 1);
-    __syncthreads();
-  }
-
-  if (row_in) {
-    float* drow = (float*)ba.dq + ((size_t)(g.b * a.Lq + g.qi) * a.Hq + g.h) * D;
-#pragma unroll
-    for (int db = 0; db < D / 32; ++db)
-#pragma unroll
-      for (int gq = 0; gq < 4; ++gq) {
-        f32x4 v;
-#pragma unroll
-        for (int j = 0; j < 4; ++j) v[j] = acc[db][4 * gq + j];
-        *(f32x4*)(drow + db * 32 + 8 * gq + 4 * half) = v;
-      }
-  }
-}
-
-template <int D, bool BIAS, int EXT>
-__global__ __launch_bounds__(kThreads, 1) void flash_bwd_dkdv_f32_kernel(FlashBwdArgs ba) {
-  const FlashArgs& a = ba.f;
-  constexpr int BQ = 32;  // queries per stage (one 32-query step)
-  constexpr int KS = D + 4;
-  constexpr int DC = D / 4;
-  constexpr int PER_T = BQ * DC / kThreads;
-  static_assert(PER_T >= 1, "tile shape");
-  __shared__ __attribute__((aligned(16))) float q_lds[2][BQ * KS];
-  __shared__ __attribute__((aligned(16))) float d_lds[2][BQ * KS];
-  __shared__ __attribute__((aligned(16))) float ld_lds[2][2 * BQ];  // lse*log2e, delta * sm_scale
-
-  const int tid = threadIdx.x, lane = tid & 63;
-  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int col = lane & 31, half = lane >> 5;
-  const int BH = a.B * a.Hkv;
-  const int bh = blockIdx.x % BH;
-  const int k0 = (blockIdx.x / BH) * kBKV;
-  const int b = bh / a.Hkv, hkv = bh % a.Hkv;
-  const int G = a.Hq / a.Hkv;
-  const int kw = k0 + 32 * w;
-  const int key = kw + col;
-  int kv_end = min(a.Lk, a.kv_valid);
-  if (a.kv_lengths) kv_end = min(kv_end, max(a.kv_lengths[b], 0));
-  const int q_hi = min(a.Lq, a.q_valid);
-  int q_begin = a.causal ? (k0 / BQ) * BQ : 0;
-  int q_end = q_hi;
-  int qlo = 0, qhi = q_hi - 1, wq_first = 0, wq_last = q_hi - 1, segk = 0;
-  int qhi_first = q_hi - 1, qlo_last = 0;  // rows seen by every key of the wave: [qlo_last, qhi_first]
-  if constexpr (EXT > 0) {
-    q_end = q_begin = 0;
-    if (k0 < kv_end) {
-      int a0, a1, b0, b1;
-      key_bounds(a.m, a.causal, b, kv_end, q_hi, k0, a0, a1);
-      key_bounds(a.m, a.causal, b, kv_end, q_hi, min(k0 + kBKV, kv_end) - 1, b0, b1);
-      q_begin = max(a0, 0);
-      q_end = b1 + 1;
-    }
-    key_bounds(a.m, a.causal, b, kv_end, q_hi, key, qlo, qhi);
-    if (kw < kv_end) {
-      key_bounds(a.m, a.causal, b, kv_end, q_hi, kw, wq_first, qhi_first);
-      key_bounds(a.m, a.causal, b, kv_end, q_hi, min(kw + 32, kv_end) - 1, qlo_last, wq_last);
-    }
-    if (a.m.seg_k && key < a.Lk) segk = a.m.seg_k[(size_t)b * a.Lk + key];
-  }
-  const int n_qt = (k0 < kv_end && q_end > q_begin) ? (q_end - q_begin + BQ - 1) / BQ : 0;
-  const int n_tiles = G * n_qt;
-
-  float kf[D / 2], vf[D / 2];
-  {
-    const bool kin = key < a.Lk;
-    const size_t koff = ((size_t)(b * a.Lk + (kin ? key : 0)) * a.Hkv + hkv) * D + half * (D / 2);
-    const float* krow = (const float*)a.k + koff;
-    const float* vrow = (const float*)a.v + koff;
-#pragma unroll
-    for (int s = 0; s < D / 8; ++s) {
-      f32x4 rk = {0.f, 0.f, 0.f, 0.f}, rv = rk;
-      if (kin) {
-        rk = *(const f32x4*)(krow + 4 * s);
-        rv = *(const f32x4*)(vrow + 4 * s);
-      }
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        kf[4 * s + j] = rk[j];
-        vf[4 * s + j] = rv[j];
-      }
-    }
-  }
-  const float cx = (BIAS || EXT == 3) ? kLog2e : a.scale * kLog2e;
-  const size_t q_row = (size_t)a.Hq * D;
-
-  f32x16 acck[D / 32], accv[D / 32];
-#pragma unroll
-  for (int i = 0; i < D / 32; ++i) {
-    acck[i] = f32x16{};
-    accv[i] = f32x16{};
-  }
-
-  f32x4 qreg[PER_T], dreg[PER_T];
-  float lreg = 0.f;
-  // last query tile first, heads innermost (as the bf16 kernel)
-  auto tile_head = [&](int t) { return hkv * G + t % G; };
-  auto tile_q0 = [&](int t) { return q_begin + (n_qt - 1 - t / G) * BQ; };
-  auto load_tile = [&](int t) {
-    const int h = tile_head(t), q0 = tile_q0(t);
-    const float* Qb = (const float*)a.q + ((size_t)b * a.Lq * a.Hq + h) * D;
-    const float* Db = (const float*)ba.dout + ((size_t)b * a.Lq * a.Hq + h) * D;
-#pragma unroll
-    for (int i = 0; i < PER_T; ++i) {
-      const int u = tid + kThreads * i;
-      const int qq = q0 + u / DC, dc = u % DC;
-      f32x4 rq = {0.f, 0.f, 0.f, 0.f}, rd = rq;
-      if (qq < a.Lq) {
-        rq = *(const f32x4*)(Qb + (size_t)qq * q_row + dc * 4);
-        rd = *(const f32x4*)(Db + (size_t)qq * q_row + dc * 4);
-      }
-      qreg[i] = rq;
-      dreg[i] = rd;
-    }
-    lreg = 0.f;
-    if (tid < 2 * BQ) {
-      const int qq = q0 + (tid % BQ);
-      const size_t li = ((size_t)b * a.Hq + h) * a.Lq + qq;
-      if (qq < a.Lq) lreg = tid < BQ ? ba.lse2[li] : ba.delta[li];
-    }
-  };
-  auto store_tile = [&](int buf) {
-#pragma unroll
-    for (int i = 0; i < PER_T; ++i) {
-      const int u = tid + kThreads * i;
-      *(f32x4*)(&q_lds[buf][(u / DC) * KS + (u % DC) * 4]) = qreg[i];
-      *(f32x4*)(&d_lds[buf][(u / DC) * KS + (u % DC) * 4]) = dreg[i];
-    }
-    if (tid < 2 * BQ) ld_lds[buf][tid] = lreg;
-  };
-
-  auto compute = [&](int t, int buf) {
-    const int h = tile_head(t), q0 = tile_q0(t);
-    if (q0 >= q_hi || kw >= kv_end) return;
-    if constexpr (EXT > 0) {
-      if (q0 > wq_last || q0 + BQ - 1 < wq_first) return;  // no row of this step sees the wave's keys
-    } else {
-      if (a.causal && q0 + BQ - 1 < kw) return;  // every query before this wave's first key
-    }
-    const float* ql = q_lds[buf];
-    const float* dl = d_lds[buf];
-    const float* lsm = ld_lds[buf];
-    // S[query][key] = Q K^T and dP = dO V^T; register r holds query
-    // q0 + 8*(r/4) + 4*half + r%4 of key `key`.
-    f32x16 s = f32x16{}, dp = f32x16{};
-    {
-      const float* qp = ql + col * KS + half * (D / 2);
-      const float* dpp = dl + col * KS + half * (D / 2);
-#pragma unroll
-      for (int st4 = 0; st4 < D / 8; ++st4) {
-        const f32x4 qv = *(const f32x4*)(qp + 4 * st4);
-        const f32x4 dv4 = *(const f32x4*)(dpp + 4 * st4);
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          s = mfma32x32x2f32(qv[j], kf[4 * st4 + j], s);
-          dp = mfma32x32x2f32(dv4[j], vf[4 * st4 + j], dp);
-        }
-      }
-    }
-    f32x16 ds;
-    if constexpr (EXT == 3) {
-      const float* bbase = nullptr;
-      if constexpr (BIAS) bbase = a.bias + (size_t)b * a.bias_bstride + (size_t)h * a.bias_hstride;
-      const HeadMods hm = head_mods(a.m, h);
-      ext_scores_S<BIAS>(a, b, hm, key, qlo, qhi, segk, s, q0, half, bbase,
-                         [&](int r, float x, float gg) {
-                           const int qi = 8 * (r >> 2) + 4 * half + (r & 3);
-                           const float p = fast_exp2(fmaf(x, cx, -lsm[qi]));
-                           s[r] = p;
-                           ds[r] = p * fmaf(dp[r], a.scale, -lsm[BQ + qi]) * gg;
-                         });
-    } else {
-    if constexpr (BIAS) {
-      const float* bbase = a.bias + (size_t)b * a.bias_bstride + (size_t)h * a.bias_hstride;
-#pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const int qr = q0 + 8 * (r >> 2) + 4 * half + (r & 3);
-        const float bv = (qr < a.Lq && key < a.Lk) ? bbase[(size_t)qr * a.Lk + key] : 0.f;
-        s[r] = fmaf(s[r], a.scale, bv);
-      }
-    }
-    if constexpr (EXT == 1)
-      ext_mask_S(s, q0, half, qlo, qhi, !(kw + 31 < kv_end && q0 >= qlo_last && q0 + BQ - 1 <= qhi_first));
-    const bool need_mask = EXT == 0 && ((a.causal && q0 < kw + 31) || (kw + 32 > kv_end) || (q0 + BQ > q_hi));
-    if (need_mask) {
-#pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const int qr = q0 + 8 * (r >> 2) + 4 * half + (r & 3);
-        const bool keep = key < kv_end && qr < q_hi && (!a.causal || qr >= key);
-        if (!keep) s[r] = -INFINITY;
-      }
-    }
-#pragma unroll
-    for (int r = 0; r < 16; ++r) {
-      const int qi = 8 * (r >> 2) + 4 * half + (r & 3);
-      const float p = fast_exp2(fmaf(s[r], cx, -lsm[qi]));
-      s[r] = p;
-      ds[r] = p * fmaf(dp[r], a.scale, -lsm[BQ + qi]);
-    }
-    }
-    // dV^T[d][key] += dO^T P and dK^T[d][key] += Q^T dS: step r contracts
-    // queries (r, half 0/1).
-#pragma unroll
-    for (int db = 0; db < D / 32; ++db)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const int qi = 8 * (r >> 2) + 4 * half + (r & 3);
-        accv[db] = mfma32x32x2f32(dl[qi * KS + db * 32 + col], s[r], accv[db]);
-        acck[db] = mfma32x32x2f32(ql[qi * KS + db * 32 + col], ds[r], acck[db]);
-      }
-  };
-
-  if (n_tiles > 0) {
-    load_tile(0);
-    store_tile(0);
-  }
-  __syncthreads();
-  for (int t = 0; t < n_tiles; ++t) {
-    if (t + 1 < n_tiles) load_tile(t + 1);
-    compute(t, t & 1);
-    if (t + 1 < n_tiles) store_tile((t + 1) & 1);
-    __syncthreads();
-  }
-
-  if (key < a.Lk) {
-    const size_t koff = ((size_t)(b * a.Lk + key) * a.Hkv + hkv) * D;
-    float* dkrow = (float*)ba.dk + koff;
-    float* dvrow = (float*)ba.dv + koff;
-#pragma unroll
-    for (int db = 0; db < D / 32; ++db)
-#pragma unroll
-      for (int gq = 0; gq < 4; ++gq) {
-        f32x4 vk, vv;
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          vk[j] = acck[db][4 * gq + j];
-          vv[j] = accv[db][4 * gq + j];
-        }
-        *(f32x4*)(dkrow + db * 32 + 8 * gq + 4 * half) = vk;
-        *(f32x4*)(dvrow + db * 32 + 8 * gq + 4 * half) = vv;
-      }
-  }
-}
-
 template <auto K>
 static int launch_dq(const FlashBwdArgs& a, hipStream_t stream, int threads = kThreads) {
   const long blocks = (long)a.f.n_qtiles * a.f.B * a.f.Hq;

@@ -32,6 +32,8 @@ struct FlashArgs {
 constexpr int kBQ = 128;
 constexpr int kThreads = 256;
 
+// fp32 forward at head dims 64 and 128 (flash_f32.hip).  Returns a PJX_* status.
+int launch_flash_f32(const FlashArgs& a, int head_dim, hipStream_t s);
 // fp32 forward at head dim 256 (flash_f32_wide.hip).  Returns a PJX_* status.
 int launch_flash_f32_wide(const FlashArgs& a, hipStream_t s);
 
@@ -78,14 +80,14 @@ __device__ __forceinline__ BlockGeom block_geom(const FlashArgs& a) { return blo
 // With extended masks: the block's key range [kv_begin, kv_stop) from the
 // interval bounds of its first and last row (both bounds are monotone in the
 // row), kv_begin rounded down to the key tile.
-__device__ __forceinline__ void ext_block_range(const FlashArgs& a, BlockGeom& g, int tile) {
+__device__ __forceinline__ void ext_block_range(const FlashArgs& a, BlockGeom& g, int tile, int rows = kBQ) {
   g.kv_begin = 0;
   if (g.q0 >= g.q_hi) {
     g.kv_stop = 0;
     return;
   }
   int lo0, hi0, lo1, hi1;
-  const int q_last = min(g.q0 + kBQ, g.q_hi) - 1;
+  const int q_last = min(g.q0 + rows, g.q_hi) - 1;
   row_bounds(a.m, a.causal, g.b, g.kv_end, g.q_hi, g.q0, lo0, hi0);
   row_bounds(a.m, a.causal, g.b, g.kv_end, g.q_hi, q_last, lo1, hi1);
   g.kv_begin = (max(lo0, 0) / tile) * tile;
@@ -194,11 +196,12 @@ __device__ __forceinline__ ExtRows ext_rows(const FlashArgs& a, const BlockGeom&
 // Measured, forward + backward: 6 packed documents, bf16 B=2 H=16 L=2048
 // D=128, 707 -> 193 us; causal slopes, bf16 B=2 H=12 L=1024 D=64, the three
 // kernels 168 -> 91 us.
-__device__ __forceinline__ void ext_segments(const FlashArgs& a, BlockGeom& g, ExtRows& er, int tile, int* sm) {
+__device__ __forceinline__ void ext_segments(const FlashArgs& a, BlockGeom& g, ExtRows& er, int tile, int* sm,
+                                             int rows = kBQ) {
   if (!a.m.seg_k) return;
   seg_range(a.m.seg_q, g.b, a.Lq, g.qw, 32, g.q_hi, er.seg_lo, er.seg_hi);
   int lo, hi;
-  seg_range(a.m.seg_q, g.b, a.Lq, g.q0, kBQ, g.q_hi, lo, hi);
+  seg_range(a.m.seg_q, g.b, a.Lq, g.q0, rows, g.q_hi, lo, hi);
   int begin = g.kv_begin, end = g.kv_stop;
   seg_narrow(a.m.seg_k, g.b, a.Lk, lo, hi, sm, begin, end);
   g.kv_begin = (begin / tile) * tile;

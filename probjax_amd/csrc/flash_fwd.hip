@@ -19,13 +19,14 @@
 // A operand reproduces), so the per-row rescale and 1/l are lane-local too.
 // bf16: K and V tiles go HBM -> LDS by buffer loads that write LDS directly,
 // both stored row-major; the A operand of P.V (V^T) comes from transposing
-// LDS reads of the row-major V tile.  fp32: tiles are staged through
-// registers.  Either way LDS holds two tiles, the loads of tile t+1 are in
-// flight while tile t is computed, and there is one barrier per tile.
+// LDS reads of the row-major V tile.  LDS holds two tiles, the loads of tile
+// t+1 are in flight while tile t is computed, and there is one barrier per
+// tile.
 //
-// This file also holds the fp32 kernel for small grids (each query block's
-// keys split over the waves of a workgroup) and pjx_flash_fwd, which picks
-// the kernel; the bf16 dense-bias kernel is in flash_bias_ring.hip.
+// This file also holds the fp32 kernel for small grids at head dim 128 (each
+// query block's keys split over the waves of a workgroup) and pjx_flash_fwd,
+// which picks the kernel; the other fp32 kernels are in flash_f32.hip and
+// flash_f32_wide.hip, the bf16 dense-bias kernel in flash_bias_ring.hip.
 //
 // Grid: one workgroup per (q tile, batch, head), ordered heaviest causal
 // q-tile first (longest-processing-time order), and batch*head fastest so
@@ -622,219 +623,22 @@ __global__ __launch_bounds__(G * kThreads, WPC) void flash_fwd_bf16_pipe_kernel(
 }
 
 // ---------------------------------------------------------------------------
-// fp32 path: v_mfma_f32_32x32x2f32 (full fp32 products) for both products.
-// The k index of one MFMA step is the wave half: half 0 contracts dim s,
-// half 1 dim D/2 + s, so each lane reads a contiguous half row of K.  For
-// P.V the step pairs key (r, half 0) with key (r, half 1) of the S^T layout,
-// so V is read in its natural [key][dim] layout: no transpose needed.
-// ---------------------------------------------------------------------------
-template <int D, bool BIAS, int EXT>
-__global__ __launch_bounds__(kThreads, 1) void flash_fwd_f32_kernel(FlashArgs a) {
-  constexpr int BK = (D == 128) ? 32 : 64;
-  constexpr int KS = D + 4;  // floats; b128 reads of 16 rows hit distinct banks
-  constexpr int VS = D + 8;  // floats; rows 4 apart land 32 banks apart
-  constexpr int DC = D / 4;  // float4 chunks per row
-  constexpr int PER_T = BK * DC / kThreads;
-  static_assert(PER_T >= 1, "tile shape");
-
-  __shared__ __attribute__((aligned(16))) float k_lds[2][BK * KS];
-  __shared__ __attribute__((aligned(16))) float v_lds[2][BK * VS];
-
-  BlockGeom g = block_geom(a);
-  if constexpr (EXT > 0) ext_block_range(a, g, BK);
-  const int tid = threadIdx.x, lane = tid & 63;
-  const int col = lane & 31, half = lane >> 5;
-  const size_t kv_row = (size_t)a.Hkv * D;
-  const float* Kb = (const float*)a.k + ((size_t)g.b * a.Lk * a.Hkv + g.hkv) * D;
-  const float* Vb = (const float*)a.v + ((size_t)g.b * a.Lk * a.Hkv + g.hkv) * D;
-  const bool row_in = g.qi < a.Lq;
-  const bool row_ok = g.qi < g.q_hi;
-
-  float qf[D / 2];
-  {
-    const float* qrow =
-        (const float*)a.q + ((size_t)(g.b * a.Lq + (row_in ? g.qi : 0)) * a.Hq + g.h) * D + half * (D / 2);
-#pragma unroll
-    for (int s = 0; s < D / 8; ++s) {
-      f32x4 r = {0.f, 0.f, 0.f, 0.f};
-      if (row_in) r = *(const f32x4*)(qrow + 4 * s);
-#pragma unroll
-      for (int j = 0; j < 4; ++j) qf[4 * s + j] = r[j];
-    }
-  }
-  const float* brow = nullptr;
-  if constexpr (BIAS) {
-    brow = a.bias + (size_t)g.b * a.bias_bstride + (size_t)g.h * a.bias_hstride +
-           (size_t)(row_in ? g.qi : 0) * a.Lk;
-  }
-  const bool bias_vec = (a.Lk & 3) == 0;
-  const float cx = (BIAS || EXT == 3) ? kLog2e : a.scale * kLog2e;
-  ExtRows er;
-  if constexpr (EXT > 0) er = ext_rows(a, g);
-
-  f32x16 acc[D / 32];
-#pragma unroll
-  for (int i = 0; i < D / 32; ++i) acc[i] = f32x16{};
-  float m_run = kMaxInit, l_run = 0.f;
-  const int t_begin = g.kv_begin / BK;
-  const int n_tiles = max((g.kv_stop + BK - 1) / BK - t_begin, 0);
-  const int q_last_w = g.qw + 31;
-
-  f32x4 kreg[PER_T], vreg[PER_T];
-  auto load_tile = [&](int t) {
-    const int k0 = (t_begin + t) * BK;
-#pragma unroll
-    for (int i = 0; i < PER_T; ++i) {
-      const int u = tid + kThreads * i;
-      const int kk = k0 + u / DC, dc = u % DC;
-      f32x4 rk = {0.f, 0.f, 0.f, 0.f}, rv = {0.f, 0.f, 0.f, 0.f};
-      if (kk < g.kv_stop) {
-        rk = *(const f32x4*)(Kb + (size_t)kk * kv_row + dc * 4);
-        rv = *(const f32x4*)(Vb + (size_t)kk * kv_row + dc * 4);
-      }
-      kreg[i] = rk;
-      vreg[i] = rv;
-    }
-  };
-  auto store_tile = [&](int buf) {
-#pragma unroll
-    for (int i = 0; i < PER_T; ++i) {
-      const int u = tid + kThreads * i;
-      *(f32x4*)(&k_lds[buf][(u / DC) * KS + (u % DC) * 4]) = kreg[i];
-      *(f32x4*)(&v_lds[buf][(u / DC) * VS + (u % DC) * 4]) = vreg[i];
-    }
-  };
-
-  auto compute = [&](int t, int buf) {
-    const int k0 = (t_begin + t) * BK;
-    if constexpr (EXT > 0) {
-      if (!er.any || k0 > er.hi_last || k0 + BK - 1 < er.lo_first) return;
-    } else {
-      if (a.causal && k0 > q_last_w) return;
-    }
-    const float* kl = k_lds[buf];
-    const float* vl = v_lds[buf];
-    f32x16 s[BK / 32];
-#pragma unroll
-    for (int kb = 0; kb < BK / 32; ++kb) {
-      s[kb] = f32x16{};
-      const float* kp = kl + (kb * 32 + col) * KS + half * (D / 2);
-#pragma unroll
-      for (int st4 = 0; st4 < D / 8; ++st4) {
-        const f32x4 kf = *(const f32x4*)(kp + 4 * st4);
-#pragma unroll
-        for (int j = 0; j < 4; ++j) s[kb] = mfma32x32x2f32(kf[j], qf[4 * st4 + j], s[kb]);
-      }
-    }
-    if constexpr (EXT == 3) {
-      ext_scores_sT<BK / 32, BIAS>(a, g, er, s, k0, half, brow, row_in,
-                                   [&](int kb, int r, float x, float) { s[kb][r] = x; });
-    } else if constexpr (BIAS) {
-#pragma unroll
-      for (int kb = 0; kb < BK / 32; ++kb)
-#pragma unroll
-        for (int gq = 0; gq < 4; ++gq) {
-          const int kk = k0 + kb * 32 + 8 * gq + 4 * half;
-          f32x4 bv = {0.f, 0.f, 0.f, 0.f};
-          if (row_in) bv = bias_vec ? load_bias4<true>(brow, kk, a.Lk) : load_bias4<false>(brow, kk, a.Lk);
-#pragma unroll
-          for (int j = 0; j < 4; ++j) s[kb][4 * gq + j] = fmaf(s[kb][4 * gq + j], a.scale, bv[j]);
-        }
-    }
-    if constexpr (EXT == 1) ext_mask_sT<BK / 32>(g, er, s, k0, half);
-    const bool need_mask = EXT == 0 && ((k0 + BK > g.kv_end) || (a.causal && k0 + BK - 1 > g.qw) ||
-                                        (g.qw + 31 >= g.q_hi));
-    if (need_mask) {
-#pragma unroll
-      for (int kb = 0; kb < BK / 32; ++kb)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          const int kk = k0 + kb * 32 + 8 * (r >> 2) + 4 * half + (r & 3);
-          const bool keep = row_ok && kk < g.kv_end && (!a.causal || kk <= g.qi);
-          if (!keep) s[kb][r] = -INFINITY;
-        }
-    }
-    float mx = -INFINITY;
-#pragma unroll
-    for (int kb = 0; kb < BK / 32; ++kb)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) mx = fmaxf(mx, s[kb][r]);
-    mx = xor32_max(mx);
-    const float m_new = fmaxf(m_run, mx * cx);
-    const float corr = fast_exp2(m_run - m_new);
-    m_run = m_new;
-    float rs = 0.f;
-#pragma unroll
-    for (int kb = 0; kb < BK / 32; ++kb)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const float p = fast_exp2(fmaf(s[kb][r], cx, -m_new));
-        rs += p;
-        s[kb][r] = p;
-      }
-    l_run = fmaf(l_run, corr, rs);
-#pragma unroll
-    for (int i = 0; i < D / 32; ++i)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) acc[i][r] *= corr;
-#pragma unroll
-    for (int db = 0; db < D / 32; ++db)
-#pragma unroll
-      for (int kb = 0; kb < BK / 32; ++kb)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          const int key = kb * 32 + 8 * (r >> 2) + 4 * half + (r & 3);
-          acc[db] = mfma32x32x2f32(vl[key * VS + db * 32 + col], s[kb][r], acc[db]);
-        }
-  };
-
-  if (n_tiles > 0) {
-    load_tile(0);
-    store_tile(0);
-  }
-  __syncthreads();
-  for (int t = 0; t < n_tiles; ++t) {
-    if (t + 1 < n_tiles) load_tile(t + 1);
-    compute(t, t & 1);
-    if (t + 1 < n_tiles) store_tile((t + 1) & 1);
-    __syncthreads();
-  }
-
-  const float l_tot = xor32_sum(l_run);
-  const float inv = l_tot > 0.f ? 1.f / l_tot : 0.f;
-  if (row_in) {
-    float* orow = (float*)a.o + ((size_t)(g.b * a.Lq + g.qi) * a.Hq + g.h) * D;
-#pragma unroll
-    for (int db = 0; db < D / 32; ++db)
-#pragma unroll
-      for (int gq = 0; gq < 4; ++gq) {
-        f32x4 v;
-#pragma unroll
-        for (int j = 0; j < 4; ++j) v[j] = acc[db][4 * gq + j] * inv;
-        *(f32x4*)(orow + db * 32 + 8 * gq + 4 * half) = v;
-      }
-    if (a.lse && half == 0)
-      a.lse[((size_t)g.b * a.Hq + g.h) * a.Lq + g.qi] =
-          l_tot > 0.f ? (m_run + __log2f(l_tot)) * kLn2 : INFINITY;
-  }
-}
-
-// ---------------------------------------------------------------------------
-// fp32, small grids: the key range of one 32-row query block is split over
-// the 8 waves of a workgroup, so a problem with few query tiles still spreads
-// over many SIMDs (the fp32 MFMA rate makes one wave's pass over all keys the
-// critical path otherwise).  Wave w takes 32-key blocks w, w+NW, w+2NW, ...;
+// fp32, head dim 128, small grids: the key range of one 32-row query block is
+// split over the waves of a workgroup, so a problem with few query tiles still
+// spreads over many SIMDs.  Wave w takes 32-key blocks w, w+NW, w+2NW, ...;
 // each block's K half-rows and V columns are loaded from global memory
 // straight into the MFMA operand registers (the next block's loads are in
 // flight while one is computed), so no LDS staging is needed.  Each wave
 // keeps its own online softmax; the partial (max, sum, O) are combined in LDS
-// at the end.  NW = 8 waves for D = 64; D = 128 uses 4 (one per SIMD): its
-// double-buffered operand blocks need more than the 256 registers of two
-// waves per SIMD.  Products and softmax are those of flash_fwd_f32_kernel
-// (v_mfma_f32_32x32x2f32, keys as MFMA rows).
+// at the end.  NW = 4 waves, one per SIMD: the double-buffered operand blocks
+// need more than the 256 registers of two.  Products on
+// v_mfma_f32_32x32x2f32, keys as MFMA rows: the k index of one step is the
+// wave half (half 0 contracts dim s, half 1 dim D/2 + s), so each lane reads a
+// contiguous half row of K, and the step of P.V pairs key (r, half 0) with key
+// (r, half 1) of the S^T layout, so V is read in its natural layout.
 // ---------------------------------------------------------------------------
 template <int D>
-constexpr int split_waves() { return D == 128 ? 4 : 8; }
+constexpr int split_waves() { return 4; }
 
 template <int D, bool BIAS>
 __global__ __launch_bounds__(64 * split_waves<D>(), 1) void flash_fwd_f32_split_kernel(FlashArgs a) {
@@ -1173,27 +977,14 @@ extern "C" int pjx_flash_fwd(int dtype, const void* q, const void* k, const void
   if (head_dim == 256) return dtype == PJX_DTYPE_F32 ? launch_flash_f32_wide(a, s) : launch_flash_wide256(a, s);
   if (dtype == PJX_DTYPE_BF16) return launch_h16<Bf16Fmt>(a, (int)head_dim, s);
   if (dtype == PJX_DTYPE_F16) return launch_h16<F16Fmt>(a, (int)head_dim, s);
-  if (a.ext) {
-    const bool full = a.ext >= 2;
-    if (head_dim == 128) {
-      if (full) return hb ? launch<flash_fwd_f32_kernel<128, true, 3>>(a, s) : launch<flash_fwd_f32_kernel<128, false, 3>>(a, s);
-      return hb ? launch<flash_fwd_f32_kernel<128, true, 1>>(a, s) : launch<flash_fwd_f32_kernel<128, false, 1>>(a, s);
-    }
-    if (full) return hb ? launch<flash_fwd_f32_kernel<64, true, 3>>(a, s) : launch<flash_fwd_f32_kernel<64, false, 3>>(a, s);
-    return hb ? launch<flash_fwd_f32_kernel<64, true, 1>>(a, s) : launch<flash_fwd_f32_kernel<64, false, 1>>(a, s);
-  }
-  // fp32 with fewer 128-row workgroups than CUs: split each query block's
-  // keys over several waves (latency-bound sizes, like the reference's CPU
-  // case).
-  if ((long)a.n_qtiles * batch * q_heads < 256) {
-    if (head_dim == 128)
-      return hb ? launch_split<128, flash_fwd_f32_split_kernel<128, true>>(a, s)
-                : launch_split<128, flash_fwd_f32_split_kernel<128, false>>(a, s);
-    return hb ? launch_split<64, flash_fwd_f32_split_kernel<64, true>>(a, s)
-              : launch_split<64, flash_fwd_f32_split_kernel<64, false>>(a, s);
-  }
-  if (head_dim == 128) return hb ? launch<flash_fwd_f32_kernel<128, true, 0>>(a, s) : launch<flash_fwd_f32_kernel<128, false, 0>>(a, s);
-  return hb ? launch<flash_fwd_f32_kernel<64, true, 0>>(a, s) : launch<flash_fwd_f32_kernel<64, false, 0>>(a, s);
+  // fp32 at head dim 128 with at most one 32-row block per CU: the keys of
+  // each block split over waves that read their operands from memory.  There
+  // the planes kernel's staging is latency nothing hides (33 against 38 us at
+  // B=1 H=4 L=512 causal; 163 against 85 us at B=4 H=8 L=1024).
+  if (head_dim == 128 && a.ext == 0 && (q_len + 31) / 32 * batch * q_heads <= 256)
+    return hb ? launch_split<128, flash_fwd_f32_split_kernel<128, true>>(a, s)
+              : launch_split<128, flash_fwd_f32_split_kernel<128, false>>(a, s);
+  return launch_flash_f32(a, (int)head_dim, s);
 }
 
 extern "C" int pjx_mla_fwd(int dtype, const void* q, const void* cache, void* o, float* lse,

@@ -1,0 +1,123 @@
+"""float32 attention on bf16 planes (forward and gradients, head dims 64 and
+128): every workgroup shape at tile edges against float64, and infinities and
+values beyond bf16's range against the same rule in float64.
+
+Bound: a product of planes drops terms below 2^-25 of it and every sum is
+float32; over at most a few hundred terms the relative error of an output (in
+2-norm) stays below 32 units of 2^-24 = 2e-6 (measured: 2e-7 to 7e-7).
+"""
+
+import math
+
+import pytest
+
+from tests._helpers import rng_normal, to_dev
+
+pytestmark = pytest.mark.gpu
+REL = 32 * 2.0 ** -24
+
+# D, B, Lq, Lk, Hq, Hkv, causal, forward, dq and dkdv workgroup shapes
+CASES = [
+    (64, 1, 1, 1, 1, 1, False, "64, 1, 4", "64, 1, 4", "64, 1, 4"),
+    (64, 2, 33, 129, 2, 1, False, "64, 1, 4", "64, 1, 4", "64, 1, 4"),
+    (64, 1, 257, 255, 4, 4, True, "64, 1, 4", "64, 1, 4", "64, 1, 4"),
+    (64, 3, 127, 300, 70, 14, True, "64, 2, 4", "64, 2, 4", "64, 2, 4"),
+    (64, 2, 65, 64, 140, 140, False, "64, 4, 2", "64, 4, 2", "64, 4, 2"),
+    (64, 1, 129, 191, 260, 260, True, "64, 4, 2", "64, 4, 2", "64, 4, 2"),
+    (128, 1, 31, 97, 2, 2, False, "split", "128, 2, 2", "128, 2, 2"),
+    (128, 2, 130, 95, 40, 20, True, "128, 2, 2", "128, 2, 2", "128, 2, 2"),
+    (128, 1, 161, 129, 260, 260, False, "128, 4, 1", "128, 4, 1", "128, 4, 1"),
+]
+
+
+def _attend64(q, k, v, scale, causal):
+    """float64 attention and the q, k, v it used (heads repeated for GQA)."""
+    import torch
+
+    q, k, v = (x.double().transpose(1, 2) for x in (q, k, v))
+    rep = q.shape[1] // k.shape[1]
+    s = torch.matmul(q, k.repeat_interleave(rep, 1).transpose(-1, -2).contiguous()) * scale
+    if causal:
+        keep = torch.ones(s.shape[-2:], dtype=torch.bool, device=s.device).tril()
+        s = s.masked_fill(~keep, float("-inf"))
+    return torch.matmul(torch.softmax(s, -1), v.repeat_interleave(rep, 1)).transpose(1, 2)
+
+
+def _rel(a, b):
+    return float((a.double() - b).norm() / b.norm().clamp_min(1e-300))
+
+
+@pytest.mark.parametrize("case", CASES)
+def test_shapes_against_float64(device, case):
+    import torch
+    from probjax_amd import native
+    from probjax_amd.hip_attention import flash_attention_bwd, flash_attention_fwd
+
+    D, B, Lq, Lk, Hq, Hkv, causal, fwd, dq, dkdv = case
+    print(f"f32 planes {case}", flush=True)
+    q, k, v, do = (to_dev(x, device, torch.float32) for x in rng_normal(
+        91, (B, Lq, Hq, D), (B, Lk, Hkv, D), (B, Lk, Hkv, D), (B, Lq, Hq, D)))
+    kw = dict(sm_scale=1 / math.sqrt(D), causal=causal)
+    o, lse = flash_attention_fwd(q, k, v, return_lse=True, **kw)
+    names = native.last_launches()
+    grads = flash_attention_bwd(q, k, v, o, do, lse, **kw)
+    names += native.last_launches()
+    prefix = ("flash_fwd_f32_split_kernel<" if fwd == "split" else f"flash_fwd_f32_planes_kernel<{fwd}",
+              f"flash_bwd_dq_f32_planes_kernel<{dq}", f"flash_bwd_dkdv_f32_planes_kernel<{dkdv}")
+    assert len(names) == 3 and all(n.startswith(p) for n, p in zip(names, prefix)), names
+    x = [t.double().requires_grad_() for t in (q, k, v)]
+    want = _attend64(*x, kw["sm_scale"], causal)
+    wg = torch.autograd.grad(want, x, do.double())
+    errs = [_rel(o, want.detach())] + [_rel(g, w) for g, w in zip(grads, wg)]
+    print(f"  rel {errs}", flush=True)
+    # one key: the softmax is constant and dq, dk are exactly 0 up to the rounding of dp - delta
+    if Lk == 1:
+        errs = [errs[0], errs[3]]
+    assert max(errs) <= REL, errs
+
+
+@pytest.mark.parametrize("D,H", [(64, 2), (64, 300), (128, 80)])
+def test_values_beyond_bf16_range(device, D, H):
+    """Infinite and float32's largest values in K and V take the float32
+    MFMAs: -inf scores drop their key, +inf scores make the row NaN, an
+    infinite V column is infinite, and finite values stay as accurate."""
+    import torch
+    from probjax_amd.hip_attention import flash_attention_bwd, flash_attention_fwd
+
+    B, L = 1, 100
+    q, k, v, do = (to_dev(x, device, torch.float32) for x in rng_normal(
+        92, (B, L, H, D), (B, L, H, D), (B, L, H, D), (B, L, H, D)))
+    kw = dict(sm_scale=1 / math.sqrt(D))
+    big = torch.finfo(torch.float32).max
+    # the largest finite value in V, reached with weight zero (its key's score is -inf)
+    k1, v1 = k.clone(), v.clone()
+    k1[0, 40] = 0
+    k1[0, 40, :, 3] = float("inf")
+    v1[0, 40] = big
+    o = flash_attention_fwd(q, k1, v1, **kw)
+    want = _attend64(q, k1, v1, kw["sm_scale"], False)
+    up = (q[0, :, :, 3] > 0)[None]
+    assert torch.isnan(o[up]).all()
+    assert _rel(o[~up], want[~up]) <= REL
+    # infinities in V: rows see them with positive weight
+    v2 = v.clone()
+    v2[0, 70, :, 5] = float("inf")
+    v2[0, 71, :, 6] = float("-inf")
+    o = flash_attention_fwd(q, k, v2, **kw)
+    assert torch.isposinf(o[..., 5]).all() and torch.isneginf(o[..., 6]).all()
+    rest = [i for i in range(D) if i not in (5, 6)]
+    want = _attend64(q, k, v, kw["sm_scale"], False)
+    assert _rel(o[..., rest], want[..., rest]) <= REL
+    # large finite values: K scaled up to float32's end, Q and sm_scale down, so
+    # that the scores are those of the unscaled call and dQ is 2^60 times its dQ
+    k3 = k * (3.9 / k.abs().max())
+    big_k, small_q, scale = k3 * 2.0 ** 126, q * 2.0 ** -60, kw["sm_scale"] * 2.0 ** -66
+    assert float(big_k.abs().max()) > 3.3e38
+    o3, lse3 = flash_attention_fwd(small_q, big_k, v, sm_scale=scale, return_lse=True)
+    x = [t.double().requires_grad_() for t in (q, k3, v)]
+    want = _attend64(*x, kw["sm_scale"], False)
+    wg = torch.autograd.grad(want, x, do.double())
+    dq, _, dv = flash_attention_bwd(small_q, big_k, v, o3, do, lse3, sm_scale=scale)
+    assert _rel(o3, want.detach()) <= REL
+    assert _rel(dq.double() * 2.0 ** -60, wg[0]) <= REL
+    assert _rel(dv, wg[2]) <= REL
