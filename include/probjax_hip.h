@@ -225,6 +225,34 @@ int pjx_flash_bwd(int dtype, const void* q, const void* k, const void* v, const 
                   float sm_scale, const pjx_score_mods* mods, void* stream);
 
 /*
+ * dL/d(bias) of pjx_flash_fwd with a dense bias, summed over the batches and
+ * heads the bias broadcasts to: dbias [bias_batch, bias_heads, Lq, Lk] fp32,
+ * fully written.  16-bit inputs, head_dim 64 or 128.  Call it after
+ * pjx_flash_bwd on the same stream with the same arguments: workspace is that
+ * call's, whose first 8 * batch * q_heads * q_len bytes (sm_scale * delta and
+ * the base-2 LSE) it reads.  (pjx_flash_bwd's own dbias argument gives the
+ * gradient per batch and query head instead, for every dtype and head_dim.)
+ */
+int pjx_flash_dbias(int dtype, const void* q, const void* k, const void* v, const void* dout,
+                    const void* workspace, float* dbias, const int32_t* kv_lengths, const float* bias,
+                    int64_t bias_batch, int64_t bias_heads, int64_t batch, int64_t q_len, int64_t kv_len,
+                    int64_t q_heads, int64_t kv_heads, int64_t head_dim, int64_t q_valid, int64_t kv_valid,
+                    int causal, float sm_scale, const pjx_score_mods* mods, void* stream);
+
+/*
+ * Flax's rule for rows without a valid key (lse [B, Hq, Lq] = +inf), which the
+ * attention kernels leave at zero: equal weights over every key
+ * (layers/attention.py:1298-1319 hands array masks to
+ * flax.linen.dot_product_attention).  grad 0: src is V [B, Lk, Hkv, D] and such
+ * rows of dst, the output [B, Lq, Hq, D], receive the mean of V.  grad 1: src is
+ * dO and dst dV [B, Lk, Hkv, D], every row of which gains the sum of such rows'
+ * dO over Lk.  head_dim <= 256.  Without such rows nothing is written.
+ */
+int pjx_empty_rows(int dtype, int grad, const float* lse, const void* src, void* dst, int64_t batch,
+                   int64_t q_len, int64_t kv_len, int64_t q_heads, int64_t kv_heads, int64_t head_dim,
+                   void* stream);
+
+/*
  * Bytes of workspace pjx_splitkv_decode / pjx_mla_decode need for these sizes
  * (partial outputs and log-sum-exp terms of every KV chunk).
  *   rows   -- query rows per (batch, kv head): (Hq/Hkv)*Lq for GQA decode,

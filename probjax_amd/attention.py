@@ -338,11 +338,15 @@ class _AttentionFunction(torch.autograd.Function):
     data get no cotangent, as in the reference (:3262-3263), unless the dense
     bias tensor is passed as ``bias``: then it is an input and receives
     dL/d(bias) (the gradient probjax's dense ``dot_product_attention`` path,
-    layers/attention.py:1293-1319, gives it)."""
+    layers/attention.py:1293-1319, gives it).  With ``fill`` rows without a
+    valid key follow Flax's rule (``pjx_empty_rows``)."""
 
     @staticmethod
-    def forward(ctx, query, key, value, bias, run_fwd, bwd_kwargs):
+    def forward(ctx, query, key, value, bias, run_fwd, bwd_kwargs, fill):
         out, lse = run_fwd(query, key, value)
+        if fill:
+            hip.empty_rows(lse, value, out, grad=False)
+        ctx.fill = fill
         ctx.save_for_backward(query, key, value, out, lse)
         ctx.bwd_kwargs = bwd_kwargs
         ctx.bias_dtype = None if bias is None else bias.dtype
@@ -353,11 +357,16 @@ class _AttentionFunction(torch.autograd.Function):
     def backward(ctx, dout, dlse=None):
         del dlse  # the LSE output is a residual, not differentiated
         q, k, v, o, lse = ctx.saved_tensors
+        db = None
         if ctx.bias_dtype is not None and ctx.needs_input_grad[3]:
-            dq, dk, dv, db = hip.flash_attention_bwd(q, k, v, o, dout, lse, bias_grad=True, **ctx.bwd_kwargs)
-            return dq, dk, dv, db.to(ctx.bias_dtype), None, None
-        dq, dk, dv = hip.flash_attention_bwd(q, k, v, o, dout, lse, **ctx.bwd_kwargs)
-        return dq, dk, dv, None, None, None
+            dq, dk, dv, db = hip.flash_attention_bwd(q, k, v, o, dout, lse, bias_grad=True, fold_bias_grad=True,
+                                                     **ctx.bwd_kwargs)
+            db = db.to(ctx.bias_dtype)
+        else:
+            dq, dk, dv = hip.flash_attention_bwd(q, k, v, o, dout, lse, **ctx.bwd_kwargs)
+        if ctx.fill:
+            hip.empty_rows(lse, dout, dv, grad=True)
+        return dq, dk, dv, db, None, None, None
 
 
 def _needs_grad(*ts) -> bool:
@@ -382,10 +391,12 @@ def _pad_features(x, width):
     return torch.nn.functional.pad(x, (0, width - x.shape[-1]))
 
 
-def _run(query, key, value, lm, lb, sm_scale, split_kv, bias_grad=False, want_lse=False):
+def _run(query, key, value, lm, lb, sm_scale, split_kv, bias_grad=False, fill=False):
     """Output of the HIP route for an eligible call (None: not computable
-    exactly); with ``want_lse`` ``(output, lse [B, Hq, Lq])``, where rows
-    without a valid key have ``lse = +inf``."""
+    exactly); with ``fill`` rows without a valid key follow Flax's rule: the
+    mean of V (``where(mask, logits, big_neg)`` gives such a row equal weights
+    over every key; with no keys at all the einsum over an empty key axis gives
+    the zeros the kernels return)."""
     d = query.shape[-1]
     width = _kernel_width(d, query.dtype)
     if width is not None and width != d:
@@ -394,10 +405,8 @@ def _run(query, key, value, lm, lb, sm_scale, split_kv, bias_grad=False, want_ls
         # width-d computation gives (the reference pads its blocks to
         # next_power_of_2(head_dim) with masked loads, kernels/attention.py:2168).
         res = _run(_pad_features(query, width), _pad_features(key, width), _pad_features(value, width),
-                   lm, lb, sm_scale, split_kv, bias_grad, want_lse)
-        if res is None:
-            return None
-        return (res[0][..., :d], res[1]) if want_lse else res[..., :d]
+                   lm, lb, sm_scale, split_kv, bias_grad, fill)
+        return None if res is None else res[..., :d]
     dense = None if lb is None else lb.dense
     bias_in = dense if bias_grad and dense is not None and _needs_grad(dense) else None
     grad = _needs_grad(query, key, value) or bias_in is not None
@@ -407,26 +416,37 @@ def _run(query, key, value, lm, lb, sm_scale, split_kv, bias_grad=False, want_ls
         plan = _decode_plan(query, key, value, lm, lb)
         if plan is not None:
             if not grad:
-                return hip.splitkv_decode(query, key, value, sm_scale=sm_scale, return_lse=want_lse, **plan)
+                return _filled(hip.splitkv_decode(query, key, value, sm_scale=sm_scale, return_lse=fill, **plan),
+                               value, fill)
             # Split-KV primal, regular backward (probjax splitkv_attention,
             # kernels/attention_splitkv.py:253-272).
             res = _AttentionFunction.apply(
                 query, key, value, None,
                 lambda q, k, v: hip.splitkv_decode(q, k, v, sm_scale=sm_scale, return_lse=True, **plan),
-                dict(sm_scale=sm_scale, kv_lengths=plan["kv_lengths"]),
+                dict(sm_scale=sm_scale, kv_lengths=plan["kv_lengths"]), fill,
             )
-            return res if want_lse else res[0]
+            return res[0]
     plan = _flash_plan(query, key, value, lm, lb)
     if plan is None:
         return None
     if not grad:
-        return hip.flash_attention_fwd(query, key, value, sm_scale=sm_scale, return_lse=want_lse, **plan)
+        return _filled(hip.flash_attention_fwd(query, key, value, sm_scale=sm_scale, return_lse=fill, **plan),
+                       value, fill)
     res = _AttentionFunction.apply(
         query, key, value, bias_in,
         lambda q, k, v: hip.flash_attention_fwd(q, k, v, sm_scale=sm_scale, return_lse=True, **plan),
-        dict(sm_scale=sm_scale, **plan),
+        dict(sm_scale=sm_scale, **plan), fill,
     )
-    return res if want_lse else res[0]
+    return res[0]
+
+
+def _filled(res, value, fill):
+    """The output of ``(output, lse)`` with Flax's rule applied to rows without
+    a valid key, or ``res`` itself without ``fill``."""
+    if not fill:
+        return res
+    hip.empty_rows(res[1], value, res[0], grad=False)
+    return res[0]
 
 
 # ---------------------------------------------------------------------------
@@ -919,9 +939,7 @@ def flex_attention(query, key, value, mask=None, bias=None, dropout_rng=None,
     e = _eligible(query, key, value, mask=mask, bias=bias, dropout_rate=active_dropout)
     if e is not None and (implementation == "hip" or device_table_enabled()):
         out = _run(query, key, value, e[0], e[1], float(sm_scale), split_kv, bias_grad=_bias_grad,
-                   want_lse=_flax_fill)
-        if out is not None and _flax_fill:
-            out = _flax_empty_rows(out[0], out[1], value)
+                   fill=_flax_fill)
     if out is None:
         raise ValueError(
             f"implementation={implementation!r}: "
@@ -938,8 +956,10 @@ def _flax_empty_rows(out, lse, value):
     """Flax's output for rows whose keys are all masked: ``where(mask,
     logits, big_neg)`` gives such a row equal weights over every key, so the
     mean of V (and dV = dO / Lk through autograd; no gradient reaches q, k or
-    the bias there).  The kernels leave such rows at zero with ``lse = +inf``,
-    so the fill is one device-side select, with no host synchronisation.
+    the bias there).  The kernels leave such rows at zero with ``lse = +inf``.
+    This states the rule in torch operations, for tensors anywhere; the calls
+    on the device apply ``hip.empty_rows``, in place and only where such a row
+    exists.
     With no keys at all the einsum over an empty key axis gives zeros, which
     the kernels already return."""
     l_k = value.shape[1]

@@ -178,6 +178,7 @@ def flash_attention_bwd(
     q, k, v, o, do, lse, *, sm_scale: float, causal: bool = False, kv_lengths=None, bias=None,
     q_valid: int | None = None, kv_valid: int | None = None, workspace=None,
     mods: ScoreModsArgs | None = None, bias_grad: bool = False, ds_route: bool | None = None,
+    fold_bias_grad: bool = False,
 ):
     """``pjx_flash_bwd``: gradients ``(dq, dk, dv)`` of ``flash_attention_fwd``
     (and, with ``bias_grad``, ``dbias``: dL/d(bias) summed to the bias's own
@@ -193,6 +194,10 @@ def flash_attention_bwd(
     modifiers) and its ``2 * B * Hq * Lq' * Lk'`` bytes of dS fit the budget
     (``_ds_budget``); True takes it whatever its size (ValueError where it
     does not exist); False never does.
+
+    ``fold_bias_grad`` (with ``bias_grad``): ``dbias`` from ``pjx_flash_dbias``,
+    summed over what the bias broadcasts to as it is computed (16-bit, head dim
+    64 or 128; elsewhere as without).
     """
     dev = _on_device(q, k, v, o, do, lse, bias)
     if q.ndim != 4 or k.ndim != 4 or v.ndim != 4:
@@ -227,7 +232,8 @@ def flash_attention_bwd(
     if bias_grad and bias is None:
         raise ValueError("bias_grad needs the bias")
     dq, dk, dv = torch.empty_like(q), torch.empty_like(k), torch.empty_like(v)
-    dbias = torch.zeros((B, Hq, Lq, Lk), dtype=torch.float32, device=dev) if bias_grad else None
+    fold = bias_grad and fold_bias_grad and D <= 128 and code != native.PJX_DTYPE_F32 and min(B, Lq, Lk) > 0
+    dbias = torch.zeros((B, Hq, Lq, Lk), dtype=torch.float32, device=dev) if bias_grad and not fold else None
     lib = native.load()
     nbytes = int(lib.pjx_flash_bwd_workspace_size(B, Hq, Lq))
     if workspace is None:
@@ -248,12 +254,39 @@ def flash_attention_bwd(
         int(bool(causal)), float(sm_scale), None if ms is None else ctypes.byref(ms[0]), _stream(dev),
     )
     native.check(rc)
+    if fold:
+        dbias = torch.empty_like(bias)
+        rc = lib.pjx_flash_dbias(
+            code, _ptr(q), _ptr(k), _ptr(v), _ptr(do), _ptr(ws), _ptr(dbias), _ptr(L), _ptr(bias), bb, bh, B, Lq, Lk,
+            Hq, Hkv, D, Lq if q_valid is None else int(q_valid), Lk if kv_valid is None else int(kv_valid),
+            int(bool(causal)), float(sm_scale), None if ms is None else ctypes.byref(ms[0]), _stream(dev),
+        )
+        native.check(rc)
+        return dq, dk, dv, dbias
     if dbias is None:
         return dq, dk, dv
     dims = [d for d, n in ((0, bb), (1, bh)) if n == 1]
     if dims:
         dbias = dbias.sum(dim=dims, keepdim=True)
     return dq, dk, dv, dbias
+
+
+def empty_rows(lse, src, dst, *, grad: bool) -> None:
+    """``pjx_empty_rows``: rows without a valid key (``lse`` = +inf) get the mean
+    of V (``src`` V, ``dst`` the output), or with ``grad`` add their ``dO / Lk``
+    (``src``) to ``dst`` = dV, in place."""
+    dev = _on_device(lse, src, dst)
+    out, val = (src, dst) if grad else (dst, src)
+    B, Lq, Hq, D = out.shape
+    _, Lk, Hkv, Dv = val.shape
+    if val.shape[0] != B or Dv != D or Hq % Hkv or tuple(lse.shape) != (B, Hq, Lq) or lse.dtype != torch.float32:
+        raise ValueError(f"incompatible shapes: output {tuple(out.shape)}, V {tuple(val.shape)}, lse {tuple(lse.shape)}")
+    if out.dtype != val.dtype or not dst.is_contiguous():
+        raise ValueError("output and V must share a dtype and the written one be contiguous")
+    lse, src = lse.contiguous(), src.contiguous()
+    rc = native.load().pjx_empty_rows(_dtype_code(out), int(grad), _ptr(lse), _ptr(src), _ptr(dst), B, Lq, Lk, Hq,
+                                      Hkv, D, _stream(dev))
+    native.check(rc)
 
 
 def _ds_budget(dev) -> int:

@@ -64,6 +64,15 @@ _SIGNATURES = {
         [ctypes.c_int, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, ctypes.c_size_t, _P, _P, _I64,
          _I64, _I64, _I64, _I64, _I64, _I64, _I64, _I64, _I64, ctypes.c_int, ctypes.c_float, _MODS, _P],
     ),
+    "pjx_flash_dbias": (
+        ctypes.c_int,
+        [ctypes.c_int, _P, _P, _P, _P, _P, _P, _P, _P, _I64, _I64, _I64, _I64, _I64, _I64, _I64, _I64, _I64,
+         _I64, ctypes.c_int, ctypes.c_float, _MODS, _P],
+    ),
+    "pjx_empty_rows": (
+        ctypes.c_int,
+        [ctypes.c_int, ctypes.c_int, _P, _P, _P, _I64, _I64, _I64, _I64, _I64, _I64, _P],
+    ),
     "pjx_decode_workspace_size": (ctypes.c_size_t, [_I64, _I64, _I64, _I64, _I64, _I64]),
     "pjx_splitkv_decode": (
         ctypes.c_int,

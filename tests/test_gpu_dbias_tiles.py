@@ -1,0 +1,94 @@
+"""dL/d(bias) folded over the broadcast (``pjx_flash_dbias``) against the
+per-(batch, head) gradient of the dQ kernel summed afterwards, and rows without
+a valid key (``pjx_empty_rows``) against the rule in torch operations.
+
+Both gradients recompute the same float32 P (dP - delta) per score from the
+same 16-bit operands (the sums inside a product may be ordered differently,
+2^-22 of the terms) and add B * Hq of them in float32: 1e-5 of the largest.
+"""
+
+import math
+
+import numpy as np
+import pytest
+
+from tests._helpers import rng_normal, to_dev, to_np
+
+pytestmark = pytest.mark.gpu
+
+CASES = [
+    # dtype, D, B, Lq, Lk, Hq, Hkv, bias batch, bias heads, causal, kv lengths, window / segments / slopes
+    ("bf16", 64, 3, 100, 130, 4, 2, 1, 4, False, [130, 64, 0], None),
+    ("f16", 128, 2, 65, 129, 2, 1, 1, 1, True, None, None),
+    ("bf16", 128, 2, 64, 128, 4, 4, 2, 4, False, None, None),
+    ("bf16", 64, 1, 1, 1, 1, 1, 1, 1, False, None, None),
+    ("bf16", 64, 2, 200, 190, 2, 2, 2, 1, True, [190, 77], None),
+    ("f16", 64, 2, 150, 150, 4, 2, 1, 4, True, None, "window"),
+    ("bf16", 128, 2, 97, 97, 2, 2, 1, 2, True, None, "segments"),
+    ("bf16", 64, 2, 97, 161, 2, 2, 1, 2, False, None, "slopes"),
+]
+
+
+@pytest.mark.parametrize("case", CASES)
+def test_folded_equals_summed(device, case):
+    import torch
+    from probjax_amd import hip_attention as hip
+    from probjax_amd import native
+
+    dtype, D, B, Lq, Lk, Hq, Hkv, bb, bh, causal, lengths, ext = case
+    print(f"dbias {case}", flush=True)
+    tdt = torch.bfloat16 if dtype == "bf16" else torch.float16
+    q, k, v, do = (to_dev(x, device, tdt) for x in rng_normal(51, (B, Lq, Hq, D), (B, Lk, Hkv, D), (B, Lk, Hkv, D),
+                                                              (B, Lq, Hq, D)))
+    bias = to_dev(rng_normal(52, (bb, bh, Lq, Lk), scale=0.5)[0], device, torch.float32)
+    bias[0, 0, 0, : Lk // 2] = float("-inf")
+    mods = None
+    if ext == "window":
+        mods = hip.ScoreModsArgs(window_left=40)
+    elif ext == "segments":
+        ids = torch.from_numpy(np.sort(np.random.default_rng(53).integers(0, 4, (B, Lq))).astype(np.int32)).to(device)
+        mods = hip.ScoreModsArgs(segment_q=ids, segment_k=ids)
+    elif ext == "slopes":
+        mods = hip.ScoreModsArgs(alibi_slopes=torch.full((Hq,), 0.25, device=device), alibi_symmetric=True, softcap=9.0)
+    L = None if lengths is None else torch.tensor(lengths, dtype=torch.int32, device=device)
+    kw = dict(sm_scale=1 / math.sqrt(D), causal=causal, kv_lengths=L, bias=bias, mods=mods)
+    o, lse = hip.flash_attention_fwd(q, k, v, return_lse=True, **kw)
+    want = hip.flash_attention_bwd(q, k, v, o, do, lse, bias_grad=True, **kw)
+    got = hip.flash_attention_bwd(q, k, v, o, do, lse, bias_grad=True, fold_bias_grad=True, **kw)
+    E = "Bf16Fmt" if dtype == "bf16" else "F16Fmt"
+    assert native.last_launches() == [f"flash_dbias_kernel<{E}, {D}, {D // 32}, {'true' if ext else 'false'}>"]
+    torch.cuda.synchronize()
+    for a, b in zip(got[:3], want[:3]):
+        np.testing.assert_allclose(to_np(a), to_np(b), rtol=2.0 ** -7, atol=2.0 ** -7 * float(b.float().abs().max()))
+    a, b = to_np(got[3]), to_np(want[3])
+    assert a.shape == b.shape == (bb, bh, Lq, Lk)
+    assert np.isfinite(a).all()
+    assert np.abs(a - b).max() <= 1e-5 * max(1.0, np.abs(b).max())
+
+
+@pytest.mark.parametrize("dtype,B,Lq,Lk,Hq,Hkv,D", [
+    ("bf16", 2, 70, 33, 4, 2, 64), ("f32", 1, 1, 257, 3, 3, 96), ("f16", 2, 300, 5, 8, 1, 256), ("f32", 2, 9, 1, 2, 1, 3)])
+def test_empty_rows(device, dtype, B, Lq, Lk, Hq, Hkv, D):
+    import torch
+    from probjax_amd import attention as A
+    from probjax_amd import hip_attention as hip
+
+    tdt = {"bf16": torch.bfloat16, "f16": torch.float16, "f32": torch.float32}[dtype]
+    o, v, do = (to_dev(x, device, tdt) for x in rng_normal(54, (B, Lq, Hq, D), (B, Lk, Hkv, D), (B, Lq, Hq, D)))
+    lse = torch.zeros((B, Hq, Lq), device=device)
+    for share in (0.0, 0.4, 1.0):
+        lse[torch.rand(lse.shape, device=device) < share] = float("inf")
+        x = v.clone().requires_grad_()
+        want = A._flax_empty_rows(o, lse, x)
+        (dv,) = torch.autograd.grad(want, x, do)
+        got, dgot = o.clone(), torch.zeros_like(v)
+        hip.empty_rows(lse, v, got, grad=False)
+        hip.empty_rows(lse, do, dgot, grad=True)
+        if share == 0.0:
+            assert torch.equal(got, o) and not dgot.any()
+        # float32 sums in another order that may round to neighbours: one spacing of the format, at most
+        # 2^-7 / 2^-10 of the value (torch rounds dV's mean and the sum over heads more often: 4 spacings)
+        eps = {"bf16": 2.0 ** -7, "f16": 2.0 ** -10, "f32": 2.0 ** -20}[dtype]
+        want, dv = want.detach().float(), dv.float()
+        assert float((got.float() - want).abs().max()) <= eps * float(want.abs().max())
+        assert float((dgot.float() - dv).abs().max()) <= 4 * eps * max(float(dv.abs().max()), 1e-6)
