@@ -149,6 +149,20 @@ int pjx_flash_fwd(int dtype, const void* q, const void* k, const void* v, void* 
                   const pjx_score_mods* mods, void* stream);
 
 /*
+ * pjx_flash_fwd on rows of row_dim elements (a multiple of 8, at most head_dim,
+ * which is 64 or 128): q, k, v and o are [B, L, H, row_dim], 16-byte aligned,
+ * and the missing features count as zeros, which change no score and no output
+ * element (the reference pads its blocks to next_power_of_2(head_dim) with
+ * masked loads, kernels/attention.py:2168).  head_dim names the kernel width.
+ */
+int pjx_flash_fwd_rows(int dtype, const void* q, const void* k, const void* v, void* o,
+                       float* lse, const int32_t* kv_lengths, const float* bias,
+                       int64_t bias_batch, int64_t bias_heads, int64_t batch, int64_t q_len,
+                       int64_t kv_len, int64_t q_heads, int64_t kv_heads, int64_t head_dim,
+                       int64_t row_dim, int64_t q_valid, int64_t kv_valid, int causal, float sm_scale,
+                       const pjx_score_mods* mods, void* stream);
+
+/*
  * Bytes of workspace pjx_flash_bwd needs: two fp32 values per query row
  * (sm_scale * delta, delta = sum_d o*do, and the base-2 LSE),
  * 8 * batch * q_heads * q_len.
@@ -225,10 +239,23 @@ int pjx_flash_bwd(int dtype, const void* q, const void* k, const void* v, const 
                   float sm_scale, const pjx_score_mods* mods, void* stream);
 
 /*
+ * pjx_flash_bwd on rows of row_dim elements (as pjx_flash_fwd_rows): dq, dk and
+ * dv have row_dim elements per row too.  The workspace sizes are head_dim's.
+ */
+int pjx_flash_bwd_rows(int dtype, const void* q, const void* k, const void* v, const void* o,
+                       const void* dout, const float* lse, void* dq, void* dk, void* dv,
+                       float* dbias, void* workspace, size_t workspace_bytes, const int32_t* kv_lengths,
+                       const float* bias, int64_t bias_batch, int64_t bias_heads, int64_t batch,
+                       int64_t q_len, int64_t kv_len, int64_t q_heads, int64_t kv_heads,
+                       int64_t head_dim, int64_t row_dim, int64_t q_valid, int64_t kv_valid, int causal,
+                       float sm_scale, const pjx_score_mods* mods, void* stream);
+
+/*
  * dL/d(bias) of pjx_flash_fwd with a dense bias, summed over the batches and
  * heads the bias broadcasts to: dbias [bias_batch, bias_heads, Lq, Lk] fp32,
- * fully written.  16-bit inputs, head_dim 64 or 128.  Call it after
- * pjx_flash_bwd on the same stream with the same arguments: workspace is that
+ * fully written.  16-bit inputs, head_dim 64 or 128, rows of row_dim elements
+ * (pjx_flash_fwd_rows; head_dim for plain ones).  Call it after pjx_flash_bwd
+ * or pjx_flash_bwd_rows on the same stream with the same arguments: workspace is that
  * call's, whose first 8 * batch * q_heads * q_len bytes (sm_scale * delta and
  * the base-2 LSE) it reads.  (pjx_flash_bwd's own dbias argument gives the
  * gradient per batch and query head instead, for every dtype and head_dim.)
@@ -236,8 +263,8 @@ int pjx_flash_bwd(int dtype, const void* q, const void* k, const void* v, const 
 int pjx_flash_dbias(int dtype, const void* q, const void* k, const void* v, const void* dout,
                     const void* workspace, float* dbias, const int32_t* kv_lengths, const float* bias,
                     int64_t bias_batch, int64_t bias_heads, int64_t batch, int64_t q_len, int64_t kv_len,
-                    int64_t q_heads, int64_t kv_heads, int64_t head_dim, int64_t q_valid, int64_t kv_valid,
-                    int causal, float sm_scale, const pjx_score_mods* mods, void* stream);
+                    int64_t q_heads, int64_t kv_heads, int64_t head_dim, int64_t row_dim, int64_t q_valid,
+                    int64_t kv_valid, int causal, float sm_scale, const pjx_score_mods* mods, void* stream);
 
 /*
  * Flax's rule for rows without a valid key (lse [B, Hq, Lq] = +inf), which the

@@ -399,7 +399,11 @@ def _run(query, key, value, lm, lb, sm_scale, split_kv, bias_grad=False, fill=Fa
     the zeros the kernels return)."""
     d = query.shape[-1]
     width = _kernel_width(d, query.dtype)
-    if width is not None and width != d:
+    rows = None
+    if width is not None and width != d and not _splitkv_ok(query, key, lm, lb is not None, 0.0, split_kv):
+        # the flash kernels take such rows as they lie in memory
+        rows = hip.rows_width(d, max(query.shape[2], key.shape[2]))
+    if width is not None and width != d and rows is None:
         # Zero features change no q.k product and add only zero output
         # columns: every kept score, weight and output element is the one the
         # width-d computation gives (the reference pads its blocks to
@@ -412,7 +416,7 @@ def _run(query, key, value, lm, lb, sm_scale, split_kv, bias_grad=False, fill=Fa
     grad = _needs_grad(query, key, value) or bias_in is not None
     if grad and query.dtype not in BACKWARD_DTYPES:
         return None
-    if _splitkv_ok(query, key, lm, lb is not None, 0.0, split_kv):
+    if rows is None and _splitkv_ok(query, key, lm, lb is not None, 0.0, split_kv):
         plan = _decode_plan(query, key, value, lm, lb)
         if plan is not None:
             if not grad:
@@ -426,9 +430,11 @@ def _run(query, key, value, lm, lb, sm_scale, split_kv, bias_grad=False, fill=Fa
                 dict(sm_scale=sm_scale, kv_lengths=plan["kv_lengths"]), fill,
             )
             return res[0]
-    plan = _flash_plan(query, key, value, lm, lb)
+    plan = _flash_plan(query, key, value, lm, lb, check_dim=rows is None)
     if plan is None:
         return None
+    if rows is not None:
+        plan["width"] = rows
     if not grad:
         return _filled(hip.flash_attention_fwd(query, key, value, sm_scale=sm_scale, return_lse=fill, **plan),
                        value, fill)

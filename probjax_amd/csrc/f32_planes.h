@@ -125,14 +125,14 @@ struct PlaneTile {
 // a buffer: lane offsets stay below 8 rows whatever the tensor's size, and
 // rows at or past `end` read as zeros.
 template <int D>
-__device__ __forceinline__ rsrc_t wave_rows(const unsigned char* base, int row, int end, uint32_t row_bytes) {
+__device__ __forceinline__ rsrc_t wave_rows(const unsigned char* base, int row, int end, uint32_t row_bytes, int rdim) {
   const int n = min(end - row, 512 / D);
-  return make_rsrc(base + (size_t)(n > 0 ? row : 0) * row_bytes, n > 0 ? (uint32_t)(n - 1) * row_bytes + D * 4 : 0u);
+  return make_rsrc(base + (size_t)(n > 0 ? row : 0) * row_bytes, n > 0 ? (uint32_t)(n - 1) * row_bytes + rdim * 4 : 0u);
 }
 template <int D>
-__device__ __forceinline__ uint32_t wave_rows_offset(uint32_t row_bytes) {
-  const int lane = threadIdx.x & 63;
-  return (lane / (D / 8)) * row_bytes + 32 * (lane % (D / 8));
+__device__ __forceinline__ uint32_t wave_rows_offset(uint32_t row_bytes, int rdim) {
+  const int lane = threadIdx.x & 63, c = lane % (D / 8);
+  return 8 * c < rdim ? (lane / (D / 8)) * row_bytes + 32 * c : kPastBuffer;
 }
 
 // Geometry of a workgroup of `rows` query rows whose wave owns rows 32*strip ..

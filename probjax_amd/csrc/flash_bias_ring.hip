@@ -79,9 +79,10 @@ __global__ __launch_bounds__(G_ * kThreads, 1) void flash_fwd_bf16_bias_ring_ker
   g.qw = __builtin_amdgcn_readfirstlane(g.q0 + 32 * w);
   g.qi = g.qw + (tid & 31);
   const int col = lane & 31, half = lane >> 5;
-  const uint32_t rowstride = (uint32_t)a.Hkv * D * 2;
-  const unsigned char* Kb = (const unsigned char*)a.k + ((size_t)g.b * a.Lk * a.Hkv + g.hkv) * ROWB;
-  const unsigned char* Vb = (const unsigned char*)a.v + ((size_t)g.b * a.Lk * a.Hkv + g.hkv) * ROWB;
+  const int rdim = a.rdim;
+  const uint32_t rowstride = (uint32_t)a.Hkv * rdim * 2;
+  const unsigned char* Kb = (const unsigned char*)a.k + ((size_t)g.b * a.Lk * a.Hkv + g.hkv) * rdim * 2;
+  const unsigned char* Vb = (const unsigned char*)a.v + ((size_t)g.b * a.Lk * a.Hkv + g.hkv) * rdim * 2;
   const float* bslice = a.bias + (size_t)g.b * a.bias_bstride + (size_t)g.h * a.bias_hstride;
   const uint32_t slice_bytes = (uint32_t)a.Lq * (uint32_t)a.Lk * 4u;
   const bool row_in = g.qi < a.Lq;
@@ -90,11 +91,11 @@ __global__ __launch_bounds__(G_ * kThreads, 1) void flash_fwd_bf16_bias_ring_ker
   typename E::v8 qf[D / 16];
   {
     const uint16_t* qrow =
-        (const uint16_t*)a.q + ((size_t)(g.b * a.Lq + (row_in ? g.qi : 0)) * a.Hq + g.h) * D;
+        (const uint16_t*)a.q + ((size_t)(g.b * a.Lq + (row_in ? g.qi : 0)) * a.Hq + g.h) * rdim;
 #pragma unroll
     for (int s = 0; s < D / 16; ++s) {
       u32x4 raw = {0u, 0u, 0u, 0u};
-      if (row_in) raw = *(const u32x4*)(qrow + 16 * s + 8 * half);
+      if (row_in && 16 * s + 8 * half < rdim) raw = *(const u32x4*)(qrow + 16 * s + 8 * half);
       qf[s] = E::as8(raw);
     }
   }
@@ -105,8 +106,8 @@ __global__ __launch_bounds__(G_ * kThreads, 1) void flash_fwd_bf16_bias_ring_ker
 #pragma unroll
   for (int j = 0; j < T::NLD; ++j) {
     const int r = 8 * w + T::RPI * j + lane / T::NC, slot = lane % T::NC;
-    voffK[j] = r * rowstride + 16 * (slot ^ T::swz_k(r));
-    voffV[j] = r * rowstride + 16 * (slot ^ T::swz_v(r));
+    voffK[j] = row_chunk(r, rowstride, slot ^ T::swz_k(r), rdim);
+    voffV[j] = row_chunk(r, rowstride, slot ^ T::swz_v(r), rdim);
   }
   uint32_t voffB[R::NLB];
 #pragma unroll
@@ -146,7 +147,7 @@ __global__ __launch_bounds__(G_ * kThreads, 1) void flash_fwd_bf16_bias_ring_ker
     unsigned char* ks = slot + grp * STAGE_B;
     const int nvalid = max(0, min(BK, g.kv_stop - k0));
     const uint32_t kvbytes =
-        __builtin_amdgcn_readfirstlane(nvalid > 0 ? (uint32_t)(nvalid - 1) * rowstride + ROWB : 0u);
+        __builtin_amdgcn_readfirstlane(nvalid > 0 ? (uint32_t)(nvalid - 1) * rowstride + rdim * 2 : 0u);
     const rsrc_t rk = make_rsrc(Kb + (size_t)max(k0, 0) * rowstride, kvbytes);
     const rsrc_t rv = make_rsrc(Vb + (size_t)max(k0, 0) * rowstride, kvbytes);
 #pragma unroll
@@ -318,11 +319,12 @@ __global__ __launch_bounds__(G_ * kThreads, 1) void flash_fwd_bf16_bias_ring_ker
   const float l_tot = xor32_sum(lsum);
   const float inv = l_tot > 0.f ? 1.f / l_tot : 0.f;
   if (row_in) {
-    uint16_t* orow = (uint16_t*)a.o + ((size_t)(g.b * a.Lq + g.qi) * a.Hq + g.h) * D;
+    uint16_t* orow = (uint16_t*)a.o + ((size_t)(g.b * a.Lq + g.qi) * a.Hq + g.h) * rdim;
 #pragma unroll
     for (int db = 0; db < D / 32; ++db)
 #pragma unroll
       for (int gq = 0; gq < 4; ++gq) {
+        if (db * 32 + 8 * gq >= rdim) continue;
         u32x2 pk;
         pk[0] = E::pack2(acc[db][4 * gq] * inv, acc[db][4 * gq + 1] * inv);
         pk[1] = E::pack2(acc[db][4 * gq + 2] * inv, acc[db][4 * gq + 3] * inv);

@@ -76,7 +76,7 @@ static int run_bwd_h16(const FlashBwdArgs& a, bool hb, hipStream_t s) {
     rc = hb ? launch_dkdv<flash_bwd_dkdv_kernel<E, D, true, EXT>>(a, s)
             : launch_dkdv<flash_bwd_dkdv_kernel<E, D, false, EXT>>(a, s);
   if (rc != PJX_OK || a.nsplit == 1) return rc;
-  const size_t n = (size_t)a.f.B * a.f.Lk * a.f.Hkv * D;
+  const size_t n = (size_t)a.f.B * a.f.Lk * a.f.Hkv * a.f.rdim;
   launch_kernel<bwd_split_reduce_kernel<E>>(dim3((unsigned)((n / 4 + kThreads - 1) / kThreads), 2), dim3(kThreads), 0, s,
                                             (const float*)a.part, a.nsplit, n, (uint16_t*)a.dk, (uint16_t*)a.dv);
   return check_launch("pjx_flash_bwd (split sum)");
@@ -126,14 +126,13 @@ extern "C" size_t pjx_flash_bwd_ds_workspace_size(int dtype, int64_t batch, int6
          wide_bwd_ds_bytes(batch, q_heads, q_len, kv_len);
 }
 
-extern "C" int pjx_flash_bwd(int dtype, const void* q, const void* k, const void* v, const void* o,
-                             const void* dout, const float* lse, void* dq, void* dk, void* dv,
-                             float* dbias, void* workspace, size_t workspace_bytes, const int32_t* kv_lengths,
-                             const float* bias, int64_t bias_batch, int64_t bias_heads,
-                             int64_t batch, int64_t q_len, int64_t kv_len, int64_t q_heads,
-                             int64_t kv_heads, int64_t head_dim, int64_t q_valid, int64_t kv_valid,
-                             int causal, float sm_scale, const pjx_score_mods* mods, void* stream) {
-  clear_error();
+static int flash_bwd(int dtype, const void* q, const void* k, const void* v, const void* o,
+                     const void* dout, const float* lse, void* dq, void* dk, void* dv,
+                     float* dbias, void* workspace, size_t workspace_bytes, const int32_t* kv_lengths,
+                     const float* bias, int64_t bias_batch, int64_t bias_heads,
+                     int64_t batch, int64_t q_len, int64_t kv_len, int64_t q_heads,
+                     int64_t kv_heads, int64_t head_dim, int64_t row_dim, int64_t q_valid, int64_t kv_valid,
+                     int causal, float sm_scale, const pjx_score_mods* mods, void* stream) {
   if (dtype != PJX_DTYPE_BF16 && dtype != PJX_DTYPE_F16 && dtype != PJX_DTYPE_F32)
     return fail(PJX_ERR_INVALID, "pjx_flash_bwd: dtype must be PJX_DTYPE_BF16, PJX_DTYPE_F16 or PJX_DTYPE_F32");
   // zero-element tensors may come as null pointers
@@ -161,9 +160,9 @@ extern "C" int pjx_flash_bwd(int dtype, const void* q, const void* k, const void
     hipStream_t s0 = (hipStream_t)stream;
     const char* who = "pjx_flash_bwd";
     auto zero = [&](void* p, size_t n) { return f32 ? fill_u32(p, 0u, n, s0, who) : zero_u16(p, n, s0, who); };
-    if (kv_len == 0) return zero(dq, (size_t)(batch * q_len * q_heads * head_dim));
-    const int rc = zero(dk, (size_t)(batch * kv_len * kv_heads * head_dim));
-    return rc != PJX_OK ? rc : zero(dv, (size_t)(batch * kv_len * kv_heads * head_dim));
+    if (kv_len == 0) return zero(dq, (size_t)(batch * q_len * q_heads * row_dim));
+    const int rc = zero(dk, (size_t)(batch * kv_len * kv_heads * row_dim));
+    return rc != PJX_OK ? rc : zero(dv, (size_t)(batch * kv_len * kv_heads * row_dim));
   }
   const size_t need = pjx_flash_bwd_workspace_size(batch, q_heads, q_len);
   if (need > 0 && (!workspace || workspace_bytes < need))
@@ -183,6 +182,7 @@ extern "C" int pjx_flash_bwd(int dtype, const void* q, const void* k, const void
   a.causal = causal ? 1 : 0;
   a.f16 = dtype == PJX_DTYPE_F16;
   a.scale = sm_scale;
+  a.rdim = (int)row_dim;
   a.n_qtiles = (int)((q_len + kBQ - 1) / kBQ);
   if ((long)a.n_qtiles * batch * q_heads > 0x7fffffffL ||
       (long)((kv_len + kBKV - 1) / kBKV) * batch * kv_heads > 0x7fffffffL)
@@ -245,4 +245,33 @@ extern "C" int pjx_flash_bwd(int dtype, const void* q, const void* k, const void
     return head_dim == 128 ? run_dkdv_f32_128(ba, s) : run_dkdv_f32_64(ba, s);
   }
   return head_dim == 128 ? run_bwd<128>(ba, dtype, hb, s) : run_bwd<64>(ba, dtype, hb, s);
+}
+
+extern "C" int pjx_flash_bwd(int dtype, const void* q, const void* k, const void* v, const void* o,
+                             const void* dout, const float* lse, void* dq, void* dk, void* dv,
+                             float* dbias, void* workspace, size_t workspace_bytes, const int32_t* kv_lengths,
+                             const float* bias, int64_t bias_batch, int64_t bias_heads,
+                             int64_t batch, int64_t q_len, int64_t kv_len, int64_t q_heads,
+                             int64_t kv_heads, int64_t head_dim, int64_t q_valid, int64_t kv_valid,
+                             int causal, float sm_scale, const pjx_score_mods* mods, void* stream) {
+  clear_error();
+  return flash_bwd(dtype, q, k, v, o, dout, lse, dq, dk, dv, dbias, workspace, workspace_bytes, kv_lengths, bias,
+                   bias_batch, bias_heads, batch, q_len, kv_len, q_heads, kv_heads, head_dim, head_dim, q_valid,
+                   kv_valid, causal, sm_scale, mods, stream);
+}
+
+extern "C" int pjx_flash_bwd_rows(int dtype, const void* q, const void* k, const void* v, const void* o,
+                                  const void* dout, const float* lse, void* dq, void* dk, void* dv,
+                                  float* dbias, void* workspace, size_t workspace_bytes, const int32_t* kv_lengths,
+                                  const float* bias, int64_t bias_batch, int64_t bias_heads,
+                                  int64_t batch, int64_t q_len, int64_t kv_len, int64_t q_heads,
+                                  int64_t kv_heads, int64_t head_dim, int64_t row_dim, int64_t q_valid,
+                                  int64_t kv_valid, int causal, float sm_scale, const pjx_score_mods* mods,
+                                  void* stream) {
+  clear_error();
+  const int rc = check_row_dim(head_dim, row_dim, q_heads, kv_heads, "pjx_flash_bwd_rows");
+  if (rc != PJX_OK) return rc;
+  return flash_bwd(dtype, q, k, v, o, dout, lse, dq, dk, dv, dbias, workspace, workspace_bytes, kv_lengths, bias,
+                   bias_batch, bias_heads, batch, q_len, kv_len, q_heads, kv_heads, head_dim, row_dim, q_valid,
+                   kv_valid, causal, sm_scale, mods, stream);
 }

@@ -186,9 +186,10 @@ __global__ __launch_bounds__(NG * kThreads, (D <= 128 ? 2 : 1)) void flash_bwd_d
   unsigned char* const st0 = smem0 + gi * STAGE_B;  // this group's stages
   unsigned char* const st1 = smem1 + gi * STAGE_B;
   const int col = lane & 31, half = lane >> 5;
-  const uint32_t rowstride = (uint32_t)a.Hkv * D * 2;
-  const unsigned char* Kb = (const unsigned char*)a.k + ((size_t)g.b * a.Lk * a.Hkv + g.hkv) * ROWB;
-  const unsigned char* Vb = (const unsigned char*)a.v + ((size_t)g.b * a.Lk * a.Hkv + g.hkv) * ROWB;
+  const int rdim = a.rdim;
+  const uint32_t rowstride = (uint32_t)a.Hkv * rdim * 2;
+  const unsigned char* Kb = (const unsigned char*)a.k + ((size_t)g.b * a.Lk * a.Hkv + g.hkv) * rdim * 2;
+  const unsigned char* Vb = (const unsigned char*)a.v + ((size_t)g.b * a.Lk * a.Hkv + g.hkv) * rdim * 2;
   const bool row_in = g.qi < a.Lq;
   const bool row_ok = g.qi < g.q_hi;
 
@@ -197,14 +198,14 @@ __global__ __launch_bounds__(NG * kThreads, (D <= 128 ? 2 : 1)) void flash_bwd_d
   typename E::v8 qf[D / 16], dof[D / 16];
   float dsum = 0.f;
   {
-    const size_t roff = ((size_t)(g.b * a.Lq + (row_in ? g.qi : 0)) * a.Hq + g.h) * D;
+    const size_t roff = ((size_t)(g.b * a.Lq + (row_in ? g.qi : 0)) * a.Hq + g.h) * rdim;
     const uint16_t* qrow = (const uint16_t*)a.q + roff;
     const uint16_t* drow = (const uint16_t*)ba.dout + roff;
     const uint16_t* orow = (const uint16_t*)a.o + roff;
 #pragma unroll
     for (int s = 0; s < D / 16; ++s) {
       u32x4 rq = {0u, 0u, 0u, 0u}, rd = rq, ro = rq;
-      if (row_in) {
+      if (row_in && 16 * s + 8 * half < rdim) {
         rq = *(const u32x4*)(qrow + 16 * s + 8 * half);
         rd = *(const u32x4*)(drow + 16 * s + 8 * half);
         ro = *(const u32x4*)(orow + 16 * s + 8 * half);
@@ -243,7 +244,7 @@ __global__ __launch_bounds__(NG * kThreads, (D <= 128 ? 2 : 1)) void flash_bwd_d
 #pragma unroll
   for (int j = 0; j < T::NLD; ++j) {
     const int r = 16 * w + T::RPI * j + lane / T::NC, slot = lane % T::NC;
-    voff[j] = r * rowstride + 16 * (slot ^ T::swz(r));
+    voff[j] = row_chunk(r, rowstride, slot ^ T::swz(r), rdim);
   }
   BwdOffsets<D> off;
   off.init(lane, gi * STAGE_B);  // fragment reads address the group's stage from smem0 / smem1
@@ -259,7 +260,7 @@ __global__ __launch_bounds__(NG * kThreads, (D <= 128 ? 2 : 1)) void flash_bwd_d
   auto issue = [&](int t, unsigned char* ks) {
     const int k0 = (t_begin + t) * BK;
     const int nvalid = min(BK, g.kv_stop - k0);
-    const uint32_t bytes = (uint32_t)(nvalid - 1) * rowstride + ROWB;
+    const uint32_t bytes = (uint32_t)(nvalid - 1) * rowstride + rdim * 2;
     const rsrc_t rk = make_rsrc(Kb + (size_t)k0 * rowstride, bytes);
     const rsrc_t rv = make_rsrc(Vb + (size_t)k0 * rowstride, bytes);
 #pragma unroll
@@ -429,11 +430,12 @@ __global__ __launch_bounds__(NG * kThreads, (D <= 128 ? 2 : 1)) void flash_bwd_d
   }
 
   if (row_in) {
-    uint16_t* drow = (uint16_t*)ba.dq + ((size_t)(g.b * a.Lq + g.qi) * a.Hq + g.h) * D;
+    uint16_t* drow = (uint16_t*)ba.dq + ((size_t)(g.b * a.Lq + g.qi) * a.Hq + g.h) * rdim;
 #pragma unroll
     for (int db = 0; db < D / 32; ++db)
 #pragma unroll
       for (int gq = 0; gq < 4; ++gq) {
+        if (db * 32 + 8 * gq >= rdim) continue;
         u32x2 pk;
         pk[0] = E::pack2(acc[db][4 * gq], acc[db][4 * gq + 1]);
         pk[1] = E::pack2(acc[db][4 * gq + 2], acc[db][4 * gq + 3]);
@@ -469,6 +471,7 @@ __global__ __launch_bounds__(NG * kThreads, (D <= 128 ? 2 : 1)) void flash_bwd_d
   unsigned char* const st0 = smem0 + gi * STAGE_B;  // this group's stages
   unsigned char* const st1 = smem1 + gi * STAGE_B;
   const int col = lane & 31, half = lane >> 5;
+  const int rdim = a.rdim;
   const int BH = a.B * a.Hkv;
   const int bh = blockIdx.x % BH;
   const int split = (blockIdx.x / BH) % ba.nsplit;
@@ -522,13 +525,13 @@ __global__ __launch_bounds__(NG * kThreads, (D <= 128 ? 2 : 1)) void flash_bwd_d
   typename E::v8 kf[D / 16], vf[D / 16];
   {
     const bool kin = key < a.Lk;
-    const size_t koff = ((size_t)(b * a.Lk + (kin ? key : 0)) * a.Hkv + hkv) * D;
+    const size_t koff = ((size_t)(b * a.Lk + (kin ? key : 0)) * a.Hkv + hkv) * rdim;
     const uint16_t* krow = (const uint16_t*)a.k + koff;
     const uint16_t* vrow = (const uint16_t*)a.v + koff;
 #pragma unroll
     for (int s = 0; s < D / 16; ++s) {
       u32x4 rk = {0u, 0u, 0u, 0u}, rv = rk;
-      if (kin) {
+      if (kin && 16 * s + 8 * half < rdim) {
         rk = *(const u32x4*)(krow + 16 * s + 8 * half);
         rv = *(const u32x4*)(vrow + 16 * s + 8 * half);
       }
@@ -538,13 +541,13 @@ __global__ __launch_bounds__(NG * kThreads, (D <= 128 ? 2 : 1)) void flash_bwd_d
   }
   const bool natural = BIAS || EXT == 3 || (EXT == 2 && a.m.alibi != nullptr);
   const float cx = natural ? kLog2e : a.scale * kLog2e;
-  const uint32_t rowstride = (uint32_t)a.Hq * D * 2;
+  const uint32_t rowstride = (uint32_t)a.Hq * rdim * 2;
 
   uint32_t voff[T::NLD];
 #pragma unroll
   for (int j = 0; j < T::NLD; ++j) {
     const int r = 16 * w + T::RPI * j + lane / T::NC, slot = lane % T::NC;
-    voff[j] = r * rowstride + 16 * (slot ^ T::swz(r));
+    voff[j] = row_chunk(r, rowstride, slot ^ T::swz(r), rdim);
   }
   BwdOffsets<D> off;
   off.init(lane, gi * STAGE_B);  // fragment reads address the group's stage from smem0 / smem1
@@ -566,8 +569,8 @@ __global__ __launch_bounds__(NG * kThreads, (D <= 128 ? 2 : 1)) void flash_bwd_d
   auto issue = [&](int t, unsigned char* st) {
     const int h = tile_head(t), q0 = tile_q0(t);
     const int nvalid = max(min(kBQs, a.Lq - q0), 1);
-    const uint32_t bytes = (uint32_t)(nvalid - 1) * rowstride + ROWB;
-    const size_t roff = ((size_t)(b * a.Lq + q0) * a.Hq + h) * ROWB;
+    const uint32_t bytes = (uint32_t)(nvalid - 1) * rowstride + rdim * 2;
+    const size_t roff = ((size_t)(b * a.Lq + q0) * a.Hq + h) * rdim * 2;
     const rsrc_t rq = make_rsrc((const unsigned char*)a.q + roff, bytes);
     const rsrc_t rd = make_rsrc((const unsigned char*)ba.dout + roff, bytes);
 #pragma unroll
@@ -775,14 +778,15 @@ __global__ __launch_bounds__(NG * kThreads, (D <= 128 ? 2 : 1)) void flash_bwd_d
 
   if (ba.nsplit > 1) {
     if (key < a.Lk) {
-      const size_t n = (size_t)a.B * a.Lk * a.Hkv * D;
-      float* pk = ba.part + split * n + ((size_t)(b * a.Lk + key) * a.Hkv + hkv) * D;
+      const size_t n = (size_t)a.B * a.Lk * a.Hkv * rdim;
+      float* pk = ba.part + split * n + ((size_t)(b * a.Lk + key) * a.Hkv + hkv) * rdim;
       float* pv = pk + ba.nsplit * n;
 #pragma unroll
       for (int db = 0; db < D / 32; ++db)
 #pragma unroll
         for (int gq = 0; gq < 4; ++gq) {
           const int d = db * 32 + 8 * gq + 4 * half;
+          if (db * 32 + 8 * gq >= rdim) continue;
           *(f32x4*)(pk + d) = f32x4{acck[db][4 * gq], acck[db][4 * gq + 1], acck[db][4 * gq + 2], acck[db][4 * gq + 3]};
           *(f32x4*)(pv + d) = f32x4{accv[db][4 * gq], accv[db][4 * gq + 1], accv[db][4 * gq + 2], accv[db][4 * gq + 3]};
         }
@@ -791,13 +795,14 @@ __global__ __launch_bounds__(NG * kThreads, (D <= 128 ? 2 : 1)) void flash_bwd_d
   }
   // dK, dV rows of this lane's key (zeros for keys past the valid length).
   if (key < a.Lk) {
-    const size_t koff = ((size_t)(b * a.Lk + key) * a.Hkv + hkv) * D;
+    const size_t koff = ((size_t)(b * a.Lk + key) * a.Hkv + hkv) * rdim;
     uint16_t* dkrow = (uint16_t*)ba.dk + koff;
     uint16_t* dvrow = (uint16_t*)ba.dv + koff;
 #pragma unroll
     for (int db = 0; db < D / 32; ++db)
 #pragma unroll
       for (int gq = 0; gq < 4; ++gq) {
+        if (db * 32 + 8 * gq >= rdim) continue;
         u32x2 pk, pv;
         pk[0] = E::pack2(acck[db][4 * gq], acck[db][4 * gq + 1]);
         pk[1] = E::pack2(acck[db][4 * gq + 2], acck[db][4 * gq + 3]);

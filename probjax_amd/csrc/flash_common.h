@@ -24,6 +24,7 @@ struct FlashArgs {
   float scale;
   int n_qtiles;
   int dv;       // output row width (elements per head); the wide kernels' V width
+  int rdim;     // elements per q / k / v / o row in memory: a multiple of 8, at most the kernel's head dim
   int ext;      // 0: none; 1: interval masks in `m`; 2: also segment ids / distance slopes; 3: all of `m`
   int f16;      // 16-bit inputs are fp16 (else bf16); read by the host-side launchers only
   ScoreMods m;
@@ -36,6 +37,19 @@ constexpr int kThreads = 256;
 int launch_flash_f32(const FlashArgs& a, int head_dim, hipStream_t s);
 // fp32 forward at head dim 256 (flash_f32_wide.hip).  Returns a PJX_* status.
 int launch_flash_f32_wide(const FlashArgs& a, hipStream_t s);
+
+// Byte offset of 16-byte chunk c of row r for a buffer load; past the row's
+// rdim elements an offset beyond the buffer, which reads zeros.  So a kernel of
+// head dim D takes narrower rows as they lie in memory: the missing features
+// are zeros in LDS, and no padded copy of Q, K, V, dO and slice of every result
+// is made (window layer, fp16 B=2 H=12 L=1531 D=96, forward + backward: 11 copy
+// launches of 59 us beside 76 us of attention kernels; the call 255 -> 173 us).
+// (A row_dim call's buffers stay below kPastBuffer bytes; the entry points
+// check it.)
+constexpr uint32_t kPastBuffer = 0x80000000u;
+__device__ __forceinline__ uint32_t row_chunk(uint32_t r, uint32_t rowstride, int c, int rdim) {
+  return 8 * c < rdim ? r * rowstride + 16 * c : kPastBuffer;
+}
 
 // Per-block geometry shared by both dtype paths.
 struct BlockGeom {
@@ -259,6 +273,9 @@ struct Bf16Tile {
 // Host: checks the C-ABI modifier block and fills a.m / a.ext; returns a
 // PJX_* status (message set on error).
 int lower_score_mods(const pjx_score_mods* mods, FlashArgs& a, const char* who);
+
+// Host: a *_rows entry point's head_dim / row_dim; returns a PJX_* status.
+int check_row_dim(int64_t head_dim, int64_t row_dim, int64_t q_heads, int64_t kv_heads, const char* who);
 
 // Launches the bf16 dense-bias kernel (flash_bias_ring.hip); returns a PJX_*
 // status.

@@ -62,20 +62,21 @@ __global__ __launch_bounds__(128 * QS, 2) void flash_dbias_kernel(DbiasArgs da) 
   // every wave loads 64 / NW rows of each tile
   constexpr int LR = 64 / NW, NLD = LR / T::RPI;
   static_assert(LR % T::RPI == 0, "whole loads per wave");
-  const uint32_t qstride = (uint32_t)a.Hq * ROWB, kstride = (uint32_t)a.Hkv * ROWB;
+  const int rdim = a.rdim;
+  const uint32_t qstride = (uint32_t)a.Hq * rdim * 2, kstride = (uint32_t)a.Hkv * rdim * 2;
   uint32_t voffq[NLD], voffk[NLD];
 #pragma unroll
   for (int j = 0; j < NLD; ++j) {
-    const int r = LR * w + T::RPI * j + lane / T::NC, c = 16 * ((lane % T::NC) ^ T::swz(r));
-    voffq[j] = r * qstride + c;
-    voffk[j] = r * kstride + c;
+    const int r = LR * w + T::RPI * j + lane / T::NC, c = (lane % T::NC) ^ T::swz(r);
+    voffq[j] = row_chunk(r, qstride, c, rdim);
+    voffk[j] = row_chunk(r, kstride, c, rdim);
   }
   // 64 rows from row0 of head `head` of a [B, L, heads, D] tensor (zeros past L)
   auto load = [&](const void* t, int b, int L, int heads, int head, int row0, uint32_t stride, const uint32_t* voff,
                   unsigned char* dst) {
     const int n = min(64, L - row0);
-    const rsrc_t rs = make_rsrc((const unsigned char*)t + ((size_t)(b * L + (n > 0 ? row0 : 0)) * heads + head) * ROWB,
-                                n > 0 ? (uint32_t)(n - 1) * stride + ROWB : 0u);
+    const rsrc_t rs = make_rsrc((const unsigned char*)t + ((size_t)(b * L + (n > 0 ? row0 : 0)) * heads + head) * rdim * 2,
+                                n > 0 ? (uint32_t)(n - 1) * stride + rdim * 2 : 0u);
 #pragma unroll
     for (int j = 0; j < NLD; ++j) buffer_load_lds16(rs, dst + (LR * w + T::RPI * j) * ROWB, voff[j]);
   };
@@ -203,14 +204,15 @@ using namespace pjx;
 extern "C" int pjx_flash_dbias(int dtype, const void* q, const void* k, const void* v, const void* dout,
                                const void* workspace, float* dbias, const int32_t* kv_lengths, const float* bias,
                                int64_t bias_batch, int64_t bias_heads, int64_t batch, int64_t q_len, int64_t kv_len,
-                               int64_t q_heads, int64_t kv_heads, int64_t head_dim, int64_t q_valid, int64_t kv_valid,
-                               int causal, float sm_scale, const pjx_score_mods* mods, void* stream) {
+                               int64_t q_heads, int64_t kv_heads, int64_t head_dim, int64_t row_dim, int64_t q_valid,
+                               int64_t kv_valid, int causal, float sm_scale, const pjx_score_mods* mods, void* stream) {
   clear_error();
   if (dtype != PJX_DTYPE_BF16 && dtype != PJX_DTYPE_F16)
     return fail(PJX_ERR_INVALID, "pjx_flash_dbias: dtype must be PJX_DTYPE_BF16 or PJX_DTYPE_F16");
-  if (head_dim != 64 && head_dim != 128) return fail(PJX_ERR_INVALID, "pjx_flash_dbias: head_dim must be 64 or 128");
   if (batch <= 0 || q_len <= 0 || kv_len <= 0 || q_heads <= 0 || kv_heads <= 0 || q_heads % kv_heads)
     return fail(PJX_ERR_INVALID, "pjx_flash_dbias: sizes must be positive and q_heads a multiple of kv_heads");
+  const int rrc = check_row_dim(head_dim, row_dim, q_heads, kv_heads, "pjx_flash_dbias");
+  if (rrc != PJX_OK) return rrc;
   if (!q || !k || !v || !dout || !workspace || !dbias || !bias)
     return fail(PJX_ERR_INVALID, "pjx_flash_dbias: pointers must be non-null");
   if (!((bias_batch == 1 || bias_batch == batch) && (bias_heads == 1 || bias_heads == q_heads)))
@@ -235,6 +237,7 @@ extern "C" int pjx_flash_dbias(int dtype, const void* q, const void* k, const vo
   a.scale = sm_scale;
   a.n_qtiles = 0;
   a.dv = (int)head_dim;
+  a.rdim = (int)row_dim;
   const int rc = lower_score_mods(mods, a, "pjx_flash_dbias");
   if (rc != PJX_OK) return rc;
   ba.dout = dout;

@@ -39,14 +39,15 @@ __global__ __launch_bounds__(64 * RS * KG, WPE) void flash_fwd_f32_planes_kernel
   const int col = lane & 31, half = lane >> 5;
   BlockGeom g = plane_geom(a, blockIdx.x, BQ, strip);
   if constexpr (EXT > 0) ext_block_range(a, g, 32, BQ);
-  const uint32_t kv_row = (uint32_t)a.Hkv * D * 4;
-  const unsigned char* Kb = (const unsigned char*)a.k + ((size_t)g.b * a.Lk * a.Hkv + g.hkv) * D * 4;
-  const unsigned char* Vb = (const unsigned char*)a.v + ((size_t)g.b * a.Lk * a.Hkv + g.hkv) * D * 4;
+  const int rdim = a.rdim;
+  const uint32_t kv_row = (uint32_t)a.Hkv * rdim * 4;
+  const unsigned char* Kb = (const unsigned char*)a.k + ((size_t)g.b * a.Lk * a.Hkv + g.hkv) * rdim * 4;
+  const unsigned char* Vb = (const unsigned char*)a.v + ((size_t)g.b * a.Lk * a.Hkv + g.hkv) * rdim * 4;
   const bool row_in = g.qi < a.Lq;
   const bool row_ok = g.qi < g.q_hi;
 
   // Q^T as the B operand: lane holds query `col`, dims 16*s + 8*half + [0,8).
-  const float* qrow = (const float*)a.q + ((size_t)(g.b * a.Lq + (row_in ? g.qi : 0)) * a.Hq + g.h) * D;
+  const float* qrow = (const float*)a.q + ((size_t)(g.b * a.Lq + (row_in ? g.qi : 0)) * a.Hq + g.h) * rdim;
   Planes qf[D / 16];
   bool q_wild;  // a value beyond the planes' range in the wave's rows
   {
@@ -54,7 +55,7 @@ __global__ __launch_bounds__(64 * RS * KG, WPE) void flash_fwd_f32_planes_kernel
 #pragma unroll
     for (int s = 0; s < D / 16; ++s) {
       float x[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-      if (row_in) {
+      if (row_in && 16 * s + 8 * half < rdim) {
         *(f32x4*)x = *(const f32x4*)(qrow + 16 * s + 8 * half);
         *(f32x4*)(x + 4) = *(const f32x4*)(qrow + 16 * s + 8 * half + 4);
       }
@@ -75,7 +76,7 @@ __global__ __launch_bounds__(64 * RS * KG, WPE) void flash_fwd_f32_planes_kernel
 
   PlaneOffsets<D> off;
   off.init(lane);
-  const uint32_t goff = wave_rows_offset<D>(kv_row);
+  const uint32_t goff = wave_rows_offset<D>(kv_row, rdim);
   uint32_t loff[PER];
 #pragma unroll
   for (int i = 0; i < PER; ++i) {
@@ -99,7 +100,7 @@ __global__ __launch_bounds__(64 * RS * KG, WPE) void flash_fwd_f32_planes_kernel
 #pragma unroll
     for (int i = 0; i < PER; ++i) {
       const int row = k0 + (64 * w8 + NT * i) % NCH / T::NC;
-      const rsrc_t r = wave_rows<D>(is_v(i) ? Vb : Kb, row, g.kv_stop, kv_row);
+      const rsrc_t r = wave_rows<D>(is_v(i) ? Vb : Kb, row, g.kv_stop, kv_row, rdim);
       *(f32x4*)reg[i] = buffer_load_f32x4(r, goff);
       *(f32x4*)(reg[i] + 4) = buffer_load_f32x4(r, goff + 16);
     }
@@ -148,7 +149,10 @@ __global__ __launch_bounds__(64 * RS * KG, WPE) void flash_fwd_f32_planes_kernel
       const float* kp = (const float*)(Kb + (size_t)(kin ? k0 + col : 0) * kv_row) + half * (D / 2);
       const float* qp = qrow + half * (D / 2);
 #pragma unroll 1
-      for (int i = 0; i < D / 2; ++i) s[0] = mfma32x32x2f32(kin ? kp[i] : 0.f, row_in ? qp[i] : 0.f, s[0]);
+      for (int i = 0; i < D / 2; ++i) {
+        const bool in = half * (D / 2) + i < rdim;
+        s[0] = mfma32x32x2f32(in && kin ? kp[i] : 0.f, in && row_in ? qp[i] : 0.f, s[0]);
+      }
     }
     if constexpr (EXT == 3) {
       ext_scores_sT<1, BIAS>(a, g, er, s, k0, half, brow, row_in, [&](int kb, int r, float x, float) { s[kb][r] = x; });
@@ -218,7 +222,7 @@ __global__ __launch_bounds__(64 * RS * KG, WPE) void flash_fwd_f32_planes_kernel
         const float* vp = (const float*)(Vb + (size_t)(vin ? key : 0) * kv_row) + col;
 #pragma unroll
         for (int db = 0; db < D / 32; ++db)
-          acc[db] = mfma32x32x2f32(vin ? vp[db * 32] : 0.f, s[0][r], acc[db]);
+          acc[db] = mfma32x32x2f32(vin && db * 32 + col < rdim ? vp[db * 32] : 0.f, s[0][r], acc[db]);
         __builtin_amdgcn_sched_barrier(0);
       }
     }
@@ -286,12 +290,13 @@ __global__ __launch_bounds__(64 * RS * KG, WPE) void flash_fwd_f32_planes_kernel
   const float l_tot = xor32_sum(l_run);
   const float inv = l_tot > 0.f ? 1.f / l_tot : 0.f;
   if (row_in) {
-    float* orow = (float*)a.o + ((size_t)(g.b * a.Lq + g.qi) * a.Hq + g.h) * D;
+    float* orow = (float*)a.o + ((size_t)(g.b * a.Lq + g.qi) * a.Hq + g.h) * rdim;
 #pragma unroll
     for (int db = 0; db < D / 32; ++db)
 #pragma unroll
       for (int gq = 0; gq < 4; ++gq)
-        *(f32x4*)(orow + db * 32 + 8 * gq + 4 * half) =
+        if (db * 32 + 8 * gq < rdim)
+          *(f32x4*)(orow + db * 32 + 8 * gq + 4 * half) =
             f32x4{acc[db][4 * gq] * inv, acc[db][4 * gq + 1] * inv, acc[db][4 * gq + 2] * inv, acc[db][4 * gq + 3] * inv};
     if (a.lse && half == 0)
       a.lse[((size_t)g.b * a.Hq + g.h) * a.Lq + g.qi] =

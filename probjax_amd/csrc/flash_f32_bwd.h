@@ -45,13 +45,14 @@ __global__ __launch_bounds__(64 * RS * KG, WPE) void flash_bwd_dq_f32_planes_ker
   const int col = lane & 31, half = lane >> 5;
   BlockGeom g = plane_geom(a, blockIdx.x, BQ, strip);
   if constexpr (EXT > 0) ext_block_range(a, g, 32, BQ);
-  const uint32_t kv_row = (uint32_t)a.Hkv * D * 4;
-  const unsigned char* Kb = (const unsigned char*)a.k + ((size_t)g.b * a.Lk * a.Hkv + g.hkv) * D * 4;
-  const unsigned char* Vb = (const unsigned char*)a.v + ((size_t)g.b * a.Lk * a.Hkv + g.hkv) * D * 4;
+  const int rdim = a.rdim;
+  const uint32_t kv_row = (uint32_t)a.Hkv * rdim * 4;
+  const unsigned char* Kb = (const unsigned char*)a.k + ((size_t)g.b * a.Lk * a.Hkv + g.hkv) * rdim * 4;
+  const unsigned char* Vb = (const unsigned char*)a.v + ((size_t)g.b * a.Lk * a.Hkv + g.hkv) * rdim * 4;
   const bool row_in = g.qi < a.Lq;
   const bool row_ok = g.qi < g.q_hi;
 
-  const size_t roff = ((size_t)(g.b * a.Lq + (row_in ? g.qi : 0)) * a.Hq + g.h) * D;
+  const size_t roff = ((size_t)(g.b * a.Lq + (row_in ? g.qi : 0)) * a.Hq + g.h) * rdim;
   const float* qrow = (const float*)a.q + roff;
   const float* drow = (const float*)ba.dout + roff;
   Planes qf[D / 16], df[D / 16];
@@ -63,7 +64,7 @@ __global__ __launch_bounds__(64 * RS * KG, WPE) void flash_bwd_dq_f32_planes_ker
 #pragma unroll
     for (int s = 0; s < D / 16; ++s) {
       float x[8] = {}, y[8] = {}, z[8] = {};
-      if (row_in) {
+      if (row_in && 16 * s + 8 * half < rdim) {
 #pragma unroll
         for (int j = 0; j < 8; j += 4) {
           *(f32x4*)(x + j) = *(const f32x4*)(qrow + 16 * s + 8 * half + j);
@@ -102,7 +103,7 @@ __global__ __launch_bounds__(64 * RS * KG, WPE) void flash_bwd_dq_f32_planes_ker
 
   PlaneOffsets<D> off;
   off.init(lane);
-  const uint32_t goff = wave_rows_offset<D>(kv_row);
+  const uint32_t goff = wave_rows_offset<D>(kv_row, rdim);
   uint32_t loff[PER];
 #pragma unroll
   for (int i = 0; i < PER; ++i) {
@@ -123,7 +124,7 @@ __global__ __launch_bounds__(64 * RS * KG, WPE) void flash_bwd_dq_f32_planes_ker
 #pragma unroll
     for (int i = 0; i < PER; ++i) {
       const int row = k0 + (64 * w8 + NT * i) % NCH / T::NC;
-      const rsrc_t r = wave_rows<D>(is_v(i) ? Vb : Kb, row, g.kv_stop, kv_row);
+      const rsrc_t r = wave_rows<D>(is_v(i) ? Vb : Kb, row, g.kv_stop, kv_row, rdim);
       *(f32x4*)reg[i] = buffer_load_f32x4(r, goff);
       *(f32x4*)(reg[i] + 4) = buffer_load_f32x4(r, goff + 16);
     }
@@ -177,8 +178,9 @@ __global__ __launch_bounds__(64 * RS * KG, WPE) void flash_bwd_dq_f32_planes_ker
       const float* dop = drow + half * (D / 2);
 #pragma unroll 1
       for (int i = 0; i < D / 2; ++i) {
-        s[0] = mfma32x32x2f32(kin ? kp[i] : 0.f, row_in ? qp[i] : 0.f, s[0]);
-        dp[0] = mfma32x32x2f32(kin ? vp[i] : 0.f, row_in ? dop[i] : 0.f, dp[0]);
+        const bool in = half * (D / 2) + i < rdim;
+        s[0] = mfma32x32x2f32(in && kin ? kp[i] : 0.f, in && row_in ? qp[i] : 0.f, s[0]);
+        dp[0] = mfma32x32x2f32(in && kin ? vp[i] : 0.f, in && row_in ? dop[i] : 0.f, dp[0]);
       }
     }
     f32x16 dbv[1];
@@ -246,7 +248,7 @@ __global__ __launch_bounds__(64 * RS * KG, WPE) void flash_bwd_dq_f32_planes_ker
         const float* kp = (const float*)(Kb + (size_t)(kin ? key : 0) * kv_row) + col;
 #pragma unroll
         for (int db = 0; db < D / 32; ++db)
-          acc[db] = mfma32x32x2f32(kin ? kp[db * 32] : 0.f, s[0][r], acc[db]);
+          acc[db] = mfma32x32x2f32(kin && db * 32 + col < rdim ? kp[db * 32] : 0.f, s[0][r], acc[db]);
         __builtin_amdgcn_sched_barrier(0);
       }
     }
@@ -299,7 +301,8 @@ __global__ __launch_bounds__(64 * RS * KG, WPE) void flash_bwd_dq_f32_planes_ker
     for (int db = 0; db < D / 32; ++db)
 #pragma unroll
       for (int gq = 0; gq < 4; ++gq)
-        *(f32x4*)(out + db * 32 + 8 * gq + 4 * half) =
+        if (db * 32 + 8 * gq < rdim)
+          *(f32x4*)(out + db * 32 + 8 * gq + 4 * half) =
             f32x4{acc[db][4 * gq], acc[db][4 * gq + 1], acc[db][4 * gq + 2], acc[db][4 * gq + 3]};
   }
 }
@@ -331,6 +334,7 @@ __global__ __launch_bounds__(64 * KS * QG, WPE) void flash_bwd_dkdv_f32_planes_k
   const int w8 = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int strip = w8 % KS, gi = w8 / KS;
   const int col = lane & 31, half = lane >> 5;
+  const int rdim = a.rdim;
   const int BH = a.B * a.Hkv;
   const int bh = blockIdx.x % BH;
   const int k0 = (blockIdx.x / BH) * BK;
@@ -376,7 +380,7 @@ __global__ __launch_bounds__(64 * KS * QG, WPE) void flash_bwd_dkdv_f32_planes_k
   // K^T and V^T as B operands: lane holds key `key`, dims 16*s + 8*half + [0,8).
   // Group 0 of each strip splits its rows into LDS.
   const bool kin = key < a.Lk;
-  const size_t koff = ((size_t)(b * a.Lk + (kin ? key : 0)) * a.Hkv + hkv) * D;
+  const size_t koff = ((size_t)(b * a.Lk + (kin ? key : 0)) * a.Hkv + hkv) * rdim;
   const float* krow = (const float*)a.k + koff;
   const float* vrow = (const float*)a.v + koff;
   PlaneOffsets<D> off;
@@ -388,7 +392,7 @@ __global__ __launch_bounds__(64 * KS * QG, WPE) void flash_bwd_dkdv_f32_planes_k
 #pragma unroll
     for (int s = 0; s < D / 16; ++s) {
       float x[8] = {}, y[8] = {};
-      if (kin) {
+      if (kin && 16 * s + 8 * half < rdim) {
 #pragma unroll
         for (int j = 0; j < 8; j += 4) {
           *(f32x4*)(x + j) = *(const f32x4*)(krow + 16 * s + 8 * half + j);
@@ -408,9 +412,9 @@ __global__ __launch_bounds__(64 * KS * QG, WPE) void flash_bwd_dkdv_f32_planes_k
   auto vfrag = [&](int st) { return VR ? vf[VR ? st : 0] : TK::rows(kv + (VR ? 0 : TK::BYTES), 32 * strip, off.row[st]); };
   const bool natural = BIAS || EXT == 3 || (EXT == 2 && a.m.alibi != nullptr);
   const float cx = natural ? kLog2e : a.scale * kLog2e;
-  const uint32_t q_row = (uint32_t)a.Hq * D * 4;
+  const uint32_t q_row = (uint32_t)a.Hq * rdim * 4;
 
-  const uint32_t goff = wave_rows_offset<D>(q_row);
+  const uint32_t goff = wave_rows_offset<D>(q_row, rdim);
   uint32_t loff[PER];
 #pragma unroll
   for (int i = 0; i < PER; ++i) {
@@ -432,11 +436,11 @@ __global__ __launch_bounds__(64 * KS * QG, WPE) void flash_bwd_dkdv_f32_planes_k
   float reg[PER][8], rreg = 0.f;
   auto load = [&](int t) {
     const int h = stage_head(t), q0 = stage_q0(t);
-    const size_t ro = ((size_t)b * a.Lq * a.Hq + h) * D * 4;
+    const size_t ro = ((size_t)b * a.Lq * a.Hq + h) * rdim * 4;
 #pragma unroll
     for (int i = 0; i < PER; ++i) {
       const int row = q0 + (64 * w8 + NT * i) % NCH / T::NC;
-      const rsrc_t r = wave_rows<D>((const unsigned char*)(is_d(i) ? ba.dout : a.q) + ro, row, a.Lq, q_row);
+      const rsrc_t r = wave_rows<D>((const unsigned char*)(is_d(i) ? ba.dout : a.q) + ro, row, a.Lq, q_row, rdim);
       *(f32x4*)reg[i] = buffer_load_f32x4(r, goff);
       *(f32x4*)(reg[i] + 4) = buffer_load_f32x4(r, goff + 16);
     }
@@ -481,8 +485,8 @@ __global__ __launch_bounds__(64 * KS * QG, WPE) void flash_bwd_dkdv_f32_planes_k
     const float* lsm = rows + 32 * gi;
     const float* dlm = lsm + SQ;
     const bool wild = k_wild || __builtin_amdgcn_readfirstlane(flags[t & 1]) == t + 1;
-    const float* Qg = (const float*)a.q + ((size_t)b * a.Lq * a.Hq + h) * D;
-    const float* Dg = (const float*)ba.dout + ((size_t)b * a.Lq * a.Hq + h) * D;
+    const float* Qg = (const float*)a.q + ((size_t)b * a.Lq * a.Hq + h) * rdim;
+    const float* Dg = (const float*)ba.dout + ((size_t)b * a.Lq * a.Hq + h) * rdim;
 
     // register r holds query q0 + 8*(r/4) + 4*half + r%4 of key `key`
     f32x16 s = f32x16{}, dp = f32x16{};
@@ -495,11 +499,12 @@ __global__ __launch_bounds__(64 * KS * QG, WPE) void flash_bwd_dkdv_f32_planes_k
       }
     } else {
       const bool qin = q0 + col < a.Lq;
-      const size_t qo = (size_t)(qin ? q0 + col : 0) * a.Hq * D + half * (D / 2);
+      const size_t qo = (size_t)(qin ? q0 + col : 0) * a.Hq * rdim + half * (D / 2);
 #pragma unroll 1
       for (int i = 0; i < D / 2; ++i) {
-        s = mfma32x32x2f32(qin ? Qg[qo + i] : 0.f, kin ? krow[half * (D / 2) + i] : 0.f, s);
-        dp = mfma32x32x2f32(qin ? Dg[qo + i] : 0.f, kin ? vrow[half * (D / 2) + i] : 0.f, dp);
+        const bool in = half * (D / 2) + i < rdim;
+        s = mfma32x32x2f32(in && qin ? Qg[qo + i] : 0.f, in && kin ? krow[half * (D / 2) + i] : 0.f, s);
+        dp = mfma32x32x2f32(in && qin ? Dg[qo + i] : 0.f, in && kin ? vrow[half * (D / 2) + i] : 0.f, dp);
       }
     }
     if constexpr (EXT == 3) {
@@ -572,11 +577,12 @@ __global__ __launch_bounds__(64 * KS * QG, WPE) void flash_bwd_dkdv_f32_planes_k
       for (int r = 0; r < 16; ++r) {
         const int qq = q0 + 8 * (r >> 2) + 4 * half + (r & 3);
         const bool qin = qq < a.Lq;
-        const size_t qo = (size_t)(qin ? qq : 0) * a.Hq * D + col;
+        const size_t qo = (size_t)(qin ? qq : 0) * a.Hq * rdim + col;
 #pragma unroll
         for (int db = 0; db < D / 32; ++db) {
-          accv[db] = mfma32x32x2f32(qin ? Dg[qo + db * 32] : 0.f, s[r], accv[db]);
-          acck[db] = mfma32x32x2f32(qin ? Qg[qo + db * 32] : 0.f, dp[r], acck[db]);
+          const bool in = qin && db * 32 + col < rdim;
+          accv[db] = mfma32x32x2f32(in ? Dg[qo + db * 32] : 0.f, s[r], accv[db]);
+          acck[db] = mfma32x32x2f32(in ? Qg[qo + db * 32] : 0.f, dp[r], acck[db]);
         }
         __builtin_amdgcn_sched_barrier(0);
       }
@@ -633,7 +639,8 @@ __global__ __launch_bounds__(64 * KS * QG, WPE) void flash_bwd_dkdv_f32_planes_k
       for (int db = 0; db < D / 32; ++db)
 #pragma unroll
         for (int gq = 0; gq < 4; ++gq)
-          *(f32x4*)(out + koff + db * 32 + 8 * gq + 4 * half) =
+          if (db * 32 + 8 * gq < rdim)
+            *(f32x4*)(out + koff + db * 32 + 8 * gq + 4 * half) =
               f32x4{acc[db][4 * gq], acc[db][4 * gq + 1], acc[db][4 * gq + 2], acc[db][4 * gq + 3]};
     }
   };

@@ -80,9 +80,10 @@ __global__ __launch_bounds__(kThreads, 2) void flash_fwd_bf16_kernel(FlashArgs a
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
   g.qw = __builtin_amdgcn_readfirstlane(g.qw);
   const int col = lane & 31, half = lane >> 5;
-  const uint32_t rowstride = (uint32_t)a.Hkv * D * 2;
-  const unsigned char* Kb = (const unsigned char*)a.k + ((size_t)g.b * a.Lk * a.Hkv + g.hkv) * ROWB;
-  const unsigned char* Vb = (const unsigned char*)a.v + ((size_t)g.b * a.Lk * a.Hkv + g.hkv) * ROWB;
+  const int rdim = a.rdim;
+  const uint32_t rowstride = (uint32_t)a.Hkv * rdim * 2;
+  const unsigned char* Kb = (const unsigned char*)a.k + ((size_t)g.b * a.Lk * a.Hkv + g.hkv) * rdim * 2;
+  const unsigned char* Vb = (const unsigned char*)a.v + ((size_t)g.b * a.Lk * a.Hkv + g.hkv) * rdim * 2;
   const bool row_in = g.qi < a.Lq;
   const bool row_ok = g.qi < g.q_hi;
 
@@ -90,11 +91,11 @@ __global__ __launch_bounds__(kThreads, 2) void flash_fwd_bf16_kernel(FlashArgs a
   typename E::v8 qf[D / 16];
   {
     const uint16_t* qrow =
-        (const uint16_t*)a.q + ((size_t)(g.b * a.Lq + (row_in ? g.qi : 0)) * a.Hq + g.h) * D;
+        (const uint16_t*)a.q + ((size_t)(g.b * a.Lq + (row_in ? g.qi : 0)) * a.Hq + g.h) * rdim;
 #pragma unroll
     for (int s = 0; s < D / 16; ++s) {
       u32x4 raw = {0u, 0u, 0u, 0u};
-      if (row_in) raw = *(const u32x4*)(qrow + 16 * s + 8 * half);
+      if (row_in && 16 * s + 8 * half < rdim) raw = *(const u32x4*)(qrow + 16 * s + 8 * half);
       qf[s] = E::as8(raw);
     }
   }
@@ -117,8 +118,8 @@ __global__ __launch_bounds__(kThreads, 2) void flash_fwd_bf16_kernel(FlashArgs a
 #pragma unroll
   for (int j = 0; j < T::NLD; ++j) {
     const int r = 16 * w + T::RPI * j + lane / T::NC, slot = lane % T::NC;
-    voffK[j] = r * rowstride + 16 * (slot ^ T::swz_k(r));
-    voffV[j] = r * rowstride + 16 * (slot ^ T::swz_v(r));
+    voffK[j] = row_chunk(r, rowstride, slot ^ T::swz_k(r), rdim);
+    voffV[j] = row_chunk(r, rowstride, slot ^ T::swz_v(r), rdim);
   }
   uint32_t offK[D / 16];  // K row `col` (of a 32-key block), dims 16*st + 8*half
 #pragma unroll
@@ -146,7 +147,7 @@ __global__ __launch_bounds__(kThreads, 2) void flash_fwd_bf16_kernel(FlashArgs a
   auto issue = [&](int t, unsigned char* ks) {
     const int k0 = (t_begin + t) * BK;
     const int nvalid = min(BK, g.kv_stop - k0);
-    const uint32_t bytes = (uint32_t)(nvalid - 1) * rowstride + ROWB;
+    const uint32_t bytes = (uint32_t)(nvalid - 1) * rowstride + rdim * 2;
     const rsrc_t rk = make_rsrc(Kb + (size_t)k0 * rowstride, bytes);
     const rsrc_t rv = make_rsrc(Vb + (size_t)k0 * rowstride, bytes);
 #pragma unroll
@@ -314,11 +315,12 @@ __global__ __launch_bounds__(kThreads, 2) void flash_fwd_bf16_kernel(FlashArgs a
   const float l_tot = xor32_sum(l_run);
   const float inv = l_tot > 0.f ? 1.f / l_tot : 0.f;
   if (row_in) {
-    uint16_t* orow = (uint16_t*)a.o + ((size_t)(g.b * a.Lq + g.qi) * a.Hq + g.h) * D;
+    uint16_t* orow = (uint16_t*)a.o + ((size_t)(g.b * a.Lq + g.qi) * a.Hq + g.h) * rdim;
 #pragma unroll
     for (int db = 0; db < D / 32; ++db)
 #pragma unroll
       for (int gq = 0; gq < 4; ++gq) {
+        if (db * 32 + 8 * gq >= rdim) continue;
         u32x2 pk;
         pk[0] = E::pack2(acc[db][4 * gq] * inv, acc[db][4 * gq + 1] * inv);
         pk[1] = E::pack2(acc[db][4 * gq + 2] * inv, acc[db][4 * gq + 3] * inv);
@@ -374,20 +376,21 @@ __global__ __launch_bounds__(G * kThreads, WPC) void flash_fwd_bf16_pipe_kernel(
   unsigned char* const st0 = smem0 + gi * STAGE_B;  // this group's stages
   unsigned char* const st1 = smem1 + gi * STAGE_B;
   const int col = lane & 31, half = lane >> 5;
-  const uint32_t rowstride = (uint32_t)a.Hkv * D * 2;
-  const unsigned char* Kb = (const unsigned char*)a.k + ((size_t)g.b * a.Lk * a.Hkv + g.hkv) * ROWB;
-  const unsigned char* Vb = (const unsigned char*)a.v + ((size_t)g.b * a.Lk * a.Hkv + g.hkv) * ROWB;
+  const int rdim = a.rdim;
+  const uint32_t rowstride = (uint32_t)a.Hkv * rdim * 2;
+  const unsigned char* Kb = (const unsigned char*)a.k + ((size_t)g.b * a.Lk * a.Hkv + g.hkv) * rdim * 2;
+  const unsigned char* Vb = (const unsigned char*)a.v + ((size_t)g.b * a.Lk * a.Hkv + g.hkv) * rdim * 2;
   const bool row_in = g.qi < a.Lq;
   const bool row_ok = g.qi < g.q_hi;
 
   typename E::v8 qf[D / 16];
   {
     const uint16_t* qrow =
-        (const uint16_t*)a.q + ((size_t)(g.b * a.Lq + (row_in ? g.qi : 0)) * a.Hq + g.h) * D;
+        (const uint16_t*)a.q + ((size_t)(g.b * a.Lq + (row_in ? g.qi : 0)) * a.Hq + g.h) * rdim;
 #pragma unroll
     for (int s = 0; s < D / 16; ++s) {
       u32x4 raw = {0u, 0u, 0u, 0u};
-      if (row_in) raw = *(const u32x4*)(qrow + 16 * s + 8 * half);
+      if (row_in && 16 * s + 8 * half < rdim) raw = *(const u32x4*)(qrow + 16 * s + 8 * half);
       qf[s] = E::as8(raw);
     }
   }
@@ -397,8 +400,8 @@ __global__ __launch_bounds__(G * kThreads, WPC) void flash_fwd_bf16_pipe_kernel(
 #pragma unroll
   for (int j = 0; j < T::NLD; ++j) {
     const int r = RPW * w + T::RPI * j + lane / T::NC, slot = lane % T::NC;
-    voffK[j] = r * rowstride + 16 * (slot ^ T::swz_k(r));
-    voffV[j] = r * rowstride + 16 * (slot ^ T::swz_v(r));
+    voffK[j] = row_chunk(r, rowstride, slot ^ T::swz_k(r), rdim);
+    voffV[j] = row_chunk(r, rowstride, slot ^ T::swz_v(r), rdim);
   }
   uint32_t offK[D / 16];
 #pragma unroll
@@ -433,7 +436,7 @@ __global__ __launch_bounds__(G * kThreads, WPC) void flash_fwd_bf16_pipe_kernel(
   auto issue = [&](const unsigned char* base, int t, unsigned char* dst, const uint32_t* voff) {
     const int k0 = t * BK;
     const int nvalid = min(BK, g.kv_stop - k0);
-    const uint32_t bytes = (uint32_t)(nvalid - 1) * rowstride + ROWB;
+    const uint32_t bytes = (uint32_t)(nvalid - 1) * rowstride + rdim * 2;
     const rsrc_t rs = make_rsrc(base + (size_t)k0 * rowstride, bytes);
 #pragma unroll
     for (int j = 0; j < T::NLD; ++j) buffer_load_lds16(rs, dst + (RPW * w + T::RPI * j) * ROWB, voff[j]);
@@ -606,11 +609,12 @@ __global__ __launch_bounds__(G * kThreads, WPC) void flash_fwd_bf16_pipe_kernel(
   const float l_tot = xor32_sum(l_run);
   const float inv = l_tot > 0.f ? 1.f / l_tot : 0.f;
   if (row_in) {
-    uint16_t* orow = (uint16_t*)a.o + ((size_t)(g.b * a.Lq + g.qi) * a.Hq + g.h) * D;
+    uint16_t* orow = (uint16_t*)a.o + ((size_t)(g.b * a.Lq + g.qi) * a.Hq + g.h) * rdim;
 #pragma unroll
     for (int db = 0; db < D / 32; ++db)
 #pragma unroll
       for (int gq = 0; gq < 4; ++gq) {
+        if (db * 32 + 8 * gq >= rdim) continue;
         u32x2 pk;
         pk[0] = E::pack2(acc[db][4 * gq] * inv, acc[db][4 * gq + 1] * inv);
         pk[1] = E::pack2(acc[db][4 * gq + 2] * inv, acc[db][4 * gq + 3] * inv);
@@ -895,7 +899,7 @@ static int make_flash_args(FlashArgs& a, const char* who, const void* q, const v
                            const float* bias, int64_t bias_batch, int64_t bias_heads, int64_t batch,
                            int64_t q_len, int64_t kv_len, int64_t q_heads, int64_t kv_heads,
                            int64_t head_dim, int64_t v_dim, int64_t q_valid, int64_t kv_valid,
-                           int causal, float sm_scale, const pjx_score_mods* mods, bool* empty) {
+                           int causal, float sm_scale, const pjx_score_mods* mods, bool* empty, int64_t row_dim) {
   char buf[256];
   *empty = false;
   // zero-element tensors may come as null pointers
@@ -944,6 +948,7 @@ static int make_flash_args(FlashArgs& a, const char* who, const void* q, const v
   a.scale = sm_scale;
   a.n_qtiles = (int)((q_len + kBQ - 1) / kBQ);
   a.dv = (int)v_dim;
+  a.rdim = (int)row_dim;
   if ((long)a.n_qtiles * batch * q_heads > 0x7fffffffL) {
     snprintf(buf, sizeof(buf), "%s: grid too large", who);
     return fail(PJX_ERR_INVALID, buf);
@@ -951,13 +956,12 @@ static int make_flash_args(FlashArgs& a, const char* who, const void* q, const v
   return lower_score_mods(mods, a, who);
 }
 
-extern "C" int pjx_flash_fwd(int dtype, const void* q, const void* k, const void* v, void* o,
-                             float* lse, const int32_t* kv_lengths, const float* bias,
-                             int64_t bias_batch, int64_t bias_heads, int64_t batch,
-                             int64_t q_len, int64_t kv_len, int64_t q_heads, int64_t kv_heads,
-                             int64_t head_dim, int64_t q_valid, int64_t kv_valid, int causal,
-                             float sm_scale, const pjx_score_mods* mods, void* stream) {
-  clear_error();
+static int flash_fwd(int dtype, const void* q, const void* k, const void* v, void* o,
+                     float* lse, const int32_t* kv_lengths, const float* bias,
+                     int64_t bias_batch, int64_t bias_heads, int64_t batch,
+                     int64_t q_len, int64_t kv_len, int64_t q_heads, int64_t kv_heads,
+                     int64_t head_dim, int64_t row_dim, int64_t q_valid, int64_t kv_valid, int causal,
+                     float sm_scale, const pjx_score_mods* mods, void* stream) {
   if (dtype != PJX_DTYPE_BF16 && dtype != PJX_DTYPE_F16 && dtype != PJX_DTYPE_F32)
     return fail(PJX_ERR_INVALID, "pjx_flash_fwd: dtype must be PJX_DTYPE_BF16, PJX_DTYPE_F16 or PJX_DTYPE_F32");
   if (head_dim != 64 && head_dim != 128 && head_dim != 256)
@@ -966,11 +970,11 @@ extern "C" int pjx_flash_fwd(int dtype, const void* q, const void* k, const void
   bool empty;
   int rc = make_flash_args(a, "pjx_flash_fwd", q, k, v, o, lse, kv_lengths, bias, bias_batch,
                            bias_heads, batch, q_len, kv_len, q_heads, kv_heads, head_dim, head_dim,
-                           q_valid, kv_valid, causal, sm_scale, mods, &empty);
+                           q_valid, kv_valid, causal, sm_scale, mods, &empty, row_dim);
   if (rc != PJX_OK || empty) return rc;
   hipStream_t s = (hipStream_t)stream;
   if (kv_len == 0)
-    return write_keyless(o, lse, (size_t)(batch * q_len * q_heads * head_dim), dtype == PJX_DTYPE_F32,
+    return write_keyless(o, lse, (size_t)(batch * q_len * q_heads * row_dim), dtype == PJX_DTYPE_F32,
                          (size_t)(batch * q_heads * q_len), s, "pjx_flash_fwd");
   const bool hb = bias != nullptr;
   a.f16 = dtype == PJX_DTYPE_F16;
@@ -981,10 +985,50 @@ extern "C" int pjx_flash_fwd(int dtype, const void* q, const void* k, const void
   // each block split over waves that read their operands from memory.  There
   // the planes kernel's staging is latency nothing hides (33 against 38 us at
   // B=1 H=4 L=512 causal; 163 against 85 us at B=4 H=8 L=1024).
-  if (head_dim == 128 && a.ext == 0 && (q_len + 31) / 32 * batch * q_heads <= 256)
+  if (head_dim == 128 && row_dim == 128 && a.ext == 0 && (q_len + 31) / 32 * batch * q_heads <= 256)
     return hb ? launch_split<128, flash_fwd_f32_split_kernel<128, true>>(a, s)
               : launch_split<128, flash_fwd_f32_split_kernel<128, false>>(a, s);
   return launch_flash_f32(a, (int)head_dim, s);
+}
+
+extern "C" int pjx_flash_fwd(int dtype, const void* q, const void* k, const void* v, void* o,
+                             float* lse, const int32_t* kv_lengths, const float* bias,
+                             int64_t bias_batch, int64_t bias_heads, int64_t batch,
+                             int64_t q_len, int64_t kv_len, int64_t q_heads, int64_t kv_heads,
+                             int64_t head_dim, int64_t q_valid, int64_t kv_valid, int causal,
+                             float sm_scale, const pjx_score_mods* mods, void* stream) {
+  clear_error();
+  return flash_fwd(dtype, q, k, v, o, lse, kv_lengths, bias, bias_batch, bias_heads, batch, q_len, kv_len, q_heads,
+                   kv_heads, head_dim, head_dim, q_valid, kv_valid, causal, sm_scale, mods, stream);
+}
+
+// Rows of row_dim elements on the kernels of head dim head_dim: what both
+// directions' *_rows entry points require of the sizes.
+int pjx::check_row_dim(int64_t head_dim, int64_t row_dim, int64_t q_heads, int64_t kv_heads, const char* who) {
+  char buf[256];
+  if ((head_dim != 64 && head_dim != 128) || row_dim <= 0 || row_dim > head_dim || row_dim % 8) {
+    snprintf(buf, sizeof(buf), "%s: head_dim must be 64 or 128 and row_dim a multiple of 8 up to it", who);
+    return fail(PJX_ERR_INVALID, buf);
+  }
+  // 128 rows of 4-byte elements below the offset that stands for "past the buffer"
+  if (std::max(q_heads, kv_heads) > (int64_t)(kPastBuffer / (128 * 4)) / row_dim) {
+    snprintf(buf, sizeof(buf), "%s: rows of all heads too long", who);
+    return fail(PJX_ERR_INVALID, buf);
+  }
+  return PJX_OK;
+}
+
+extern "C" int pjx_flash_fwd_rows(int dtype, const void* q, const void* k, const void* v, void* o,
+                                  float* lse, const int32_t* kv_lengths, const float* bias,
+                                  int64_t bias_batch, int64_t bias_heads, int64_t batch,
+                                  int64_t q_len, int64_t kv_len, int64_t q_heads, int64_t kv_heads,
+                                  int64_t head_dim, int64_t row_dim, int64_t q_valid, int64_t kv_valid, int causal,
+                                  float sm_scale, const pjx_score_mods* mods, void* stream) {
+  clear_error();
+  const int rc = check_row_dim(head_dim, row_dim, q_heads, kv_heads, "pjx_flash_fwd_rows");
+  if (rc != PJX_OK) return rc;
+  return flash_fwd(dtype, q, k, v, o, lse, kv_lengths, bias, bias_batch, bias_heads, batch, q_len, kv_len, q_heads,
+                   kv_heads, head_dim, row_dim, q_valid, kv_valid, causal, sm_scale, mods, stream);
 }
 
 extern "C" int pjx_mla_fwd(int dtype, const void* q, const void* cache, void* o, float* lse,
@@ -1010,7 +1054,7 @@ extern "C" int pjx_mla_fwd(int dtype, const void* q, const void* cache, void* o,
   bool empty;
   int rc = make_flash_args(a, "pjx_mla_fwd", q, cache, cache, o, lse, kv_lengths, bias, bias_batch,
                            bias_heads, batch, q_len, kv_len, heads, 1, rank, v_dim, q_valid,
-                           kv_valid, causal, sm_scale, mods, &empty);
+                           kv_valid, causal, sm_scale, mods, &empty, rank);
   if (rc != PJX_OK || empty) return rc;
   if (kv_len == 0)
     return write_keyless(o, lse, (size_t)(batch * q_len * heads * v_dim), false, (size_t)(batch * heads * q_len),

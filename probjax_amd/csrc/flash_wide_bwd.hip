@@ -1351,6 +1351,7 @@ extern "C" int pjx_mla_bwd(int dtype, const void* q, const void* cache, const vo
   a.scale = sm_scale;
   a.n_qtiles = (int)((q_len + kBQ - 1) / kBQ);
   a.dv = (int)v_dim;
+  a.rdim = (int)rank;
   const int mrc = lower_score_mods(mods, a, who);
   if (mrc != PJX_OK) return mrc;
   ba.dout = dout;

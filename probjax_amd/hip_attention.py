@@ -39,6 +39,21 @@ def _half_code(who: str, *ts) -> int:
     return _DTYPES[ts[0].dtype]
 
 
+def rows_width(head_dim: int, heads: int):
+    """The kernel head dim (64 or 128) that takes rows of ``head_dim`` elements
+    as they lie in memory (``pjx_flash_fwd_rows`` / ``pjx_flash_bwd_rows``), or
+    None: a multiple of 8, so that rows are whole 16-byte chunks, up to 128,
+    with the rows of all ``heads`` short enough for a tile's 32-bit offsets."""
+    if head_dim <= 0 or head_dim > 128 or head_dim % 8 or heads > (1 << 22) // head_dim:
+        return None
+    return 64 if head_dim <= 64 else 128
+
+
+def _aligned(t):
+    """``t`` (contiguous), copied if it does not start on 16 bytes."""
+    return t if t.data_ptr() % 16 == 0 else t.clone()
+
+
 def _on_device(*ts):
     dev = None
     for t in ts:
@@ -125,14 +140,15 @@ def _mods_struct(m: ScoreModsArgs | None, B, Lq, Lk, Hq, dev):
 def flash_attention_fwd(
     q, k, v, *, sm_scale: float, causal: bool = False, kv_lengths=None, bias=None,
     q_valid: int | None = None, kv_valid: int | None = None, return_lse: bool = False,
-    mods: ScoreModsArgs | None = None,
+    mods: ScoreModsArgs | None = None, width: int | None = None,
 ):
     """``pjx_flash_fwd``: ``q [B, Lq, Hq, D]``, ``k/v [B, Lk, Hkv, D]`` -> ``o``.
 
     ``bias`` is fp32 ``[1|B, 1|Hq, Lq, Lk]``; ``kv_lengths`` int ``[B]``;
     ``q_valid``/``kv_valid`` are static query/key lengths (QKVLengthMask).
     Returns ``o`` (and the natural-log LSE ``[B, Hq, Lq]`` with ``return_lse``).
-    ``mods``: extended masks / score modifiers.
+    ``mods``: extended masks / score modifiers.  ``width``: the kernel head dim
+    for a narrower D (``pjx_flash_fwd_rows``; see ``rows_width``).
     """
     dev = _on_device(q, k, v, bias)
     if q.ndim != 4 or k.ndim != 4 or v.ndim != 4:
@@ -145,12 +161,14 @@ def flash_attention_fwd(
         raise ValueError("q, k, v must share a dtype")
     if Hq % Hkv:
         raise ValueError(f"query heads {Hq} must be a multiple of kv heads {Hkv}")
-    if D not in (64, 128, 256):
+    if width is None and D not in (64, 128, 256):
         raise ValueError(f"head_dim {D} not supported (64, 128 or 256)")
     if not sm_scale > 0:
         raise ValueError("sm_scale must be > 0")
     code = _dtype_code(q)
     q, k, v = q.contiguous(), k.contiguous(), v.contiguous()
+    if width is not None:
+        q, k, v = _aligned(q), _aligned(k), _aligned(v)
     bb = bh = 1
     if bias is not None:
         if bias.ndim != 4 or tuple(bias.shape[-2:]) != (Lq, Lk):
@@ -164,9 +182,9 @@ def flash_attention_fwd(
     o = torch.empty_like(q)
     lse = torch.empty((B, Hq, Lq), dtype=torch.float32, device=dev) if return_lse else None
     lib = native.load()
-    rc = lib.pjx_flash_fwd(
+    rc = (lib.pjx_flash_fwd if width is None else lib.pjx_flash_fwd_rows)(
         code, _ptr(q), _ptr(k), _ptr(v), _ptr(o), _ptr(lse), _ptr(L), _ptr(bias), bb, bh,
-        B, Lq, Lk, Hq, Hkv, D, Lq if q_valid is None else int(q_valid),
+        B, Lq, Lk, Hq, Hkv, *((D,) if width is None else (width, D)), Lq if q_valid is None else int(q_valid),
         Lk if kv_valid is None else int(kv_valid), int(bool(causal)), float(sm_scale),
         None if ms is None else ctypes.byref(ms[0]), _stream(dev),
     )
@@ -178,7 +196,7 @@ def flash_attention_bwd(
     q, k, v, o, do, lse, *, sm_scale: float, causal: bool = False, kv_lengths=None, bias=None,
     q_valid: int | None = None, kv_valid: int | None = None, workspace=None,
     mods: ScoreModsArgs | None = None, bias_grad: bool = False, ds_route: bool | None = None,
-    fold_bias_grad: bool = False,
+    fold_bias_grad: bool = False, width: int | None = None,
 ):
     """``pjx_flash_bwd``: gradients ``(dq, dk, dv)`` of ``flash_attention_fwd``
     (and, with ``bias_grad``, ``dbias``: dL/d(bias) summed to the bias's own
@@ -213,11 +231,14 @@ def flash_attention_bwd(
     code = _dtype_code(q)
     if Hq % Hkv:
         raise ValueError(f"query heads {Hq} must be a multiple of kv heads {Hkv}")
-    if D not in (64, 128, 256):
+    if width is None and D not in (64, 128, 256):
         raise ValueError(f"head_dim {D} not supported (64, 128 or 256)")
     if not sm_scale > 0:
         raise ValueError("sm_scale must be > 0")
     q, k, v, o, do = (t.contiguous() for t in (q, k, v, o, do))
+    KD = D if width is None else int(width)  # the kernels' head dim
+    if width is not None:
+        q, k, v, o, do = (_aligned(t) for t in (q, k, v, o, do))
     lse = lse.to(torch.float32).contiguous()
     bb = bh = 1
     if bias is not None:
@@ -232,24 +253,25 @@ def flash_attention_bwd(
     if bias_grad and bias is None:
         raise ValueError("bias_grad needs the bias")
     dq, dk, dv = torch.empty_like(q), torch.empty_like(k), torch.empty_like(v)
-    fold = bias_grad and fold_bias_grad and D <= 128 and code != native.PJX_DTYPE_F32 and min(B, Lq, Lk) > 0
+    fold = bias_grad and fold_bias_grad and KD <= 128 and code != native.PJX_DTYPE_F32 and min(B, Lq, Lk) > 0
     dbias = torch.zeros((B, Hq, Lq, Lk), dtype=torch.float32, device=dev) if bias_grad and not fold else None
     lib = native.load()
     nbytes = int(lib.pjx_flash_bwd_workspace_size(B, Hq, Lq))
     if workspace is None:
         ds_bytes = 0
         if bias is None and ms is None:
-            ds_bytes = int(lib.pjx_flash_bwd_ds_workspace_size(code, B, Hq, Lq, Lk, D))
+            ds_bytes = int(lib.pjx_flash_bwd_ds_workspace_size(code, B, Hq, Lq, Lk, KD))
         nbytes = _ds_route_bytes(nbytes, ds_bytes, ds_route, dev,
                                  "the dS route takes 16-bit inputs at head dim 256 without bias or score modifiers")
         if mods is None or (mods.window_left < 0 and mods.window_right < 0 and mods.seq_lengths is None
                             and mods.segment_k is None):
-            split = lib.pjx_flash_bwd_split_workspace_size(code, B, Hq, Hkv, Lq, Lk, D, int(bool(causal)))
+            split = lib.pjx_flash_bwd_split_workspace_size(code, B, Hq, Hkv, Lq, Lk, KD, int(bool(causal)))
             nbytes = max(nbytes, int(split))
     ws = _workspace(nbytes, dev, workspace)
-    rc = lib.pjx_flash_bwd(
+    rc = (lib.pjx_flash_bwd if width is None else lib.pjx_flash_bwd_rows)(
         code, _ptr(q), _ptr(k), _ptr(v), _ptr(o), _ptr(do), _ptr(lse), _ptr(dq),
-        _ptr(dk), _ptr(dv), _ptr(dbias), _ptr(ws), ws.numel(), _ptr(L), _ptr(bias), bb, bh, B, Lq, Lk, Hq, Hkv, D,
+        _ptr(dk), _ptr(dv), _ptr(dbias), _ptr(ws), ws.numel(), _ptr(L), _ptr(bias), bb, bh, B, Lq, Lk, Hq, Hkv,
+        *((D,) if width is None else (KD, D)),
         Lq if q_valid is None else int(q_valid), Lk if kv_valid is None else int(kv_valid),
         int(bool(causal)), float(sm_scale), None if ms is None else ctypes.byref(ms[0]), _stream(dev),
     )
@@ -258,7 +280,7 @@ def flash_attention_bwd(
         dbias = torch.empty_like(bias)
         rc = lib.pjx_flash_dbias(
             code, _ptr(q), _ptr(k), _ptr(v), _ptr(do), _ptr(ws), _ptr(dbias), _ptr(L), _ptr(bias), bb, bh, B, Lq, Lk,
-            Hq, Hkv, D, Lq if q_valid is None else int(q_valid), Lk if kv_valid is None else int(kv_valid),
+            Hq, Hkv, KD, D, Lq if q_valid is None else int(q_valid), Lk if kv_valid is None else int(kv_valid),
             int(bool(causal)), float(sm_scale), None if ms is None else ctypes.byref(ms[0]), _stream(dev),
         )
         native.check(rc)

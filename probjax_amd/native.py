@@ -55,6 +55,11 @@ _SIGNATURES = {
         [ctypes.c_int, _P, _P, _P, _P, _P, _P, _P, _I64, _I64, _I64, _I64, _I64, _I64,
          _I64, _I64, _I64, _I64, ctypes.c_int, ctypes.c_float, _MODS, _P],
     ),
+    "pjx_flash_fwd_rows": (
+        ctypes.c_int,
+        [ctypes.c_int, _P, _P, _P, _P, _P, _P, _P, _I64, _I64, _I64, _I64, _I64, _I64,
+         _I64, _I64, _I64, _I64, _I64, ctypes.c_int, ctypes.c_float, _MODS, _P],
+    ),
     "pjx_flash_bwd_workspace_size": (ctypes.c_size_t, [_I64, _I64, _I64]),
     "pjx_flash_bwd_ds_workspace_size": (ctypes.c_size_t, [ctypes.c_int, _I64, _I64, _I64, _I64, _I64]),
     "pjx_flash_bwd_split_workspace_size": (ctypes.c_size_t, [ctypes.c_int, _I64, _I64, _I64, _I64, _I64, _I64,
@@ -64,9 +69,14 @@ _SIGNATURES = {
         [ctypes.c_int, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, ctypes.c_size_t, _P, _P, _I64,
          _I64, _I64, _I64, _I64, _I64, _I64, _I64, _I64, _I64, ctypes.c_int, ctypes.c_float, _MODS, _P],
     ),
+    "pjx_flash_bwd_rows": (
+        ctypes.c_int,
+        [ctypes.c_int, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, ctypes.c_size_t, _P, _P, _I64, _I64,
+         _I64, _I64, _I64, _I64, _I64, _I64, _I64, _I64, _I64, ctypes.c_int, ctypes.c_float, _MODS, _P],
+    ),
     "pjx_flash_dbias": (
         ctypes.c_int,
-        [ctypes.c_int, _P, _P, _P, _P, _P, _P, _P, _P, _I64, _I64, _I64, _I64, _I64, _I64, _I64, _I64, _I64,
+        [ctypes.c_int, _P, _P, _P, _P, _P, _P, _P, _P, _I64, _I64, _I64, _I64, _I64, _I64, _I64, _I64, _I64, _I64,
          _I64, ctypes.c_int, ctypes.c_float, _MODS, _P],
     ),
     "pjx_empty_rows": (
