@@ -156,6 +156,17 @@ def _int_tensor(x, shape, device):
         return None
 
 
+def _slopes(lb: LoweredBias, h_q: int, device):
+    """Distance slopes per query head, formed on the device: a host tensor would
+    be copied from pageable memory, which waits for the stream.  ALiBi's
+    2^-(h+1) as float32 bit patterns (exponent 126 - h), exact while normal."""
+    if lb.alibi == "decay":
+        return torch.full((h_q,), lb.alibi_alpha, dtype=torch.float32, device=device)
+    if h_q > 126:
+        return torch.tensor([2.0 ** (-(h + 1.0)) for h in range(h_q)], dtype=torch.float32).to(device)
+    return (torch.arange(126, 126 - h_q, -1, dtype=torch.int32, device=device) << 23).view(torch.float32)
+
+
 def _score_mods(lm: LoweredMask, lb: LoweredBias | None, B, l_q, l_k, h_q, device):
     """``ScoreModsArgs`` of the extended masks / modifiers (None when there
     are none), or False when their data does not fit the call."""
@@ -186,11 +197,7 @@ def _score_mods(lm: LoweredMask, lb: LoweredBias | None, B, l_q, l_k, h_q, devic
             return False
     if lb is not None:
         if lb.alibi is not None:
-            if lb.alibi == "decay":
-                slopes = torch.full((h_q,), lb.alibi_alpha, dtype=torch.float32)
-            else:
-                slopes = torch.tensor([2.0 ** (-(h + 1.0)) for h in range(h_q)], dtype=torch.float32)
-            m.alibi_slopes = slopes.to(device)
+            m.alibi_slopes = _slopes(lb, h_q, device)
             m.alibi_symmetric = lb.alibi != "causal"
         m.softcap = float(lb.softcap)
         m.constant = float(lb.constant)
@@ -351,11 +358,14 @@ class _AttentionFunction(torch.autograd.Function):
         ctx.bwd_kwargs = bwd_kwargs
         ctx.bias_dtype = None if bias is None else bias.dtype
         ctx.mark_non_differentiable(lse)
+        ctx.set_materialize_grads(False)  # no zeros for the LSE's gradient
         return out, lse
 
     @staticmethod
     def backward(ctx, dout, dlse=None):
         del dlse  # the LSE output is a residual, not differentiated
+        if dout is None:
+            return None, None, None, None, None, None, None
         q, k, v, o, lse = ctx.saved_tensors
         db = None
         if ctx.bias_dtype is not None and ctx.needs_input_grad[3]:

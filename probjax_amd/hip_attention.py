@@ -69,11 +69,14 @@ def _on_device(*ts):
 
 
 def _ptr(t):
-    return None if t is None else ctypes.c_void_p(t.data_ptr())
+    return None if t is None else t.data_ptr()
 
 
-def _stream(dev) -> ctypes.c_void_p:
-    return ctypes.c_void_p(torch.cuda.current_stream(dev).cuda_stream)
+def _stream(dev) -> int:
+    """The handle of torch's current stream on ``dev`` (as
+    ``torch.cuda.current_stream(dev).cuda_stream``, without building a Stream:
+    0.2 against 2.5 us on every call)."""
+    return torch._C._cuda_getCurrentRawStream(dev.index if dev.index is not None else torch.cuda.current_device())
 
 
 def _lengths(kv_lengths, batch, dev):
@@ -259,7 +262,7 @@ def flash_attention_bwd(
     nbytes = int(lib.pjx_flash_bwd_workspace_size(B, Hq, Lq))
     if workspace is None:
         ds_bytes = 0
-        if bias is None and ms is None:
+        if bias is None and ms is None and (KD == 256 or ds_route):
             ds_bytes = int(lib.pjx_flash_bwd_ds_workspace_size(code, B, Hq, Lq, Lk, KD))
         nbytes = _ds_route_bytes(nbytes, ds_bytes, ds_route, dev,
                                  "the dS route takes 16-bit inputs at head dim 256 without bias or score modifiers")

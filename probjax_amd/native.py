@@ -128,6 +128,8 @@ class NativeLibraryError(RuntimeError):
 def load() -> ctypes.CDLL:
     """Load (once) and return the kernel library; raise if it is unavailable."""
     global _lib
+    if _lib is not None:  # set once, after every symbol is bound
+        return _lib
     with _lock:
         if _lib is not None:
             return _lib

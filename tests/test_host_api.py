@@ -529,3 +529,17 @@ def test_ds_route_workspace_choice(monkeypatch):
     assert H._ds_route_bytes(100, 0, None, dev, "x") == 100
     with pytest.raises(ValueError, match="no route"):
         H._ds_route_bytes(100, 0, True, dev, "no route")
+
+
+def test_slopes_are_exact_powers_of_two():
+    """ALiBi slopes formed as bit patterns equal 2^-(h+1) rounded to float32,
+    also past the last normal exponent."""
+    import torch
+    from probjax_amd import attention as A
+    from probjax_amd.masks import CausalAlibiBias, DistanceDecayBias, lower_bias
+
+    for h in (1, 7, 126, 127, 150):
+        got = A._slopes(lower_bias(CausalAlibiBias()), h, torch.device("cpu"))
+        assert got.dtype == torch.float32
+        assert torch.equal(got, torch.tensor([2.0 ** -(i + 1.0) for i in range(h)], dtype=torch.float32))
+    assert torch.equal(A._slopes(lower_bias(DistanceDecayBias(0.3)), 3, torch.device("cpu")), torch.full((3,), 0.3))
