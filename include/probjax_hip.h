@@ -457,6 +457,21 @@ int pjx_mla_project(int dtype, const void* cache, const void* wk, const void* wv
                     void* v, int64_t batch, int64_t kv_len, int64_t heads, int64_t rank,
                     int64_t qk_dim, int64_t v_dim, int64_t width, void* stream);
 
+/*
+ * Gradients of pjx_mla_project: with dk, dv [B, S, H, width] (the gradients of
+ * its outputs), dcache [B, S, R] = dK W_K + dV W_V, dwk [H, qk_dim, R] = dK^T C,
+ * dwv [H, v_dim, R] = dV^T C (kernels/latent_attention.py:571-589), float32 sums
+ * rounded once.  16-bit; rank, qk_dim and v_dim multiples of 8, width a multiple
+ * of 64, H * width and rank at most 2^20; pointers 16-byte aligned.  workspace: fp32 parts of dW
+ * (pjx_mla_project_bwd_workspace_size bytes), added in a fixed order.
+ */
+size_t pjx_mla_project_bwd_workspace_size(int64_t batch, int64_t kv_len, int64_t heads, int64_t rank,
+                                          int64_t width);
+int pjx_mla_project_bwd(int dtype, const void* cache, const void* wk, const void* wv, const void* dk,
+                        const void* dv, void* dcache, void* dwk, void* dwv, void* workspace,
+                        size_t workspace_bytes, int64_t batch, int64_t kv_len, int64_t heads, int64_t rank,
+                        int64_t qk_dim, int64_t v_dim, int64_t width, void* stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -589,8 +589,9 @@ class _MaterializedMLAFunction(torch.autograd.Function):
     attends the zero-padded ``q`` over them.  Backward: the VJP of that
     materialised computation, as in the reference (:571-589): the flash
     backward gives ``dq, dK, dV``; the projection's chain rule gives
-    ``dC = dK W_K + dV W_V``, ``dW_K = dK^T C``, ``dW_V = dV^T C`` (plain
-    GEMMs, the reference's einsum VJPs).  K and V are kept from the forward
+    ``dC = dK W_K + dV W_V``, ``dW_K = dK^T C``, ``dW_V = dV^T C``
+    (``pjx_mla_project_bwd``; plain GEMMs in float32 and for ranks or head dims
+    that are no multiple of 8).  K and V are kept from the forward
     rather than formed a second time."""
 
     @staticmethod
@@ -608,6 +609,9 @@ class _MaterializedMLAFunction(torch.autograd.Function):
         dk_dim, dv_dim, width = st["dk"], st["dv"], st["width"]
         dop = _pad_head(dout.to(o.dtype), width)
         dqp, dkp, dvp = hip.flash_attention_bwd(qp, k, v, o, dop, lse, sm_scale=st["sm_scale"], **st["plan"])
+        dq = dqp if dk_dim == width else dqp[..., :dk_dim].contiguous()
+        if hip.mla_project_bwd_supported(cache, wk, wv, width):
+            return dq, *hip.mla_project_bwd(cache, wk, wv, dkp, dvp), None
         B, S, R = cache.shape
         H = wk.shape[0]
         dK = dkp[..., :dk_dim].reshape(B * S, H * dk_dim)
@@ -616,7 +620,6 @@ class _MaterializedMLAFunction(torch.autograd.Function):
         dcache = dK @ wk.reshape(H * dk_dim, R) + dV @ wv.reshape(H * dv_dim, R)
         dwk = (dK.t().contiguous() @ c2).reshape(H, dk_dim, R)
         dwv = (dV.t().contiguous() @ c2).reshape(H, dv_dim, R)
-        dq = dqp if dk_dim == width else dqp[..., :dk_dim].contiguous()
         return dq, dcache.reshape(B, S, R), dwk, dwv, None
 
 

@@ -525,3 +525,34 @@ def mla_project(cache, wk, wv, *, width: int):
     )
     native.check(rc)
     return k, v
+
+
+def mla_project_bwd(cache, wk, wv, dk, dv):
+    """``pjx_mla_project_bwd``: ``(dcache, dwk, dwv)`` from the gradients ``dk``,
+    ``dv`` ``[B, S, H, width]`` of ``mla_project``'s outputs (bf16 / fp16; see
+    ``mla_project_bwd_supported``)."""
+    dev = _on_device(cache, wk, wv, dk, dv)
+    code = _half_code("the projection's backward", cache, wk, wv, dk, dv)
+    B, S, R = cache.shape
+    H, dk_dim, dv_dim, width = wk.shape[0], wk.shape[1], wv.shape[1], dk.shape[-1]
+    if tuple(dk.shape) != (B, S, H, width) or dv.shape != dk.shape or wk.shape[2] != R or tuple(wv.shape) != (H, dv_dim, R):
+        raise ValueError("incompatible shapes for the projection's backward")
+    cache, wk, wv, dk, dv = (_aligned(t.contiguous()) for t in (cache, wk, wv, dk, dv))
+    dcache, dwk, dwv = torch.empty_like(cache), torch.empty_like(wk), torch.empty_like(wv)
+    lib = native.load()
+    ws = _workspace(int(lib.pjx_mla_project_bwd_workspace_size(B, S, H, R, width)), dev, None)
+    rc = lib.pjx_mla_project_bwd(
+        code, _ptr(cache), _ptr(wk), _ptr(wv), _ptr(dk), _ptr(dv), _ptr(dcache), _ptr(dwk), _ptr(dwv), _ptr(ws),
+        ws.numel(), B, S, H, R, dk_dim, dv_dim, width, _stream(dev),
+    )
+    native.check(rc)
+    return dcache, dwk, dwv
+
+
+def mla_project_bwd_supported(cache, wk, wv, width: int) -> bool:
+    """Whether ``mla_project_bwd`` takes a latent ``cache [B, S, R]`` projected by
+    ``wk`` / ``wv`` to heads of ``width``: 16-bit, rank and head dims multiples of
+    8 (16-byte loads), sizes its 32-bit tile offsets hold."""
+    R = cache.shape[-1]
+    return (cache.dtype in HALF_DTYPES and not (R % 8 or width % 64 or wk.shape[1] % 8 or wv.shape[1] % 8)
+            and cache.numel() > 0 and max(R, wk.shape[0] * width) <= 1 << 20)

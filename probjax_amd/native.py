@@ -114,6 +114,12 @@ _SIGNATURES = {
         ctypes.c_int,
         [ctypes.c_int, _P, _P, _P, _P, _P, _I64, _I64, _I64, _I64, _I64, _I64, _I64, _P],
     ),
+    "pjx_mla_project_bwd_workspace_size": (ctypes.c_size_t, [_I64, _I64, _I64, _I64, _I64]),
+    "pjx_mla_project_bwd": (
+        ctypes.c_int,
+        [ctypes.c_int, _P, _P, _P, _P, _P, _P, _P, _P, _P, ctypes.c_size_t, _I64, _I64, _I64, _I64, _I64, _I64,
+         _I64, _P],
+    ),
 }
 EXPORTED = tuple(_SIGNATURES)
 
