@@ -322,6 +322,20 @@ int pjx_splitkv_decode(int dtype, const void* q, const void* k, const void* v,
                        int64_t head_dim, int64_t v_dim, float sm_scale, int64_t chunk, void* stream);
 
 /*
+ * pjx_splitkv_decode on rows of row_dim elements (q, k, v and o; a multiple of 8
+ * up to head_dim, 64 or 128, the kernel's width), 16-bit: what zero-padding the
+ * rows to head_dim and slicing the output gives, without the copies.  q, k, v
+ * start on 16 bytes, o on 8; the cache is read with ordinary loads at any size.
+ * workspace: pjx_decode_workspace_size(B, Hkv, rows,
+ * Lk, head_dim, chunk) bytes.
+ */
+int pjx_splitkv_decode_rows(int dtype, const void* q, const void* k, const void* v,
+                            const int32_t* kv_lengths, void* o, float* lse, void* workspace,
+                            size_t workspace_bytes, int64_t batch, int64_t q_len, int64_t kv_len,
+                            int64_t q_heads, int64_t kv_heads, int64_t head_dim, int64_t row_dim,
+                            float sm_scale, int64_t chunk, void* stream);
+
+/*
  * Size of the library-held device array behind pjx_splitkv_decode_static:
  * 32 MiB on each GPU the library runs on, held until the process ends.
  */

@@ -134,13 +134,13 @@ def _row_kv_lengths(kl, B, l_q, device):
     return out
 
 
-def _decode_plan(query, key, value, lm: LoweredMask, lb: LoweredBias | None):
+def _decode_plan(query, key, value, lm: LoweredMask, lb: LoweredBias | None, check_dim: bool = True):
     """Arguments of the split-KV decode for this call, or None."""
     if lb is not None or lm.causal or lm.extended or lm.q_valid is not None or lm.kv_valid is not None:
         return None
     if query.dtype not in KERNEL_DTYPES:
         return None
-    if query.shape[-1] not in DECODE_HEAD_DIMS or value.shape[-1] not in DECODE_HEAD_DIMS:
+    if check_dim and (query.shape[-1] not in DECODE_HEAD_DIMS or value.shape[-1] not in DECODE_HEAD_DIMS):
         return None
     return dict(kv_lengths=lm.kv_lengths)
 
@@ -410,8 +410,10 @@ def _run(query, key, value, lm, lb, sm_scale, split_kv, bias_grad=False, fill=Fa
     d = query.shape[-1]
     width = _kernel_width(d, query.dtype)
     rows = None
-    if width is not None and width != d and not _splitkv_ok(query, key, lm, lb is not None, 0.0, split_kv):
-        # the flash kernels take such rows as they lie in memory
+    split = _splitkv_ok(query, key, lm, lb is not None, 0.0, split_kv)
+    if width is not None and width != d and (
+            not split or (query.dtype in HALF_DTYPES and not _needs_grad(query, key, value))):
+        # the flash kernels, and the 16-bit decode, take such rows as they lie in memory
         rows = hip.rows_width(d, max(query.shape[2], key.shape[2]))
     if width is not None and width != d and rows is None:
         # Zero features change no q.k product and add only zero output
@@ -426,12 +428,12 @@ def _run(query, key, value, lm, lb, sm_scale, split_kv, bias_grad=False, fill=Fa
     grad = _needs_grad(query, key, value) or bias_in is not None
     if grad and query.dtype not in BACKWARD_DTYPES:
         return None
-    if rows is None and _splitkv_ok(query, key, lm, lb is not None, 0.0, split_kv):
-        plan = _decode_plan(query, key, value, lm, lb)
+    if split:
+        plan = _decode_plan(query, key, value, lm, lb, check_dim=rows is None)
         if plan is not None:
             if not grad:
-                return _filled(hip.splitkv_decode(query, key, value, sm_scale=sm_scale, return_lse=fill, **plan),
-                               value, fill)
+                return _filled(hip.splitkv_decode(query, key, value, sm_scale=sm_scale, return_lse=fill, width=rows,
+                                                  **plan), value, fill)
             # Split-KV primal, regular backward (probjax splitkv_attention,
             # kernels/attention_splitkv.py:253-272).
             res = _AttentionFunction.apply(
@@ -548,8 +550,9 @@ def splitkv_forward(q, k, v, *, sm_scale: float, num_splits: int | None = None,
     """Split-KV ("flash-decoding") forward (probjax ``splitkv_forward``,
     kernels/attention_splitkv.py:137-250): bf16 / fp16 / fp32
     ``q [B, Lq, Hq, D]``, ``k [B, Lkv, Hkv, D]``, ``v [B, Lkv, Hkv, Dv]``
-    -> ``[B, Lq, Hq, Dv]``; D and Dv up to 256 (zero-padded to 64, 128 or
-    256, as the reference pads its blocks to the next power of two,
+    -> ``[B, Lq, Hq, Dv]``; D and Dv up to 256 (16-bit D = Dv of a
+    multiple of 8 up to 128 as the rows lie in memory, others zero-padded to 64,
+    128 or 256, as the reference pads its blocks to the next power of two,
     :155-172), any number of packed rows ``(Hq/Hkv)*Lq``.
 
     ``num_splits`` maps to KV chunks of ``ceil(Lkv / num_splits)`` keys rounded
@@ -563,9 +566,12 @@ def splitkv_forward(q, k, v, *, sm_scale: float, num_splits: int | None = None,
     width, v_width = _decode_width(d), _decode_width(dv)
     if width is None or v_width is None:
         raise ValueError(f"splitkv_forward: head dims up to {DECODE_HEAD_DIMS[-1]}, got D={d}, Dv={dv}")
-    if width != d:
+    rows = None
+    if width != d and dv == d and q.dtype in HALF_DTYPES and hip_device(q):
+        rows = hip.rows_width(d, max(q.shape[-2], k.shape[-2]))
+    if width != d and rows is None:
         q, k = _pad_features(q, width), _pad_features(k, width)
-    if v_width != dv:
+    if v_width != dv and rows is None:
         v = _pad_features(v, v_width)
     chunk = 0
     if num_splits is not None:
@@ -574,8 +580,8 @@ def splitkv_forward(q, k, v, *, sm_scale: float, num_splits: int | None = None,
         per = -(-k.shape[1] // num_splits)
         chunk = max(128, -(-per // 128) * 128)
     res = hip.splitkv_decode(q, k, v, sm_scale=float(sm_scale), kv_lengths=kv_lengths,
-                             chunk=chunk, return_lse=return_lse)
-    if v_width == dv:
+                             chunk=chunk, return_lse=return_lse, **({} if rows is None else {"width": rows}))
+    if v_width == dv or rows is not None:
         return res
     return (res[0][..., :dv], res[1]) if return_lse else res[..., :dv]
 

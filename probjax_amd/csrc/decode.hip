@@ -51,7 +51,8 @@ struct DecodeArgs {
   int B, Lq, Lk, Hq, G, rows;
   int fold;      // 1: row = t*H + h (MLA); 0: row = gi*Lq + t (GQA)
   int chunk, nch;
-  int dv;        // output dims
+  int dv;        // output dims of the kernel (the partials' row)
+  int orow;      // elements of an output row in memory (0: dv), and of q, k and v rows in the rows kernels
   float cx;      // sm_scale * log2(e)
   // Query rows per row group: the rows of a KV head are split into groups of
   // `rpg` (16 per MFMA column block of the kernel), one per blockIdx.y; each
@@ -95,7 +96,7 @@ __device__ __forceinline__ void emit_row_elem(const DecodeArgs& a, int b, int g,
     int t, h;
     row_to_head(a, g, r, t, h);
     const float out = Ls > 0.f ? O / Ls : 0.f;
-    const size_t oi = ((size_t)(b * a.Lq + t) * a.Hq + h) * a.dv + d;
+    const size_t oi = ((size_t)(b * a.Lq + t) * a.Hq + h) * a.orow + d;
     if (a.o32)
       a.o32[oi] = out;
     else
@@ -195,7 +196,7 @@ __device__ __forceinline__ void emit_row_quad(const DecodeArgs& a, int b, int g,
     int t, h;
     row_to_head(a, g, r, t, h);
     const float inv = Ls > 0.f ? 1.f / Ls : 0.f;
-    const size_t oi = ((size_t)(b * a.Lq + t) * a.Hq + h) * a.dv + d;
+    const size_t oi = ((size_t)(b * a.Lq + t) * a.Hq + h) * a.orow + d;
     if (a.o32) {
       *(f32x4*)(a.o32 + oi) = O * inv;
     } else {
@@ -258,6 +259,7 @@ __device__ __forceinline__ void combine_rows(const DecodeArgs& a, float* red, co
   const int nr = min(16, a.rows - row0 - 16 * rb);
   for (int e = tid; e < nr * D; e += 256) {
     const int r = e / D, d = e % D;
+    if (d >= a.orow) continue;
     float M = kMaxInit;
 #pragma unroll
     for (int ww = 0; ww < 4; ++ww) M = fmaxf(M, red_ml[(ww * 16 + r) * 2]);
@@ -277,13 +279,16 @@ __device__ __forceinline__ void combine_rows(const DecodeArgs& a, float* red, co
 template <int D, int DV, int NRB>
 constexpr int decode_occupancy() { return (NRB == 4 || D > 128 || DV > 128) ? 1 : 2; }
 
-template <typename E, int D, int DV, int NRB, bool STREAM>
-__global__ __launch_bounds__(256, (decode_occupancy<D, DV, NRB>())) void gqa_decode_kernel(DecodeArgs a) {
+// ROWS: q, k, v and o rows hold a.orow elements (a multiple of 8, below D = DV)
+// and the lanes whose chunk lies past a row's end hold zeros instead of loading.
+template <typename E, int D, int DV, int NRB, bool STREAM, bool ROWS>
+__device__ __forceinline__ void gqa_decode(const DecodeArgs& a) {
   constexpr int KSTEPS = D / 32;  // 32-dim MFMA k-steps of Q.K
   constexpr int NDB = DV / 16;    // 16-dim output blocks
   constexpr int DC = DV / 8;      // 16-byte chunks per V row
   constexpr int VU = DV / 64;     // (4 keys x 8 dims) V units per lane per 32 keys
   constexpr int CR = D / 8;       // 16-byte chunks per K row
+  static_assert(!(ROWS && STREAM), "rows of any length take ordinary loads");
   constexpr int KLD = D / 16;     // K chunks per lane per 32-key step (32 * CR / 64 = 2 * KSTEPS)
   static_assert(D % 64 == 0 && DV % 64 == 0, "head dims");
   // Each wave's V^T tile: DV rows (output dims) of the step's 32 keys, 64
@@ -319,6 +324,7 @@ __global__ __launch_bounds__(256, (decode_occupancy<D, DV, NRB>())) void gqa_dec
   const int w1 = min(w0 + per_wave, L);
 
   const int row0 = blockIdx.y * 16 * NRB;  // this row group's first row
+  const int rd = ROWS ? a.orow : D, rdv = ROWS ? a.orow : DV;
   typename E::v8 qf[NRB][KSTEPS];
 #pragma unroll
   for (int rb = 0; rb < NRB; ++rb) {
@@ -326,17 +332,17 @@ __global__ __launch_bounds__(256, (decode_occupancy<D, DV, NRB>())) void gqa_dec
     const bool rv = row < a.rows;
     int t = 0, h = 0;
     if (rv) row_to_head(a, g, row, t, h);
-    const uint16_t* qrow = a.q + ((size_t)(b * a.Lq + t) * a.Hq + h) * D;
+    const uint16_t* qrow = a.q + ((size_t)(b * a.Lq + t) * a.Hq + h) * rd;
 #pragma unroll
     for (int s = 0; s < KSTEPS; ++s) {
       u32x4 r = {0u, 0u, 0u, 0u};
-      if (rv) r = *(const u32x4*)(qrow + 32 * s + 8 * q4);
+      if (rv && (!ROWS || 32 * s + 8 * q4 < rd)) r = *(const u32x4*)(qrow + 32 * s + 8 * q4);
       qf[rb][s] = E::as8(r);
     }
   }
-  const size_t k_tok = (size_t)a.G * D, v_tok = (size_t)a.G * DV;
-  const uint16_t* Kb = a.k + ((size_t)b * a.Lk * a.G + g) * D;
-  const uint16_t* Vb = a.v + ((size_t)b * a.Lk * a.G + g) * DV;
+  const size_t k_tok = (size_t)a.G * rd, v_tok = (size_t)a.G * rdv;
+  const uint16_t* Kb = a.k + ((size_t)b * a.Lk * a.G + g) * rd;
+  const uint16_t* Vb = a.v + ((size_t)b * a.Lk * a.G + g) * rdv;
   uint16_t* vl = vt_lds + w * DV * 32;
   // Element offset of 8-byte unit u (keys 4u .. 4u+3) of V^T row r.  The 32
   // units of a 256-byte line (rows 4L .. 4L+3) are XOR-swizzled by F(L) so
@@ -390,7 +396,7 @@ __global__ __launch_bounds__(256, (decode_occupancy<D, DV, NRB>())) void gqa_dec
 #pragma unroll
         for (int s = 0; s < KSTEPS; ++s) {
           u32x4 r = {0u, 0u, 0u, 0u};
-          if (ok) r = *(const u32x4*)(p + 32 * s);
+          if (ok && (!ROWS || 32 * s + 8 * q4 < rd)) r = *(const u32x4*)(p + 32 * s);
           kr[kb * KSTEPS + s] = r;
         }
       }
@@ -412,7 +418,7 @@ __global__ __launch_bounds__(256, (decode_occupancy<D, DV, NRB>())) void gqa_dec
       for (int j = 0; j < 4; ++j) {
         const int key = k0 + 4 * kq + j;
         u32x4 r = {0u, 0u, 0u, 0u};
-        if (key < w1) r = ld16(Vb + (size_t)key * v_tok + 8 * dc);
+        if (key < w1 && (!ROWS || 8 * dc < rdv)) r = ld16(Vb + (size_t)key * v_tok + 8 * dc);
         vr[i][j] = r;
       }
     }
@@ -545,6 +551,24 @@ __global__ __launch_bounds__(256, (decode_occupancy<D, DV, NRB>())) void gqa_dec
   for (int rb = 0; rb < NRB; ++rb)
     combine_rows<DV>(a, (float*)vt_lds, acc[rb], m_run[rb], xor32_sum(xor16_sum(l_run[rb])), row0, rb, b, g,
                      part, final_out);
+}
+
+template <typename E, int D, int DV, int NRB, bool STREAM>
+__global__ __launch_bounds__(256, (decode_occupancy<D, DV, NRB>())) void gqa_decode_kernel(DecodeArgs a) {
+  gqa_decode<E, D, DV, NRB, STREAM, false>(a);
+}
+
+// Head dims that are no kernel width, on the cache as it lies in memory: bound
+// by its bytes, like the kernels above, at about the rate of a plain copy.
+// Zero-padding the cache to the width on every step read it once and wrote and
+// read it width / dim times as large.  bf16, us, padded -> rows (B, S, Hq, Hkv,
+// D): (1,2048,8,8,80) 43 -> 14; (16,8192,32,8,96) 388 -> 85; (32,8192,32,8,80)
+// 831 -> 153 (4.4 TB/s); (32,8192,32,8,40) 536 -> 129.  Non-temporal loads, which
+// need whole 128-byte lines, were slower at every size (1.3 GB at D = 80: 326
+// against 294 us), so these rows always take ordinary ones.
+template <typename E, int D, int NRB>
+__global__ __launch_bounds__(256, (decode_occupancy<D, D, NRB>())) void gqa_decode_rows_kernel(DecodeArgs a) {
+  gqa_decode<E, D, D, NRB, false, true>(a);
 }
 
 // ---------------------------------------------------------------------------
@@ -950,7 +974,7 @@ __global__ __launch_bounds__(kDecThreads, 1) void mla_decode_kernel(DecodeArgs a
 constexpr int kMergeThreads = 128;
 constexpr int kMergeBatch = 16;
 __global__ __launch_bounds__(kMergeThreads) void decode_merge_kernel(DecodeArgs a) {
-  const int nq = a.dv / 4;
+  const int nq = a.orow / 4;
   const long gid = (long)blockIdx.x * kMergeThreads + threadIdx.x;
   const long item = gid / nq;
   const int u = (int)(gid % nq);
@@ -1014,7 +1038,7 @@ __global__ __launch_bounds__(kMergeThreads) void decode_merge_kernel(DecodeArgs 
   int t, h;
   row_to_head(a, g, r, t, h);
   const float inv = den > 0.f ? 1.f / den : 0.f;
-  const size_t oi = ((size_t)(b * a.Lq + t) * a.Hq + h) * a.dv + 4 * u;
+  const size_t oi = ((size_t)(b * a.Lq + t) * a.Hq + h) * a.orow + 4 * u;
   if (a.o32) {
     *(f32x4*)(a.o32 + oi) = num * inv;
   } else {
@@ -1060,6 +1084,7 @@ static size_t ws_size(int64_t batch, int64_t groups, int64_t rows, int64_t kv_le
 template <auto K>
 static int run_decode(DecodeArgs& a, void* workspace, size_t ws_bytes,
                       hipStream_t stream, const char* name) {
+  if (a.orow == 0) a.orow = a.dv;
   const size_t need = ws_size(a.B, a.G, a.rows, a.Lk, a.dv, a.chunk);
   if (!workspace || ws_bytes < need) return fail(PJX_ERR_WORKSPACE, "decode: workspace missing or too small");
   const size_t parts = (size_t)a.B * a.G * a.nch * a.rows;
@@ -1072,7 +1097,7 @@ static int run_decode(DecodeArgs& a, void* workspace, size_t ws_bytes,
   launch_kernel<K>(dim3((unsigned)blocks, (unsigned)groups), dim3(kDecThreads), 0, stream, a);
   int rc = check_launch(name);
   if (rc) return rc;
-  const long merge_threads = (long)a.B * a.G * a.rows * (a.dv / 4);
+  const long merge_threads = (long)a.B * a.G * a.rows * (a.orow / 4);
   launch_kernel<decode_merge_kernel>(dim3((unsigned)((merge_threads + kMergeThreads - 1) / kMergeThreads)),
                      dim3(kMergeThreads), 0, stream, a);
   return check_launch(name);
@@ -1101,6 +1126,21 @@ static int run_gqa_dims(DecodeArgs& a, int nrb, bool streamed, void* ws, size_t 
                         const char* who) {
   return streamed ? run_gqa_nrb<E, D, DV, true>(a, nrb, ws, ws_bytes, s, who)
                   : run_gqa_nrb<E, D, DV, false>(a, nrb, ws, ws_bytes, s, who);
+}
+
+// Rows of a.orow <= D elements (gqa_decode_rows_kernel), q/k and v alike.
+template <typename E, int D>
+static int run_gqa_rows(DecodeArgs& a, int nrb, void* ws, size_t ws_bytes, hipStream_t s, const char* who) {
+  if (nrb == 1) return run_decode<gqa_decode_rows_kernel<E, D, 1>>(a, ws, ws_bytes, s, who);
+  if (nrb == 2) return run_decode<gqa_decode_rows_kernel<E, D, 2>>(a, ws, ws_bytes, s, who);
+  return run_decode<gqa_decode_rows_kernel<E, D, 4>>(a, ws, ws_bytes, s, who);
+}
+
+template <typename E>
+static int run_gqa_rows_dim(DecodeArgs& a, int head_dim, int nrb, void* ws, size_t ws_bytes, hipStream_t s,
+                            const char* who) {
+  return head_dim == 64 ? run_gqa_rows<E, 64>(a, nrb, ws, ws_bytes, s, who)
+                        : run_gqa_rows<E, 128>(a, nrb, ws, ws_bytes, s, who);
 }
 
 template <int D, int DV>
@@ -1202,23 +1242,27 @@ extern "C" size_t pjx_decode_workspace_size(int64_t batch, int64_t groups, int64
   return ws_size(batch, groups, rows, kv_len, v_dim, chunk);
 }
 
-extern "C" int pjx_splitkv_decode(int dtype, const void* q, const void* k, const void* v,
-                                  const int32_t* kv_lengths, void* o, float* lse,
-                                  void* workspace, size_t workspace_bytes, int64_t batch,
-                                  int64_t q_len, int64_t kv_len, int64_t q_heads,
-                                  int64_t kv_heads, int64_t head_dim, int64_t v_dim, float sm_scale,
-                                  int64_t chunk, void* stream) {
+// row_dim: elements of the q, k, v and o rows of a call at head_dim = v_dim, the
+// kernel's width (0: rows of head_dim and v_dim).
+static int gqa_decode_entry(const char* who, int dtype, const void* q, const void* k, const void* v,
+                            const int32_t* kv_lengths, void* o, float* lse, void* workspace,
+                            size_t workspace_bytes, int64_t batch, int64_t q_len, int64_t kv_len, int64_t q_heads,
+                            int64_t kv_heads, int64_t head_dim, int64_t v_dim, int64_t row_dim, float sm_scale,
+                            int64_t chunk, void* stream) {
   clear_error();
-  const char* who = "pjx_splitkv_decode";
   const int vrc = check_gqa_decode(who, dtype, batch, q_len, kv_len, q_heads, kv_heads, head_dim, v_dim, sm_scale,
                                    &chunk);
   if (vrc != PJX_OK) return vrc;
   // an empty cache (kv_len == 0) may come as null pointers
-  if (!q || !o || (batch * kv_len > 0 && (!k || !v))) return fail(PJX_ERR_INVALID, "pjx_splitkv_decode: null pointer");
+  if (!q || !o || (batch * kv_len > 0 && (!k || !v))) {
+    char buf[64];
+    snprintf(buf, sizeof(buf), "%s: null pointer", who);
+    return fail(PJX_ERR_INVALID, buf);
+  }
   const bool f32 = dtype == PJX_DTYPE_F32;
   if (batch == 0) return PJX_OK;
   if (kv_len == 0)
-    return write_keyless(o, lse, (size_t)(batch * q_len * q_heads * v_dim), f32, (size_t)(batch * q_heads * q_len),
+    return write_keyless(o, lse, (size_t)(batch * q_len * q_heads * (row_dim ? row_dim : v_dim)), f32, (size_t)(batch * q_heads * q_len),
                          (hipStream_t)stream, who);
   const int64_t rows = (q_heads / kv_heads) * q_len;
   DecodeArgs a = {};
@@ -1232,15 +1276,46 @@ extern "C" int pjx_splitkv_decode(int dtype, const void* q, const void* k, const
   a.B = (int)batch; a.Lq = (int)q_len; a.Lk = (int)kv_len; a.Hq = (int)q_heads; a.G = (int)kv_heads;
   a.rows = (int)rows; a.fold = 0; a.chunk = (int)chunk;
   a.nch = (int)std::max<int64_t>((kv_len + chunk - 1) / chunk, 1);
-  a.dv = (int)v_dim; a.cx = sm_scale * kLog2e;
+  a.dv = (int)v_dim; a.orow = (int)row_dim; a.cx = sm_scale * kLog2e;
   const int nrb = gqa_row_blocks(rows, head_dim, v_dim, f32);
   a.rpg = kRows * nrb;
   hipStream_t s = (hipStream_t)stream;
   const int d = (int)head_dim, dv = (int)v_dim;
+  if (row_dim)
+    return a.f16 ? run_gqa_rows_dim<F16Fmt>(a, d, nrb, workspace, workspace_bytes, s, who)
+                 : run_gqa_rows_dim<Bf16Fmt>(a, d, nrb, workspace, workspace_bytes, s, who);
   const bool streamed = !f32 && decode_streams_kv(batch * kv_len * kv_heads * (head_dim + v_dim) * 2, kStreamBytes);
   if (f32) return run_gqa<Bf16Fmt, true>(a, d, dv, nrb, false, workspace, workspace_bytes, s, who);
   return a.f16 ? run_gqa<F16Fmt, false>(a, d, dv, nrb, streamed, workspace, workspace_bytes, s, who)
                : run_gqa<Bf16Fmt, false>(a, d, dv, nrb, streamed, workspace, workspace_bytes, s, who);
+}
+
+extern "C" int pjx_splitkv_decode(int dtype, const void* q, const void* k, const void* v,
+                                  const int32_t* kv_lengths, void* o, float* lse,
+                                  void* workspace, size_t workspace_bytes, int64_t batch,
+                                  int64_t q_len, int64_t kv_len, int64_t q_heads,
+                                  int64_t kv_heads, int64_t head_dim, int64_t v_dim, float sm_scale,
+                                  int64_t chunk, void* stream) {
+  return gqa_decode_entry("pjx_splitkv_decode", dtype, q, k, v, kv_lengths, o, lse, workspace, workspace_bytes, batch,
+                          q_len, kv_len, q_heads, kv_heads, head_dim, v_dim, 0, sm_scale, chunk, stream);
+}
+
+extern "C" int pjx_splitkv_decode_rows(int dtype, const void* q, const void* k, const void* v,
+                                       const int32_t* kv_lengths, void* o, float* lse, void* workspace,
+                                       size_t workspace_bytes, int64_t batch, int64_t q_len, int64_t kv_len,
+                                       int64_t q_heads, int64_t kv_heads, int64_t head_dim, int64_t row_dim,
+                                       float sm_scale, int64_t chunk, void* stream) {
+  clear_error();
+  if (dtype != PJX_DTYPE_BF16 && dtype != PJX_DTYPE_F16)
+    return fail(PJX_ERR_INVALID, "pjx_splitkv_decode_rows: dtype must be PJX_DTYPE_BF16 or PJX_DTYPE_F16");
+  if ((head_dim != 64 && head_dim != 128) || row_dim <= 0 || row_dim % 8 || row_dim > head_dim)
+    return fail(PJX_ERR_INVALID,
+                "pjx_splitkv_decode_rows: head_dim must be 64 or 128, row_dim a multiple of 8 up to it");
+  if (((uintptr_t)q | (uintptr_t)k | (uintptr_t)v) % 16 || (uintptr_t)o % 8)
+    return fail(PJX_ERR_INVALID, "pjx_splitkv_decode_rows: q, k, v must start on 16 bytes and o on 8");
+  return gqa_decode_entry("pjx_splitkv_decode_rows", dtype, q, k, v, kv_lengths, o, lse, workspace, workspace_bytes,
+                          batch, q_len, kv_len, q_heads, kv_heads, head_dim, head_dim, row_dim, sm_scale, chunk,
+                          stream);
 }
 
 // ---------------------------------------------------------------------------

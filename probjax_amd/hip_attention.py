@@ -350,11 +350,12 @@ def _workspace(nbytes, dev, workspace):
 
 def splitkv_decode(
     q, k, v, *, sm_scale: float, kv_lengths=None, chunk: int = 0, return_lse: bool = False,
-    workspace=None,
+    workspace=None, width: int | None = None,
 ):
     """``pjx_splitkv_decode``: bf16, fp16 or fp32 ``q [B, Lq, Hq, D]``,
     ``k [B, S, Hkv, D]``, ``v [B, S, Hkv, Dv]`` -> ``o [B, Lq, Hq, Dv]``; D and
-    Dv each 64, 128 or 256, any number of packed rows ``(Hq/Hkv)*Lq``."""
+    Dv each 64, 128 or 256, any number of packed rows ``(Hq/Hkv)*Lq``.  With
+    ``width`` (``rows_width(D)``, 16-bit, Dv = D): ``pjx_splitkv_decode_rows``."""
     dev = _on_device(q, k, v)
     if q.ndim != 4 or k.ndim != 4 or v.ndim != 4 or k.shape[:3] != v.shape[:3]:
         raise ValueError("q must be [B, Lq, Hq, D], k [B, S, Hkv, D] and v [B, S, Hkv, Dv]")
@@ -365,18 +366,27 @@ def splitkv_decode(
         raise ValueError(f"incompatible shapes q {tuple(q.shape)}, k {tuple(k.shape)}")
     if q.dtype not in _DTYPES or k.dtype != q.dtype or v.dtype != q.dtype:
         raise ValueError("split-KV decode takes bfloat16, float16 or float32 q, k, v of one dtype")
-    if D not in (64, 128, 256) or Dv not in (64, 128, 256):
+    if width is not None:
+        if q.dtype not in HALF_DTYPES or Dv != D or width not in (64, 128) or D % 8 or not 0 < D <= width:
+            raise ValueError(f"split-KV decode at width {width}: 16-bit rows of a multiple of 8 elements up to it, "
+                             f"Dv = D; got D={D}, Dv={Dv}")
+    elif D not in (64, 128, 256) or Dv not in (64, 128, 256):
         raise ValueError(f"split-KV decode needs head dims 64, 128 or 256, got D={D}, Dv={Dv}")
     rows = (Hq // Hkv) * Lq
     q, k, v = q.contiguous(), k.contiguous(), v.contiguous()
     L = _lengths(kv_lengths, B, dev)
-    nbytes = decode_workspace_bytes(B, Hkv, rows, S, Dv, chunk)
+    nbytes = decode_workspace_bytes(B, Hkv, rows, S, Dv if width is None else width, chunk)
     ws = _workspace(nbytes, dev, workspace)
     o = torch.empty((B, Lq, Hq, Dv), dtype=q.dtype, device=dev)
     lse = torch.empty((B, Hq, Lq), dtype=torch.float32, device=dev) if return_lse else None
-    rc = native.load().pjx_splitkv_decode(
+    if width is None:
+        entry, dims = native.load().pjx_splitkv_decode, (D, Dv)
+    else:
+        entry, dims = native.load().pjx_splitkv_decode_rows, (width, D)
+        q, k, v = _aligned(q), _aligned(k), _aligned(v)
+    rc = entry(
         _dtype_code(q), _ptr(q), _ptr(k), _ptr(v), _ptr(L), _ptr(o), _ptr(lse), _ptr(ws),
-        nbytes, B, Lq, S, Hq, Hkv, D, Dv, float(sm_scale), int(chunk), _stream(dev),
+        nbytes, B, Lq, S, Hq, Hkv, *dims, float(sm_scale), int(chunk), _stream(dev),
     )
     native.check(rc)
     return (o, lse) if return_lse else o
