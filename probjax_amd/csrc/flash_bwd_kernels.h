@@ -1,4 +1,5 @@
-// Flash-attention backward for gfx950 (bf16, fp16 or fp32 inputs, fp32 accumulation).
+// Flash-attention backward for gfx950 (bf16 or fp16 inputs, fp32 accumulation; the
+// fp32 kernels, of the same math, are in flash_f32_bwd.h and flash_f32_wide.hip).
 //
 // Replaces the Pallas backward of probjax's `mha`:
 //   _preprocess_backward_kernel (probjax/nn/pallas_kernels/kernels/attention.py:853-867)
@@ -8,7 +9,7 @@
 //   delta = sum_d o * do;  p = exp2(s * log2e - lse * log2e);  dp = do . v^T
 //   ds = p * (dp - delta) * sm_scale
 //   dv = sum_q r(p)^T do,  dk = sum_q r(ds)^T q,  dq = sum_k r(ds) k,
-// r() rounding to the input's 16-bit format (bf16 or fp16; none in fp32).
+// r() rounding to the input's 16-bit format (bf16 or fp16).
 // s is the forward's score: sm_scale * q.k [+ bias], masked keys excluded.
 // lse is the forward's natural-log residual (+inf for rows without a valid
 // key: p = 0 there, so those rows contribute nothing).

@@ -2,10 +2,10 @@
 // v_mfma_f32_16x16x4f32 (full fp32 products, the 1e-5 bar).
 //
 // The reference's fused route takes float32 with head dims up to 256
-// (probjax/nn/layers/attention.py:1187, 1193-1195).  The fp32 kernels of
-// flash_fwd.hip / flash_bwd_kernels.h hold half rows of 32 queries (or keys)
-// per lane on v_mfma_f32_32x32x2f32, which at D = 256 needs more than a wave's
-// 512 registers; these hold 16 rows per wave instead:
+// (probjax/nn/layers/attention.py:1187, 1193-1195).  The narrower
+// fp32 kernels (flash_f32.hip, flash_f32_bwd.h) hold three bf16 planes and the
+// sums of 32 queries (or keys) per wave, which at D = 256 needs more than a
+// wave's 512 registers; these hold 16 rows per wave instead:
 //   * 16x16x4 MFMA layouts (lane l = 16*q4 + c16): A lane l holds
 //     A[c16][q4], B lane l holds B[q4][c16], C lane l holds C[4*q4 + i][c16]
 //     in register i.  Products contracting the head dim take dims
