@@ -367,13 +367,20 @@ class _AttentionFunction(torch.autograd.Function):
         if dout is None:
             return None, None, None, None, None, None, None
         q, k, v, o, lse = ctx.saved_tensors
+        do = dout
+        if ctx.fill:
+            # A row without a valid key reaches q, k and the bias by no path, so
+            # the kernels see zeros there: their P = 0 times an infinite or NaN
+            # dO (or mean of V) would be NaN in dq, dk and dbias.
+            empty = torch.isinf(lse).transpose(1, 2)[..., None]
+            do, o = torch.where(empty, 0, dout), torch.where(empty, 0, o)
         db = None
         if ctx.bias_dtype is not None and ctx.needs_input_grad[3]:
-            dq, dk, dv, db = hip.flash_attention_bwd(q, k, v, o, dout, lse, bias_grad=True, fold_bias_grad=True,
+            dq, dk, dv, db = hip.flash_attention_bwd(q, k, v, o, do, lse, bias_grad=True, fold_bias_grad=True,
                                                      **ctx.bwd_kwargs)
             db = db.to(ctx.bias_dtype)
         else:
-            dq, dk, dv = hip.flash_attention_bwd(q, k, v, o, dout, lse, **ctx.bwd_kwargs)
+            dq, dk, dv = hip.flash_attention_bwd(q, k, v, o, do, lse, **ctx.bwd_kwargs)
         if ctx.fill:
             hip.empty_rows(lse, dout, dv, grad=True)
         return dq, dk, dv, db, None, None, None

@@ -92,3 +92,31 @@ def test_empty_rows(device, dtype, B, Lq, Lk, Hq, Hkv, D):
         want, dv = want.detach().float(), dv.float()
         assert float((got.float() - want).abs().max()) <= eps * float(want.abs().max())
         assert float((dgot.float() - dv).abs().max()) <= 4 * eps * max(float(dv.abs().max()), 1e-6)
+
+
+@pytest.mark.parametrize("dtype,D,bias", [("bf16", 64, True), ("f16", 96, False), ("f32", 64, True), ("bf16", 256, False)])
+def test_empty_rows_keep_nonfinite_gradients(device, dtype, D, bias):
+    """An infinite or NaN dO in a row without a valid key reaches dV alone (the
+    row's output is the mean of V): dq, dk and dbias are bitwise those of a
+    finite dO there."""
+    import torch
+    from probjax_amd import attention as A
+
+    tdt = {"bf16": torch.bfloat16, "f16": torch.float16, "f32": torch.float32}[dtype]
+    B, L, H = 2, 130, 2
+    q, k, v, do = (to_dev(x, device, tdt) for x in rng_normal(55, *[(B, L, H, D)] * 4))
+    keep = torch.ones((B, 1, L, L), dtype=torch.bool, device=device)
+    keep[0, 0, 5] = False
+    keep[1, 0, 64:70] = False
+    tb = torch.zeros((H, L, L), device=device).requires_grad_() if bias else None
+    leaves = [x.requires_grad_() for x in (q, k, v)] + ([tb] if bias else [])
+    bad = do.clone()
+    bad[0, 5, 0] = float("inf")
+    bad[1, 66, 1] = float("nan")
+    out = A.dot_product_attention(q, k, v, mask=keep, bias=tb, implementation="hip")
+    want = torch.autograd.grad(out, leaves, do, retain_graph=True)
+    got = torch.autograd.grad(out, leaves, bad)
+    for i in (i for i in range(len(leaves)) if i != 2):
+        assert torch.isfinite(want[i]).all() and torch.equal(got[i], want[i])
+    assert not torch.isfinite(got[2][0, :, 0]).any() and not torch.isfinite(got[2][1, :, 1]).any()
+    assert torch.equal(got[2][0, :, 1], want[2][0, :, 1])

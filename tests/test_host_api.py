@@ -543,3 +543,33 @@ def test_slopes_are_exact_powers_of_two():
         assert got.dtype == torch.float32
         assert torch.equal(got, torch.tensor([2.0 ** -(i + 1.0) for i in range(h)], dtype=torch.float32))
     assert torch.equal(A._slopes(lower_bias(DistanceDecayBias(0.3)), 3, torch.device("cpu")), torch.full((3,), 0.3))
+
+
+def test_flax_empty_rows_backward_inputs(monkeypatch):
+    """The backward kernels see zeros in dO and in the output of a row without a
+    valid key, whatever dO holds there; dV's share takes dO itself."""
+    q, k, v = (torch.randn(2, 3, 2, 8, requires_grad=True) for _ in range(3))
+    lse = torch.zeros(2, 2, 3)
+    lse[0, 1, 2] = float("inf")
+    seen = {}
+
+    def fill(lse, src, dst, *, grad):
+        seen["grad" if grad else "fwd"] = src
+        if not grad:
+            dst[0, 2, 1] = float("nan")  # the mean of a V with a NaN
+
+    def bwd(q, k, v, o, do, lse, **kw):
+        seen.update(o=o, do=do)
+        return torch.zeros_like(q), torch.zeros_like(k), torch.zeros_like(v)
+
+    monkeypatch.setattr(A.hip, "empty_rows", fill)
+    monkeypatch.setattr(A.hip, "flash_attention_bwd", bwd)
+    raw = torch.randn(2, 3, 2, 8)
+    out, _ = A._AttentionFunction.apply(q, k, v, None, lambda *_: (raw.clone(), lse), {}, True)
+    do = torch.randn(2, 3, 2, 8)
+    do[0, 2, 1, 0] = float("inf")
+    torch.autograd.grad(out, (q, k, v), do)
+    want_o, want_do = raw.clone(), do.clone()
+    want_o[0, 2, 1], want_do[0, 2, 1] = 0, 0
+    assert torch.equal(seen["o"], want_o) and torch.equal(seen["do"], want_do)
+    assert torch.equal(seen["grad"], do)
