@@ -280,6 +280,17 @@ int pjx_empty_rows(int dtype, int grad, const float* lse, const void* src, void*
                    void* stream);
 
 /*
+ * The output and dO [B, Lq, Hq, D] that pjx_flash_bwd takes after
+ * pjx_empty_rows filled the output: copies (o_rows, dout_rows; not the sources)
+ * with zeros in the rows without a valid key, which reach q, k and the bias by
+ * no path.  head_dim <= 256; rows are whole 16-byte chunks and all but lse start
+ * on 16 bytes.
+ */
+int pjx_zero_empty_rows(int dtype, const float* lse, const void* o, const void* dout, void* o_rows,
+                        void* dout_rows, int64_t batch, int64_t q_len, int64_t q_heads, int64_t head_dim,
+                        void* stream);
+
+/*
  * Bytes of workspace pjx_splitkv_decode / pjx_mla_decode need for these sizes
  * (partial outputs and log-sum-exp terms of every KV chunk).
  *   rows   -- query rows per (batch, kv head): (Hq/Hkv)*Lq for GQA decode,

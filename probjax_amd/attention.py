@@ -372,8 +372,7 @@ class _AttentionFunction(torch.autograd.Function):
             # A row without a valid key reaches q, k and the bias by no path, so
             # the kernels see zeros there: their P = 0 times an infinite or NaN
             # dO (or mean of V) would be NaN in dq, dk and dbias.
-            empty = torch.isinf(lse).transpose(1, 2)[..., None]
-            do, o = torch.where(empty, 0, dout), torch.where(empty, 0, o)
+            o, do = hip.zero_empty_rows(lse, o, dout)
         db = None
         if ctx.bias_dtype is not None and ctx.needs_input_grad[3]:
             dq, dk, dv, db = hip.flash_attention_bwd(q, k, v, o, do, lse, bias_grad=True, fold_bias_grad=True,

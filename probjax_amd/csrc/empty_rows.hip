@@ -111,6 +111,30 @@ __global__ __launch_bounds__(kEmptyThreads) void empty_rows_grad_kernel(EmptyArg
   }
 }
 
+// The output and dO as the backward kernels see them: copies with zeros in such
+// rows, blockIdx.z 0 and 1.  One pass over memory, 16 bytes a lane (a row of any
+// kernel's head dim is whole 16-byte chunks), indexed in 32 bits within a batch
+// entry.  A step over 2x2048x8x64 in bf16 with a learned bias: 350 us with torch
+// operations (compare, two selects by row) here, 319 with this kernel.
+struct ZeroArgs {
+  const float* lse;     // [B, Hq, Lq]
+  const u32x4* src[2];  // [B, Lq, Hq, per]
+  u32x4* dst[2];
+  int B, Lq, Hq, per;
+};
+
+__global__ __launch_bounds__(kEmptyThreads) void zero_empty_rows_kernel(ZeroArgs a) {
+  const uint32_t e = blockIdx.x * (uint32_t)kEmptyThreads + threadIdx.x;
+  const uint32_t n = (uint32_t)a.Lq * a.Hq * a.per;
+  if (e >= n) return;
+  const uint32_t row = e / a.per, t = row / a.Hq, h = row % a.Hq;
+  for (int b = blockIdx.y; b < a.B; b += gridDim.y) {
+    u32x4 x = a.src[blockIdx.z][(size_t)b * n + e];
+    if (__float_as_uint(a.lse[((size_t)b * a.Hq + h) * a.Lq + t]) == kPosInfBits) x = u32x4{0u, 0u, 0u, 0u};
+    a.dst[blockIdx.z][(size_t)b * n + e] = x;
+  }
+}
+
 template <int DT>
 static int launch_empty(const EmptyArgs& a, bool grad, hipStream_t s) {
   if (grad)
@@ -140,4 +164,28 @@ extern "C" int pjx_empty_rows(int dtype, int grad, const float* lse, const void*
   if (dtype == PJX_DTYPE_F32) return launch_empty<PJX_DTYPE_F32>(a, grad != 0, s);
   return dtype == PJX_DTYPE_F16 ? launch_empty<PJX_DTYPE_F16>(a, grad != 0, s)
                                 : launch_empty<PJX_DTYPE_BF16>(a, grad != 0, s);
+}
+
+extern "C" int pjx_zero_empty_rows(int dtype, const float* lse, const void* o, const void* dout, void* o_rows,
+                                   void* dout_rows, int64_t batch, int64_t q_len, int64_t q_heads, int64_t head_dim,
+                                   void* stream) {
+  clear_error();
+  if (dtype != PJX_DTYPE_BF16 && dtype != PJX_DTYPE_F16 && dtype != PJX_DTYPE_F32)
+    return fail(PJX_ERR_INVALID, "pjx_zero_empty_rows: dtype must be PJX_DTYPE_BF16, PJX_DTYPE_F16 or PJX_DTYPE_F32");
+  const int64_t row_bytes = head_dim * (dtype == PJX_DTYPE_F32 ? 4 : 2), per = row_bytes / 16;
+  // the chunks of a batch entry, and the last block's threads, count in 32 bits
+  if (batch < 0 || batch > 0x7fffffffL || q_len < 0 || q_len > (1 << 30) || q_heads <= 0 || q_heads > (1 << 30) ||
+      head_dim <= 0 || head_dim > kEmptyThreads || row_bytes % 16 || q_len * q_heads > (int64_t)0xffff0000 / per)
+    return fail(PJX_ERR_INVALID, "pjx_zero_empty_rows: sizes out of range, or rows that are no whole 16-byte chunks");
+  if (batch == 0 || q_len == 0) return PJX_OK;
+  if (!lse || !o || !dout || !o_rows || !dout_rows)
+    return fail(PJX_ERR_INVALID, "pjx_zero_empty_rows: pointers must be non-null");
+  if (((uintptr_t)o | (uintptr_t)dout | (uintptr_t)o_rows | (uintptr_t)dout_rows) % 16)
+    return fail(PJX_ERR_INVALID, "pjx_zero_empty_rows: tensors must start on 16 bytes");
+  const ZeroArgs a = {lse, {(const u32x4*)o, (const u32x4*)dout}, {(u32x4*)o_rows, (u32x4*)dout_rows},
+                      (int)batch, (int)q_len, (int)q_heads, (int)per};
+  const dim3 grid((unsigned)((q_len * q_heads * per + kEmptyThreads - 1) / kEmptyThreads),
+                  (unsigned)std::min<int64_t>(batch, 65535), 2);
+  launch_kernel<zero_empty_rows_kernel>(grid, dim3(kEmptyThreads), 0, (hipStream_t)stream, a);
+  return check_launch("pjx_zero_empty_rows");
 }

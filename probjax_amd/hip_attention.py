@@ -314,6 +314,21 @@ def empty_rows(lse, src, dst, *, grad: bool) -> None:
     native.check(rc)
 
 
+def zero_empty_rows(lse, o, dout):
+    """``pjx_zero_empty_rows``: copies of the output and dO ``[B, Lq, Hq, D]`` with
+    zeros in the rows without a valid key (``lse`` = +inf)."""
+    dev = _on_device(lse, o, dout)
+    B, Lq, Hq, D = o.shape
+    if dout.shape != o.shape or dout.dtype != o.dtype or tuple(lse.shape) != (B, Hq, Lq) or lse.dtype != torch.float32:
+        raise ValueError(f"incompatible shapes: output {tuple(o.shape)}, dO {tuple(dout.shape)}, lse {tuple(lse.shape)}")
+    lse, o, dout = lse.contiguous(), _aligned(o.contiguous()), _aligned(dout.contiguous())
+    o_rows, dout_rows = torch.empty_like(o), torch.empty_like(dout)
+    rc = native.load().pjx_zero_empty_rows(_dtype_code(o), _ptr(lse), _ptr(o), _ptr(dout), _ptr(o_rows),
+                                           _ptr(dout_rows), B, Lq, Hq, D, _stream(dev))
+    native.check(rc)
+    return o_rows, dout_rows
+
+
 def _ds_budget(dev) -> int:
     """Bytes of dS a backward call may keep in its workspace (the dS route):
     ``PJX_BWD_DS_MAX_BYTES`` if set, else 1/16 of the device's memory, at most

@@ -83,6 +83,10 @@ _SIGNATURES = {
         ctypes.c_int,
         [ctypes.c_int, ctypes.c_int, _P, _P, _P, _I64, _I64, _I64, _I64, _I64, _I64, _P],
     ),
+    "pjx_zero_empty_rows": (
+        ctypes.c_int,
+        [ctypes.c_int, _P, _P, _P, _P, _P, _I64, _I64, _I64, _I64, _P],
+    ),
     "pjx_decode_workspace_size": (ctypes.c_size_t, [_I64, _I64, _I64, _I64, _I64, _I64]),
     "pjx_splitkv_decode": (
         ctypes.c_int,

@@ -120,3 +120,23 @@ def test_empty_rows_keep_nonfinite_gradients(device, dtype, D, bias):
         assert torch.isfinite(want[i]).all() and torch.equal(got[i], want[i])
     assert not torch.isfinite(got[2][0, :, 0]).any() and not torch.isfinite(got[2][1, :, 1]).any()
     assert torch.equal(got[2][0, :, 1], want[2][0, :, 1])
+
+
+@pytest.mark.parametrize("dtype,B,L,H,D,shift", [
+    ("bf16", 2, 70, 3, 64, 0), ("f16", 1, 33, 1, 8, 0), ("f32", 2, 1, 5, 100, 0), ("f32", 3, 257, 2, 12, 0),
+    ("bf16", 1, 40, 2, 256, 1)])
+def test_zero_empty_rows(device, dtype, B, L, H, D, shift):
+    """A copy with zeros in the rows of +inf lse, bitwise; ``shift`` starts the
+    sources off 16 bytes."""
+    import torch
+    from probjax_amd import hip_attention as hip
+
+    tdt = {"bf16": torch.bfloat16, "f16": torch.float16, "f32": torch.float32}[dtype]
+    n = B * L * H * D
+    o, do = (to_dev(x, device, tdt)[shift:shift + n].view(B, L, H, D) for x in rng_normal(56, (n + 8,), (n + 8,)))
+    lse = torch.zeros((B, H, L), device=device)
+    for share in (0.0, 0.4, 1.0):
+        lse[torch.rand(lse.shape, device=device) < share] = float("inf")
+        empty = torch.isinf(lse).transpose(1, 2)[..., None]
+        o_rows, do_rows = hip.zero_empty_rows(lse, o, do)
+        assert torch.equal(o_rows, torch.where(empty, 0, o)) and torch.equal(do_rows, torch.where(empty, 0, do))
