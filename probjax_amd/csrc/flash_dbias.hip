@@ -71,10 +71,11 @@ __global__ __launch_bounds__(128 * QS, 2) void flash_dbias_kernel(DbiasArgs da) 
     voffq[j] = row_chunk(r, qstride, c, rdim);
     voffk[j] = row_chunk(r, kstride, c, rdim);
   }
-  // 64 rows from row0 of head `head` of a [B, L, heads, D] tensor (zeros past L)
-  auto load = [&](const void* t, int b, int L, int heads, int head, int row0, uint32_t stride, const uint32_t* voff,
-                  unsigned char* dst) {
-    const int n = min(64, L - row0);
+  // 64 rows from row0 of head `head` of a [B, L, heads, D] tensor; zeros from row `end` on: a key past a
+  // sequence's end has P = 0, and a non-finite V there would make P dP a NaN
+  auto load = [&](const void* t, int b, int L, int end, int heads, int head, int row0, uint32_t stride,
+                  const uint32_t* voff, unsigned char* dst) {
+    const int n = min(64, end - row0);
     const rsrc_t rs = make_rsrc((const unsigned char*)t + ((size_t)(b * L + (n > 0 ? row0 : 0)) * heads + head) * rdim * 2,
                                 n > 0 ? (uint32_t)(n - 1) * stride + rdim * 2 : 0u);
 #pragma unroll
@@ -107,13 +108,13 @@ __global__ __launch_bounds__(128 * QS, 2) void flash_dbias_kernel(DbiasArgs da) 
       if (!first) __syncthreads();  // the tiles of the head before are consumed
 #pragma unroll
       for (int i = 0; i < QT; ++i) {
-        load(a.q, b, a.Lq, a.Hq, h, qt0 + 64 * i, qstride, voffq, smem + i * TILE_B);
-        load(ba.dout, b, a.Lq, a.Hq, h, qt0 + 64 * i, qstride, voffq, smem + (QT + i) * TILE_B);
+        load(a.q, b, a.Lq, a.Lq, a.Hq, h, qt0 + 64 * i, qstride, voffq, smem + i * TILE_B);
+        load(ba.dout, b, a.Lq, a.Lq, a.Hq, h, qt0 + 64 * i, qstride, voffq, smem + (QT + i) * TILE_B);
       }
 #pragma unroll
       for (int i = 0; i < 2; ++i) {
-        load(a.k, b, a.Lk, a.Hkv, hkv, kt0 + 64 * i, kstride, voffk, smem + (2 * QT + i) * TILE_B);
-        load(a.v, b, a.Lk, a.Hkv, hkv, kt0 + 64 * i, kstride, voffk, smem + (2 * QT + 2 + i) * TILE_B);
+        load(a.k, b, a.Lk, kv_end, a.Hkv, hkv, kt0 + 64 * i, kstride, voffk, smem + (2 * QT + i) * TILE_B);
+        load(a.v, b, a.Lk, kv_end, a.Hkv, hkv, kt0 + 64 * i, kstride, voffk, smem + (2 * QT + 2 + i) * TILE_B);
       }
       if (first) {
 #pragma unroll

@@ -66,6 +66,33 @@ def test_folded_equals_summed(device, case):
     assert np.abs(a - b).max() <= 1e-5 * max(1.0, np.abs(b).max())
 
 
+@pytest.mark.parametrize("dtype,D,causal,lengths", [
+    ("bf16", 64, False, [130, 70]), ("f16", 128, False, [65, 129]), ("bf16", 64, True, [1, 200]), ("bf16", 128, True, [97, 31])])
+def test_nonfinite_padding(device, dtype, D, causal, lengths):
+    """K and V past a sequence's end may hold anything (a buffer from
+    ``torch.empty``): the folded gradient, which also adds the other sequences',
+    is bitwise that of finite padding."""
+    import torch
+    from probjax_amd import hip_attention as hip
+
+    tdt = torch.bfloat16 if dtype == "bf16" else torch.float16
+    B, L, H = len(lengths), 200, 2
+    q, k, v, do = (to_dev(x, device, tdt) for x in rng_normal(57, *[(B, L, H, D)] * 4))
+    bias = to_dev(rng_normal(58, (1, H, L, L), scale=0.5)[0], device, torch.float32)
+    kw = dict(sm_scale=1 / math.sqrt(D), causal=causal, bias=bias,
+              kv_lengths=torch.tensor(lengths, dtype=torch.int32, device=device))
+    o, lse = hip.flash_attention_fwd(q, k, v, return_lse=True, **kw)
+    want = hip.flash_attention_bwd(q, k, v, o, do, lse, bias_grad=True, fold_bias_grad=True, **kw)
+    for b, n in enumerate(lengths):
+        k[b, n:], v[b, n:] = float("nan"), float("inf")
+        v[b, n::2] = float("nan")
+    got = hip.flash_attention_bwd(q, k, v, o, do, lse, bias_grad=True, fold_bias_grad=True, **kw)
+    assert torch.isfinite(want[3]).all() and torch.equal(got[3], want[3])
+    assert torch.equal(got[0], want[0])
+    for b, n in enumerate(lengths):
+        assert torch.equal(got[1][b, :n], want[1][b, :n]) and torch.equal(got[2][b, :n], want[2][b, :n])
+
+
 @pytest.mark.parametrize("dtype,B,Lq,Lk,Hq,Hkv,D", [
     ("bf16", 2, 70, 33, 4, 2, 64), ("f32", 1, 1, 257, 3, 3, 96), ("f16", 2, 300, 5, 8, 1, 256), ("f32", 2, 9, 1, 2, 1, 3)])
 def test_empty_rows(device, dtype, B, Lq, Lk, Hq, Hkv, D):
