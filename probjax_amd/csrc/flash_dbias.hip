@@ -148,7 +148,7 @@ __global__ __launch_bounds__(128 * QS, 2) void flash_dbias_kernel(DbiasArgs da) 
         if constexpr (EXT) {
           const HeadMods hm = head_mods(a.m, h);
           ext_scores_S<false>(a, b, hm, key, qlo[kb], qhi[kb], segk[kb], s, q0, half, nullptr,
-                              [&](int r, float x, float) { s[r] = x + bv[kb][r]; });
+                              [&](int r, float x, float) { s[r] = x == -INFINITY ? x : x + bv[kb][r]; });
         } else {
           const bool mask = (a.causal && q0 < kw + 31) || kw + 32 > kv_end || q0 + 32 > q_hi;
 #pragma unroll
@@ -166,7 +166,9 @@ __global__ __launch_bounds__(128 * QS, 2) void flash_dbias_kernel(DbiasArgs da) 
           for (int j = 0; j < 4; ++j) {
             const int r = 4 * gq + j;
             const float p = fast_exp2(fmaf(s[r], kLog2e, -l4[j]));
-            acc[kb][r] = fmaf(p, dp[r] - d4[j], acc[kb][r]);
+            // a dropped score adds nothing, also where its key's V (of another
+            // document, outside the window, after the query) or its row's dO is not finite
+            acc[kb][r] = fmaf(p, s[r] == -INFINITY ? 0.f : dp[r] - d4[j], acc[kb][r]);
           }
         }
       }

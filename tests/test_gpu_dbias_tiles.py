@@ -93,6 +93,46 @@ def test_nonfinite_padding(device, dtype, D, causal, lengths):
         assert torch.equal(got[1][b, :n], want[1][b, :n]) and torch.equal(got[2][b, :n], want[2][b, :n])
 
 
+@pytest.mark.parametrize("mask", ["causal", "window", "segments", "slopes"])
+@pytest.mark.parametrize("D", [64, 128])
+def test_nonfinite_at_masked_scores(device, D, mask):
+    """What the mask drops has gradient 0 and changes no other, bitwise: an
+    infinite or NaN bias there, and V of keys that the rows of a tile do not see."""
+    import torch
+    from probjax_amd import hip_attention as hip
+
+    B, L, H = 2, 150, 2
+    q, k, v, do = (to_dev(x, device, torch.bfloat16) for x in rng_normal(59, *[(B, L, H, D)] * 4))
+    bias = to_dev(rng_normal(60, (1, H, L, L), scale=0.5)[0], device, torch.float32)
+    i, j = torch.arange(L, device=device)[:, None], torch.arange(L, device=device)[None, :]
+    keep, mods = j <= i, None
+    if mask == "window":
+        keep, mods = keep & (j >= i - 20), hip.ScoreModsArgs(window_left=20)
+    elif mask == "segments":
+        ids = (j[0] >= 77).to(torch.int32)
+        keep, mods = keep & (ids[:, None] == ids[None, :]), hip.ScoreModsArgs(
+            segment_q=ids.repeat(B, 1), segment_k=ids.repeat(B, 1))
+    elif mask == "slopes":
+        mods = hip.ScoreModsArgs(alibi_slopes=torch.full((H,), 0.25, device=device))
+    kw = dict(sm_scale=1 / math.sqrt(D), causal=True, mods=mods, bias_grad=True, fold_bias_grad=True)
+
+    def grads(bias):
+        o, lse = hip.flash_attention_fwd(q, k, v, return_lse=True, sm_scale=kw["sm_scale"], causal=True, mods=mods,
+                                         bias=bias)
+        return o, lse, hip.flash_attention_bwd(q, k, v, o, do, lse, bias=bias, **kw)
+
+    o, lse, want = grads(bias)
+    assert torch.isfinite(want[3]).all() and not want[3][:, :, ~keep].any()
+    for x in ("inf", "nan"):
+        got = grads(bias.masked_fill(~keep, float(x)))[2]
+        for a, b in zip(got, want):
+            assert torch.equal(a, b)
+    # the last key's V, seen by the last row alone
+    v[:, L - 1] = float("nan")
+    got = hip.flash_attention_bwd(q, k, v, o, do, lse, bias=bias, **kw)
+    assert torch.equal(got[3][:, :, :-1], want[3][:, :, :-1])
+
+
 @pytest.mark.parametrize("dtype,B,Lq,Lk,Hq,Hkv,D", [
     ("bf16", 2, 70, 33, 4, 2, 64), ("f32", 1, 1, 257, 3, 3, 96), ("f16", 2, 300, 5, 8, 1, 256), ("f32", 2, 9, 1, 2, 1, 3)])
 def test_empty_rows(device, dtype, B, Lq, Lk, Hq, Hkv, D):
