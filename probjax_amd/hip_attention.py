@@ -49,6 +49,13 @@ def rows_width(head_dim: int, heads: int):
     return 64 if head_dim <= 64 else 128
 
 
+def bias_grad_folds(dtype, q_heads: int, kv_heads: int, head_dim: int, row_dim: int) -> bool:
+    """Whether ``pjx_flash_dbias`` takes a call's sizes: 16-bit rows at kernel
+    head dims 64 and 128, with the rows of all heads short enough for its tiles'
+    32-bit offsets (``pjx_flash_bwd`` takes more heads)."""
+    return dtype in HALF_DTYPES and head_dim <= 128 and max(q_heads, kv_heads) <= (1 << 22) // row_dim
+
+
 def _aligned(t):
     """``t`` (contiguous), copied if it does not start on 16 bytes."""
     return t if t.data_ptr() % 16 == 0 else t.clone()
@@ -217,8 +224,8 @@ def flash_attention_bwd(
     does not exist); False never does.
 
     ``fold_bias_grad`` (with ``bias_grad``): ``dbias`` from ``pjx_flash_dbias``,
-    summed over what the bias broadcasts to as it is computed (16-bit, head dim
-    64 or 128; elsewhere as without).
+    summed over what the bias broadcasts to as it is computed, where
+    ``bias_grad_folds``; elsewhere as without.
     """
     dev = _on_device(q, k, v, o, do, lse, bias)
     if q.ndim != 4 or k.ndim != 4 or v.ndim != 4:
@@ -256,7 +263,7 @@ def flash_attention_bwd(
     if bias_grad and bias is None:
         raise ValueError("bias_grad needs the bias")
     dq, dk, dv = torch.empty_like(q), torch.empty_like(k), torch.empty_like(v)
-    fold = bias_grad and fold_bias_grad and KD <= 128 and code != native.PJX_DTYPE_F32 and min(B, Lq, Lk) > 0
+    fold = bias_grad and fold_bias_grad and min(B, Lq, Lk) > 0 and bias_grad_folds(q.dtype, Hq, Hkv, KD, D)
     dbias = torch.zeros((B, Hq, Lq, Lk), dtype=torch.float32, device=dev) if bias_grad and not fold else None
     lib = native.load()
     nbytes = int(lib.pjx_flash_bwd_workspace_size(B, Hq, Lq))

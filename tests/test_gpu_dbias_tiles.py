@@ -133,6 +133,23 @@ def test_nonfinite_at_masked_scores(device, D, mask):
     assert torch.equal(got[3][:, :, :-1], want[3][:, :, :-1])
 
 
+def test_more_heads_than_the_tiles_address(device):
+    """Heads whose rows exceed the folded kernel's offsets take the dQ kernel's
+    gradient, as ``pjx_flash_bwd`` does for them."""
+    import torch
+    from probjax_amd import hip_attention as hip
+
+    H, D, L = (1 << 22) // 128 + 1, 128, 2
+    q, k, v, do = (to_dev(x, device, torch.bfloat16) for x in rng_normal(61, *[(1, L, H, D)] * 4))
+    bias = to_dev(rng_normal(62, (1, 1, L, L))[0], device, torch.float32)
+    kw = dict(sm_scale=1 / math.sqrt(D), bias=bias)
+    o, lse = hip.flash_attention_fwd(q, k, v, return_lse=True, **kw)
+    want = hip.flash_attention_bwd(q, k, v, o, do, lse, bias_grad=True, **kw)
+    got = hip.flash_attention_bwd(q, k, v, o, do, lse, bias_grad=True, fold_bias_grad=True, **kw)
+    for a, b in zip(got, want):
+        assert torch.equal(a, b)
+
+
 @pytest.mark.parametrize("dtype,B,Lq,Lk,Hq,Hkv,D", [
     ("bf16", 2, 70, 33, 4, 2, 64), ("f32", 1, 1, 257, 3, 3, 96), ("f16", 2, 300, 5, 8, 1, 256), ("f32", 2, 9, 1, 2, 1, 3)])
 def test_empty_rows(device, dtype, B, Lq, Lk, Hq, Hkv, D):
