@@ -49,11 +49,29 @@ def rows_width(head_dim: int, heads: int):
     return 64 if head_dim <= 64 else 128
 
 
-def bias_grad_folds(dtype, q_heads: int, kv_heads: int, head_dim: int, row_dim: int) -> bool:
-    """Whether ``pjx_flash_dbias`` takes a call's sizes: 16-bit rows at kernel
-    head dims 64 and 128, with the rows of all heads short enough for its tiles'
-    32-bit offsets (``pjx_flash_bwd`` takes more heads)."""
-    return dtype in HALF_DTYPES and head_dim <= 128 and max(q_heads, kv_heads) <= (1 << 22) // row_dim
+def bias_grad_folds(dtype, bias_shape, batch: int, q_heads: int, kv_heads: int, head_dim: int, row_dim: int) -> bool:
+    """Whether the gradient of a dense bias ``[bb, bh, Lq, Lk]`` takes
+    ``pjx_flash_dbias`` rather than one copy per (batch, head), summed.
+
+    It takes 16-bit rows at kernel head dims 64 and 128, with the rows of all
+    heads short enough for its tiles' 32-bit offsets (``pjx_flash_bwd`` takes
+    more heads).  A workgroup owns a tile of one bias slice, 64 x 128 scores at
+    head dim 64 and 128 x 128 at 128, and walks the (batch, head) pairs of the
+    slice one after the other, about 2.3 and 4 us each; the copies fill the
+    device at any size but cost 16 bytes a score.  So it needs half a device of
+    workgroups, or few enough pairs that the copies' extra launches cost as much.
+    Backward on the device, us, folded / summed (B, Hq, L, D, bias heads; workgroups, pairs):
+      (64,16,128,64,1; 2, 1024) 2256 / 145    (8,8,512,64,1; 32, 64) 197 / 96
+      (8,8,768,64,1; 72, 64)     254 / 182    (8,8,1024,64,1; 128, 64) 288 / 302
+      (32,8,1024,64,1; 128, 256) 1044 / 1102  (8,8,1024,128,1; 64, 64) 446 / 409
+      (8,8,512,128,8; 128, 8)    117 / 120    (4,8,128,64,8; 16, 4)     40 / 34
+    """
+    if dtype not in HALF_DTYPES or head_dim > 128 or max(q_heads, kv_heads) > (1 << 22) // row_dim:
+        return False
+    bb, bh, l_q, l_k = bias_shape
+    workgroups = -(-l_q // head_dim) * -(-l_k // 128) * bb * bh
+    pairs = (batch // bb) * (q_heads // bh)
+    return pairs <= 4 or workgroups >= 128
 
 
 def _aligned(t):
@@ -263,7 +281,8 @@ def flash_attention_bwd(
     if bias_grad and bias is None:
         raise ValueError("bias_grad needs the bias")
     dq, dk, dv = torch.empty_like(q), torch.empty_like(k), torch.empty_like(v)
-    fold = bias_grad and fold_bias_grad and min(B, Lq, Lk) > 0 and bias_grad_folds(q.dtype, Hq, Hkv, KD, D)
+    fold = bias_grad and fold_bias_grad and min(B, Lq, Lk) > 0 and bias_grad_folds(
+        q.dtype, bias.shape, B, Hq, Hkv, KD, D)
     dbias = torch.zeros((B, Hq, Lq, Lk), dtype=torch.float32, device=dev) if bias_grad and not fold else None
     lib = native.load()
     nbytes = int(lib.pjx_flash_bwd_workspace_size(B, Hq, Lq))

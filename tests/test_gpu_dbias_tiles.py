@@ -150,6 +150,27 @@ def test_more_heads_than_the_tiles_address(device):
         assert torch.equal(a, b)
 
 
+@pytest.mark.parametrize("B,H,L,D,bh,folds", [
+    (16, 4, 64, 64, 1, False), (5, 1, 130, 128, 1, False), (4, 3, 100, 64, 3, True), (2, 8, 384, 64, 8, True),
+    (6, 4, 384, 128, 1, False), (5, 8, 500, 128, 8, True), (7, 3, 257, 64, 3, False)])
+def test_route_by_grid(device, B, H, L, D, bh, folds):
+    """Few tiles with many (batch, head) pairs each take the summed copies,
+    with the same gradient (the bound of the tests above)."""
+    import torch
+    from probjax_amd import hip_attention as hip
+    from probjax_amd import native
+
+    q, k, v, do = (to_dev(x, device, torch.bfloat16) for x in rng_normal(63, *[(B, L, H, D)] * 4))
+    bias = to_dev(rng_normal(64, (1, bh, L, L), scale=0.5)[0], device, torch.float32)
+    kw = dict(sm_scale=1 / math.sqrt(D), bias=bias, bias_grad=True)
+    o, lse = hip.flash_attention_fwd(q, k, v, return_lse=True, sm_scale=kw["sm_scale"], bias=bias)
+    want = hip.flash_attention_bwd(q, k, v, o, do, lse, **kw)
+    got = hip.flash_attention_bwd(q, k, v, o, do, lse, fold_bias_grad=True, **kw)
+    assert any(n.startswith("flash_dbias_kernel") for n in native.last_launches()) == folds
+    a, b = to_np(got[3]), to_np(want[3])
+    assert a.shape == b.shape and np.abs(a - b).max() <= 1e-5 * max(1.0, np.abs(b).max())
+
+
 @pytest.mark.parametrize("dtype,B,Lq,Lk,Hq,Hkv,D", [
     ("bf16", 2, 70, 33, 4, 2, 64), ("f32", 1, 1, 257, 3, 3, 96), ("f16", 2, 300, 5, 8, 1, 256), ("f32", 2, 9, 1, 2, 1, 3)])
 def test_empty_rows(device, dtype, B, Lq, Lk, Hq, Hkv, D):
