@@ -199,6 +199,41 @@ def test_empty_rows(device, dtype, B, Lq, Lk, Hq, Hkv, D):
         assert float((dgot.float() - dv).abs().max()) <= 4 * eps * max(float(dv.abs().max()), 1e-6)
 
 
+@pytest.mark.parametrize("dtype,B,Lq,Lk,Hq,Hkv,D,shift", [
+    ("bf16", 1, 520, 700, 6, 2, 128, 0), ("f16", 3, 65, 64, 2, 2, 72, 0), ("f32", 1, 257, 66, 1, 1, 20, 0),
+    ("bf16", 1, 1, 513, 8, 1, 256, 0), ("bf16", 2, 130, 70, 2, 1, 64, 1), ("f32", 1, 33, 129, 2, 2, 200, 1),
+    ("f16", 1, 1030, 5, 40, 1, 8, 0)])
+def test_empty_rows_split(device, dtype, B, Lq, Lk, Hq, Hkv, D, shift):
+    """The edges of the row chunks, column groups and blocks of 256 rows, and
+    tensors that start off 16 bytes (``shift``): sums against float64, to the
+    spacing of the format, rows with valid keys untouched."""
+    import torch
+    from probjax_amd import hip_attention as hip
+
+    tdt = {"bf16": torch.bfloat16, "f16": torch.float16, "f32": torch.float32}[dtype]
+    o, v, do, dv = (to_dev(x, device, tdt)[shift:shift + n].view(s) for x, n, s in (
+        (rng_normal(65 + i, (math.prod(s) + 8,))[0], math.prod(s), s)
+        for i, s in enumerate(((B, Lq, Hq, D), (B, Lk, Hkv, D), (B, Lq, Hq, D), (B, Lk, Hkv, D)))))
+    lse = torch.zeros((B, Hq, Lq), device=device)
+    for rows in ((Lq - 1,), range(0, Lq, 3), range(Lq)):
+        lse[:, :, list(rows)] = float("inf")
+        if Hq > 1:
+            lse[:, 0] = 0.0  # a head without such rows
+        empty = torch.isinf(lse).transpose(1, 2)[..., None]
+        mean = v.double().mean(1, keepdim=True).repeat_interleave(Hq // Hkv, 2)
+        got, dgot = o.clone(), dv.clone()
+        if shift:
+            got, dgot = (torch.cat((x.new_zeros(shift), x.flatten()))[shift:].view(x.shape) for x in (got, dgot))
+        hip.empty_rows(lse, v, got, grad=False)
+        hip.empty_rows(lse, do, dgot, grad=True)
+        assert torch.equal(torch.where(empty, 0, got), torch.where(empty, 0, o))
+        add = torch.where(empty, do, 0).double().sum(1).view(B, Hkv, Hq // Hkv, D).sum(2)[:, None] / Lk
+        # one rounding to the format, and float32 sums of up to 41200 terms of size sqrt of that
+        eps = {"bf16": 2.0 ** -8, "f16": 2.0 ** -11, "f32": 0.0}[dtype]
+        for x, want in ((got, torch.where(empty, mean, o.double())), (dgot, dv.double() + add)):
+            assert float((x.double() - want).abs().max()) <= (eps + 2.0 ** -20) * max(1.0, float(want.abs().max()))
+
+
 @pytest.mark.parametrize("dtype,D,bias", [("bf16", 64, True), ("f16", 96, False), ("f32", 64, True), ("bf16", 256, False)])
 def test_empty_rows_keep_nonfinite_gradients(device, dtype, D, bias):
     """An infinite or NaN dO in a row without a valid key reaches dV alone (the
