@@ -9,17 +9,20 @@
 // v_mfma_f32_32x32x16_bf16 of 32 cycles contract 16 indices where
 // v_mfma_f32_32x32x2f32 takes 8 of 64 cycles: 192 against 512 cycles.
 //
-// Range: h of a finite value above kPlaneMax would round to infinity, and an
-// infinite plane times another operand's zero plane is NaN.  Tiles with such a
-// value are flagged where they are split and take the float32 MFMAs from
-// memory instead, so infinities and the largest values give what they gave.
+// Range: where h*h overflows, h*m and m*h (2^-9 of it, of either sign) may
+// overflow to the other infinity, and an infinite plane times another operand's
+// zero plane is NaN; a float32 product gives its one infinity.  Up to kPlaneMax
+// no product of two operands, nor the sum of any row of them, overflows.  Tiles
+// with a larger value are flagged where they are split and take the float32
+// MFMAs from memory instead, so that infinities and large values give what they
+// give there.
 #pragma once
 
 #include "flash_common.h"
 
 namespace pjx {
 
-constexpr float kPlaneMax = 3.38e38f;  // below bf16's largest finite value (3.3895e38)
+constexpr float kPlaneMax = 0x1p60f;
 
 // Eight consecutive values as three bf16 operands.
 struct Planes {

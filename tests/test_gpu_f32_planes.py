@@ -121,3 +121,29 @@ def test_values_beyond_bf16_range(device, D, H):
     assert _rel(o3, want.detach()) <= REL
     assert _rel(dq.double() * 2.0 ** -60, wg[0]) <= REL
     assert _rel(dv, wg[2]) <= REL
+
+
+@pytest.mark.parametrize("D,H", [(64, 2), (64, 300), (128, 80)])
+def test_products_beyond_float32(device, D, H):
+    """Finite q and k whose product lies below float32's range drop that key,
+    forward and backward, as a score of -inf does."""
+    import torch
+    from probjax_amd.hip_attention import flash_attention_bwd, flash_attention_fwd
+
+    B, L = 1, 100
+    q, k, v, do = (to_dev(x, device, torch.float32) for x in rng_normal(93, *[(B, L, H, D)] * 4))
+    q[..., 3] = 1e22 * (1 + q[..., 3].abs())
+    k[..., 3] = 0
+    k[0, 40, :, 3] = -1e22 * (1 + k[0, 40, :, 4].abs())
+    kw = dict(sm_scale=1 / math.sqrt(D))
+    o, lse = flash_attention_fwd(q, k, v, return_lse=True, **kw)
+    grads = flash_attention_bwd(q, k, v, o, do, lse, **kw)
+    rest = [i for i in range(L) if i != 40]
+    x = [t.double().requires_grad_() for t in (q, k[:, rest], v[:, rest])]
+    want = _attend64(*x, kw["sm_scale"], False)
+    wg = torch.autograd.grad(want, x, do.double())
+    assert torch.isfinite(lse).all()
+    assert not grads[1][:, 40].any() and not grads[2][:, 40].any()
+    errs = [_rel(o, want.detach()), _rel(grads[0], wg[0])] + [_rel(g[:, rest], w) for g, w in zip(grads[1:], wg[1:])]
+    print(f"  rel {errs}", flush=True)
+    assert max(errs) <= REL, errs
