@@ -51,7 +51,7 @@ __global__ __launch_bounds__(64 * RS * KG, WPE) void flash_fwd_f32_planes_kernel
   Planes qf[D / 16];
   bool q_wild;  // a value beyond the planes' range in the wave's rows
   {
-    float mx = 0.f;
+    bool beyond = false;
 #pragma unroll
     for (int s = 0; s < D / 16; ++s) {
       float x[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
@@ -59,10 +59,10 @@ __global__ __launch_bounds__(64 * RS * KG, WPE) void flash_fwd_f32_planes_kernel
         *(f32x4*)x = *(const f32x4*)(qrow + 16 * s + 8 * half);
         *(f32x4*)(x + 4) = *(const f32x4*)(qrow + 16 * s + 8 * half + 4);
       }
-      mx = abs_max8(x, mx);
+      beyond |= beyond_planes(x);
       qf[s] = planes8(x);
     }
-    q_wild = wave_any(mx > kPlaneMax);
+    q_wild = wave_any(beyond);
   }
   const float* brow = nullptr;
   if constexpr (BIAS)
@@ -108,13 +108,13 @@ __global__ __launch_bounds__(64 * RS * KG, WPE) void flash_fwd_f32_planes_kernel
   // flags[t % 2] == t + 1: stage t holds a value beyond the planes' range
   auto store = [&](int t) {
     unsigned char* st = smem + (NBUF == 2 ? (t & 1) * 2 * T::BYTES : 0);
-    float mx = 0.f;
+    bool beyond = false;
 #pragma unroll
     for (int i = 0; i < PER; ++i) {
-      mx = abs_max8(reg[i], mx);
+      beyond |= beyond_planes(reg[i]);
       T::store(st, loff[i], reg[i]);
     }
-    if (mx > kPlaneMax) flags[t & 1] = t + 1;
+    if (beyond) flags[t & 1] = t + 1;
   };
 
   auto compute = [&](int t) {

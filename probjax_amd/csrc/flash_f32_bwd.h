@@ -60,7 +60,7 @@ __global__ __launch_bounds__(64 * RS * KG, WPE) void flash_bwd_dq_f32_planes_ker
   bool q_wild;
   {
     const float* orow = (const float*)a.o + roff;
-    float mx = 0.f;
+    bool beyond = false;
 #pragma unroll
     for (int s = 0; s < D / 16; ++s) {
       float x[8] = {}, y[8] = {}, z[8] = {};
@@ -72,13 +72,13 @@ __global__ __launch_bounds__(64 * RS * KG, WPE) void flash_bwd_dq_f32_planes_ker
           *(f32x4*)(z + j) = *(const f32x4*)(orow + 16 * s + 8 * half + j);
         }
       }
-      mx = abs_max8(y, abs_max8(x, mx));
+      beyond |= beyond_planes(x) || beyond_planes(y);
 #pragma unroll
       for (int j = 0; j < 8; ++j) dsum = fmaf(z[j], y[j], dsum);
       qf[s] = planes8(x);
       df[s] = planes8(y);
     }
-    q_wild = wave_any(mx > kPlaneMax);
+    q_wild = wave_any(beyond);
   }
   const float delta = xor32_sum(dsum);
   const float dsc = delta * a.scale;  // the workspace holds delta * sm_scale
@@ -131,13 +131,13 @@ __global__ __launch_bounds__(64 * RS * KG, WPE) void flash_bwd_dq_f32_planes_ker
   };
   auto store = [&](int t) {
     unsigned char* st = smem + (NBUF == 2 ? (t & 1) * 2 * T::BYTES : 0);
-    float mx = 0.f;
+    bool beyond = false;
 #pragma unroll
     for (int i = 0; i < PER; ++i) {
-      mx = abs_max8(reg[i], mx);
+      beyond |= beyond_planes(reg[i]);
       T::store(st, loff[i], reg[i]);
     }
-    if (mx > kPlaneMax) flags[t & 1] = t + 1;
+    if (beyond) flags[t & 1] = t + 1;
   };
 
   auto compute = [&](int t) {
@@ -388,7 +388,7 @@ __global__ __launch_bounds__(64 * KS * QG, WPE) void flash_bwd_dkdv_f32_planes_k
   Planes vf[VR ? D / 16 : 1];
   bool k_wild;
   {
-    float mx = 0.f;
+    bool beyond = false;
 #pragma unroll
     for (int s = 0; s < D / 16; ++s) {
       float x[8] = {}, y[8] = {};
@@ -399,14 +399,14 @@ __global__ __launch_bounds__(64 * KS * QG, WPE) void flash_bwd_dkdv_f32_planes_k
           *(f32x4*)(y + j) = *(const f32x4*)(vrow + 16 * s + 8 * half + j);
         }
       }
-      mx = abs_max8(y, abs_max8(x, mx));
+      beyond |= beyond_planes(x) || beyond_planes(y);
       if (gi == 0) {
         TK::store(kv, 32 * strip * TK::ROWB + off.row[s], x);
         if (!VR) TK::store(kv + TK::BYTES, 32 * strip * TK::ROWB + off.row[s], y);
       }
       if (VR) vf[s] = planes8(y);
     }
-    k_wild = wave_any(mx > kPlaneMax);
+    k_wild = wave_any(beyond);
   }
   auto kfrag = [&](int st) { return TK::rows(kv, 32 * strip, off.row[st]); };
   auto vfrag = [&](int st) { return VR ? vf[VR ? st : 0] : TK::rows(kv + (VR ? 0 : TK::BYTES), 32 * strip, off.row[st]); };
@@ -452,13 +452,13 @@ __global__ __launch_bounds__(64 * KS * QG, WPE) void flash_bwd_dkdv_f32_planes_k
     }
   };
   auto store = [&](int t) {
-    float mx = 0.f;
+    bool beyond = false;
 #pragma unroll
     for (int i = 0; i < PER; ++i) {
-      mx = abs_max8(reg[i], mx);
+      beyond |= beyond_planes(reg[i]);
       T::store(smem, loff[i], reg[i]);
     }
-    if (mx > kPlaneMax) flags[t & 1] = t + 1;
+    if (beyond) flags[t & 1] = t + 1;
     if (tid < 2 * SQ) rows[tid] = rreg;
   };
 

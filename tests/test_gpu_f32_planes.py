@@ -147,3 +147,43 @@ def test_products_beyond_float32(device, D, H):
     errs = [_rel(o, want.detach()), _rel(grads[0], wg[0])] + [_rel(g[:, rest], w) for g, w in zip(grads[1:], wg[1:])]
     print(f"  rel {errs}", flush=True)
     assert max(errs) <= REL, errs
+
+
+@pytest.mark.parametrize("D,H", [(64, 2), (64, 300), (128, 80)])
+@pytest.mark.parametrize("which", ["v", "do", "k", "row"])
+def test_small_values(device, D, H, which):
+    """Operands so small that a bf16 plane would lose bits (V, dO, K against a
+    larger scale, some rows of K and V among ordinary ones): as accurate as any."""
+    import torch
+    from probjax_amd.hip_attention import flash_attention_bwd, flash_attention_fwd
+
+    B, L, scale = 1, 100, 1 / math.sqrt(D)
+    for e in (-101, -112, -118):
+        q, k, v, do = (to_dev(x, device, torch.float32) for x in rng_normal(94, *[(B, L, H, D)] * 4))
+        sm_scale = scale
+        if which == "v":
+            v *= 2.0 ** e
+        elif which == "do":
+            do *= 2.0 ** e
+        elif which == "k":
+            k *= 2.0 ** e
+            q *= 2.0 ** 50
+            sm_scale *= 2.0 ** (-e - 50)
+        else:
+            # these rows alone make the last feature block of the output
+            v[:, 40:44, :, 32:] *= 2.0 ** e
+            v[:, :40, :, 32:] = v[:, 44:, :, 32:] = 0
+            k[:, 40:44] *= 2.0 ** e
+        kw = dict(sm_scale=sm_scale)
+        o, lse = flash_attention_fwd(q, k, v, return_lse=True, **kw)
+        grads = flash_attention_bwd(q, k, v, o, do, lse, **kw)
+        x = [t.double().requires_grad_() for t in (q, k, v)]
+        want = _attend64(*x, sm_scale, False)
+        wg = torch.autograd.grad(want, x, do.double())
+        errs = [_rel(o, want.detach())] + [_rel(g, w) for g, w in zip(grads, wg)]
+        if which == "row":
+            errs.append(_rel(o[..., 32:], want.detach()[..., 32:]))
+        print(f"  2^{e} rel {errs}", flush=True)
+        # dS of a small V or dO is small itself: its products have a test of their own
+        checked = {"v": (0, 3), "do": (0, 3)}.get(which, range(len(errs)))
+        assert max(errs[i] for i in checked) <= REL, errs
