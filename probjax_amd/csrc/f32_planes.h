@@ -24,6 +24,10 @@
 
 #include "flash_common.h"
 
+// A stage's loads and stores share registers: called out of line they would go
+// through scratch memory (forward of (1, 4, 512, 64) 16.9 -> 31.4 us).
+#define PJX_INLINE_LAMBDA __attribute__((always_inline))
+
 namespace pjx {
 
 constexpr float kPlaneMax = 0x1p60f, kPlaneMin = 0x1p-100f;
@@ -68,13 +72,24 @@ __device__ __forceinline__ Planes planes_step(const f32x16& x, int c) {
   return planes8(v);
 }
 
-// Whether 8 consecutive values are beyond the planes' range.
-__device__ __forceinline__ bool beyond_planes(const float* x) {
-  float m = 0.f;
+// The range of the chunks of 8 consecutive values seen so far: the largest
+// chunk's and the smallest non-zero one's largest magnitude, as bits (`lo` less
+// one, so that a chunk of zeros is none): three operations a chunk, compared
+// once a stage.
+struct PlaneSpan {
+  uint32_t hi = 0u, lo = ~0u;
+  __device__ __forceinline__ void add(const float* x) {
+    float m = 0.f;
 #pragma unroll
-  for (int j = 0; j < 8; ++j) m = fmaxf(m, fabsf(x[j]));
-  return m > kPlaneMax || (m > 0.f && m < kPlaneMin);
-}
+    for (int j = 0; j < 8; ++j) m = fmaxf(m, fabsf(x[j]));
+    hi = max(hi, __float_as_uint(m));
+    lo = min(lo, __float_as_uint(m) - 1u);
+  }
+  // beyond the planes' range
+  __device__ __forceinline__ bool beyond_planes() const {
+    return (hi > __float_as_uint(kPlaneMax)) | (lo < __float_as_uint(kPlaneMin) - 1u);
+  }
+};
 
 // c += a b over 16 indices, smallest terms first.
 __device__ __forceinline__ f32x16 mma_planes(const Planes& a, const Planes& b, f32x16 c) {

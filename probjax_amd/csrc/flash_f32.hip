@@ -51,7 +51,7 @@ __global__ __launch_bounds__(64 * RS * KG, WPE) void flash_fwd_f32_planes_kernel
   Planes qf[D / 16];
   bool q_wild;  // a value beyond the planes' range in the wave's rows
   {
-    bool beyond = false;
+    PlaneSpan span;
 #pragma unroll
     for (int s = 0; s < D / 16; ++s) {
       float x[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
@@ -59,10 +59,10 @@ __global__ __launch_bounds__(64 * RS * KG, WPE) void flash_fwd_f32_planes_kernel
         *(f32x4*)x = *(const f32x4*)(qrow + 16 * s + 8 * half);
         *(f32x4*)(x + 4) = *(const f32x4*)(qrow + 16 * s + 8 * half + 4);
       }
-      beyond |= beyond_planes(x);
+      span.add(x);
       qf[s] = planes8(x);
     }
-    q_wild = wave_any(beyond);
+    q_wild = wave_any(span.beyond_planes());
   }
   const float* brow = nullptr;
   if constexpr (BIAS)
@@ -95,7 +95,7 @@ __global__ __launch_bounds__(64 * RS * KG, WPE) void flash_fwd_f32_planes_kernel
   // chunk i is V's (PER == 1: the second half of the waves')
   auto is_v = [&](int i) { return PER == 1 ? w8 >= RS * KG / 2 : i >= PER / 2; };
   float reg[PER][8];
-  auto load = [&](int t) {
+  auto load = [&](int t) PJX_INLINE_LAMBDA {
     const int k0 = g.kv_begin + t * SK;
 #pragma unroll
     for (int i = 0; i < PER; ++i) {
@@ -106,18 +106,18 @@ __global__ __launch_bounds__(64 * RS * KG, WPE) void flash_fwd_f32_planes_kernel
     }
   };
   // flags[t % 2] == t + 1: stage t holds a value beyond the planes' range
-  auto store = [&](int t) {
+  auto store = [&](int t) PJX_INLINE_LAMBDA {
     unsigned char* st = smem + (NBUF == 2 ? (t & 1) * 2 * T::BYTES : 0);
-    bool beyond = false;
+    PlaneSpan span;
 #pragma unroll
     for (int i = 0; i < PER; ++i) {
-      beyond |= beyond_planes(reg[i]);
+      span.add(reg[i]);
       T::store(st, loff[i], reg[i]);
     }
-    if (beyond) flags[t & 1] = t + 1;
+    if (span.beyond_planes()) flags[t & 1] = t + 1;
   };
 
-  auto compute = [&](int t) {
+  auto compute = [&](int t) PJX_INLINE_LAMBDA {
     const int k0 = g.kv_begin + t * SK + 32 * gi;
     if constexpr (EXT > 0) {
       if (!er.any || k0 > er.hi_last || k0 + 31 < er.lo_first) return;

@@ -60,7 +60,7 @@ __global__ __launch_bounds__(64 * RS * KG, WPE) void flash_bwd_dq_f32_planes_ker
   bool q_wild;
   {
     const float* orow = (const float*)a.o + roff;
-    bool beyond = false;
+    PlaneSpan span;
 #pragma unroll
     for (int s = 0; s < D / 16; ++s) {
       float x[8] = {}, y[8] = {}, z[8] = {};
@@ -72,13 +72,14 @@ __global__ __launch_bounds__(64 * RS * KG, WPE) void flash_bwd_dq_f32_planes_ker
           *(f32x4*)(z + j) = *(const f32x4*)(orow + 16 * s + 8 * half + j);
         }
       }
-      beyond |= beyond_planes(x) || beyond_planes(y);
+      span.add(x);
+      span.add(y);
 #pragma unroll
       for (int j = 0; j < 8; ++j) dsum = fmaf(z[j], y[j], dsum);
       qf[s] = planes8(x);
       df[s] = planes8(y);
     }
-    q_wild = wave_any(beyond);
+    q_wild = wave_any(span.beyond_planes());
   }
   const float delta = xor32_sum(dsum);
   const float dsc = delta * a.scale;  // the workspace holds delta * sm_scale
@@ -119,7 +120,7 @@ __global__ __launch_bounds__(64 * RS * KG, WPE) void flash_bwd_dq_f32_planes_ker
 
   auto is_v = [&](int i) { return PER == 1 ? w8 >= RS * KG / 2 : i >= PER / 2; };
   float reg[PER][8];
-  auto load = [&](int t) {
+  auto load = [&](int t) PJX_INLINE_LAMBDA {
     const int k0 = g.kv_begin + t * SK;
 #pragma unroll
     for (int i = 0; i < PER; ++i) {
@@ -129,18 +130,18 @@ __global__ __launch_bounds__(64 * RS * KG, WPE) void flash_bwd_dq_f32_planes_ker
       *(f32x4*)(reg[i] + 4) = buffer_load_f32x4(r, goff + 16);
     }
   };
-  auto store = [&](int t) {
+  auto store = [&](int t) PJX_INLINE_LAMBDA {
     unsigned char* st = smem + (NBUF == 2 ? (t & 1) * 2 * T::BYTES : 0);
-    bool beyond = false;
+    PlaneSpan span;
 #pragma unroll
     for (int i = 0; i < PER; ++i) {
-      beyond |= beyond_planes(reg[i]);
+      span.add(reg[i]);
       T::store(st, loff[i], reg[i]);
     }
-    if (beyond) flags[t & 1] = t + 1;
+    if (span.beyond_planes()) flags[t & 1] = t + 1;
   };
 
-  auto compute = [&](int t) {
+  auto compute = [&](int t) PJX_INLINE_LAMBDA {
     const int k0 = g.kv_begin + t * SK + 32 * gi;
     if constexpr (EXT > 0) {
       if (!er.any || k0 > er.hi_last || k0 + 31 < er.lo_first) return;
@@ -388,7 +389,7 @@ __global__ __launch_bounds__(64 * KS * QG, WPE) void flash_bwd_dkdv_f32_planes_k
   Planes vf[VR ? D / 16 : 1];
   bool k_wild;
   {
-    bool beyond = false;
+    PlaneSpan span;
 #pragma unroll
     for (int s = 0; s < D / 16; ++s) {
       float x[8] = {}, y[8] = {};
@@ -399,14 +400,15 @@ __global__ __launch_bounds__(64 * KS * QG, WPE) void flash_bwd_dkdv_f32_planes_k
           *(f32x4*)(y + j) = *(const f32x4*)(vrow + 16 * s + 8 * half + j);
         }
       }
-      beyond |= beyond_planes(x) || beyond_planes(y);
+      span.add(x);
+      span.add(y);
       if (gi == 0) {
         TK::store(kv, 32 * strip * TK::ROWB + off.row[s], x);
         if (!VR) TK::store(kv + TK::BYTES, 32 * strip * TK::ROWB + off.row[s], y);
       }
       if (VR) vf[s] = planes8(y);
     }
-    k_wild = wave_any(beyond);
+    k_wild = wave_any(span.beyond_planes());
   }
   auto kfrag = [&](int st) { return TK::rows(kv, 32 * strip, off.row[st]); };
   auto vfrag = [&](int st) { return VR ? vf[VR ? st : 0] : TK::rows(kv + (VR ? 0 : TK::BYTES), 32 * strip, off.row[st]); };
@@ -434,7 +436,7 @@ __global__ __launch_bounds__(64 * KS * QG, WPE) void flash_bwd_dkdv_f32_planes_k
   auto stage_q0 = [&](int t) { return q_begin + (n_qt - 1 - t / G) * SQ; };
   auto is_d = [&](int i) { return PER == 1 ? w8 >= KS * QG / 2 : i >= PER / 2; };
   float reg[PER][8], rreg = 0.f;
-  auto load = [&](int t) {
+  auto load = [&](int t) PJX_INLINE_LAMBDA {
     const int h = stage_head(t), q0 = stage_q0(t);
     const size_t ro = ((size_t)b * a.Lq * a.Hq + h) * rdim * 4;
 #pragma unroll
@@ -451,18 +453,18 @@ __global__ __launch_bounds__(64 * KS * QG, WPE) void flash_bwd_dkdv_f32_planes_k
       if (qq < a.Lq) rreg = tid < SQ ? ba.lse2[li] : ba.delta[li];
     }
   };
-  auto store = [&](int t) {
-    bool beyond = false;
+  auto store = [&](int t) PJX_INLINE_LAMBDA {
+    PlaneSpan span;
 #pragma unroll
     for (int i = 0; i < PER; ++i) {
-      beyond |= beyond_planes(reg[i]);
+      span.add(reg[i]);
       T::store(smem, loff[i], reg[i]);
     }
-    if (beyond) flags[t & 1] = t + 1;
+    if (span.beyond_planes()) flags[t & 1] = t + 1;
     if (tid < 2 * SQ) rows[tid] = rreg;
   };
 
-  auto compute = [&](int t) {
+  auto compute = [&](int t) PJX_INLINE_LAMBDA {
     const int h = stage_head(t), q0 = stage_q0(t) + 32 * gi;
     if (q0 >= q_hi || kw >= kv_end) return;
     if constexpr (EXT > 0) {
