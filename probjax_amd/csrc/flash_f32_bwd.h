@@ -37,7 +37,7 @@ __global__ __launch_bounds__(64 * RS * KG, WPE) void flash_bwd_dq_f32_planes_ker
   static_assert(PER >= 1 && 2 * NCH % NT == 0 && (PER == 1 || PER % 2 == 0), "stage shape");
   static_assert((KG - 1) * RS * 64 * (D / 2) * 4 <= NBUF * 2 * T::BYTES, "the sum fits the stages");
   __shared__ __attribute__((aligned(1024))) unsigned char smem[NBUF * 2 * T::BYTES];
-  __shared__ int flags[2];
+  __shared__ int flags[4];  // [t % 2], [2 + t % 2] == t + 1: stage t is beyond_sure, beyond_planes
 
   const int tid = threadIdx.x, lane = tid & 63;
   const int w8 = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -57,7 +57,7 @@ __global__ __launch_bounds__(64 * RS * KG, WPE) void flash_bwd_dq_f32_planes_ker
   const float* drow = (const float*)ba.dout + roff;
   Planes qf[D / 16], df[D / 16];
   float dsum = 0.f;
-  bool q_wild;
+  bool q_wild, q_sure;
   {
     const float* orow = (const float*)a.o + roff;
     PlaneSpan span;
@@ -80,9 +80,11 @@ __global__ __launch_bounds__(64 * RS * KG, WPE) void flash_bwd_dq_f32_planes_ker
       df[s] = planes8(y);
     }
     q_wild = wave_any(span.beyond_planes());
+    q_sure = !wave_any(span.beyond_sure());
   }
   const float delta = xor32_sum(dsum);
   const float dsc = delta * a.scale;  // the workspace holds delta * sm_scale
+  q_sure = q_sure && !wave_any(!(fabsf(dsc) < kSureScoreGrad));
   float lse2 = 0.f;
   const size_t lidx = ((size_t)g.b * a.Hq + g.h) * a.Lq + g.qi;
   if (row_in) {
@@ -101,6 +103,8 @@ __global__ __launch_bounds__(64 * RS * KG, WPE) void flash_bwd_dq_f32_planes_ker
   ExtRows er;
   if constexpr (EXT > 0) er = ext_rows(a, g);
   if constexpr (EXT == 2) ext_segments(a, g, er, 32, (int*)smem, BQ);
+  const float wscale = EXT == 3 ? a.scale * er.hm.hscale : a.scale;  // bounds d(score) of the modifiers
+  q_sure = q_sure && !scale_beyond_sure(wscale);
 
   PlaneOffsets<D> off;
   off.init(lane);
@@ -138,7 +142,10 @@ __global__ __launch_bounds__(64 * RS * KG, WPE) void flash_bwd_dq_f32_planes_ker
       span.add(reg[i]);
       T::store(st, loff[i], reg[i]);
     }
-    if (span.beyond_planes()) flags[t & 1] = t + 1;
+    if (span.beyond_sure()) {
+      flags[t & 1] = t + 1;
+      if (span.beyond_planes()) flags[2 + (t & 1)] = t + 1;
+    }
   };
 
   auto compute = [&](int t) PJX_INLINE_LAMBDA {
@@ -161,7 +168,8 @@ __global__ __launch_bounds__(64 * RS * KG, WPE) void flash_bwd_dq_f32_planes_ker
     }
     const unsigned char* kt = smem + (NBUF == 2 ? (t & 1) * 2 * T::BYTES : 0);
     const unsigned char* vt = kt + T::BYTES;
-    const bool wild = q_wild || __builtin_amdgcn_readfirstlane(flags[t & 1]) == t + 1;
+    const bool sure = q_sure && __builtin_amdgcn_readfirstlane(flags[t & 1]) != t + 1;
+    const bool wild = !sure && (q_wild || __builtin_amdgcn_readfirstlane(flags[2 + (t & 1)]) == t + 1);
 
     // register r holds key k0 + 8*(r/4) + 4*half + r%4 of query `col`
     f32x16 s[1] = {f32x16{}}, dp[1] = {f32x16{}};
@@ -184,6 +192,8 @@ __global__ __launch_bounds__(64 * RS * KG, WPE) void flash_bwd_dq_f32_planes_ker
         dp[0] = mfma32x32x2f32(in && kin ? vp[i] : 0.f, in && row_in ? dop[i] : 0.f, dp[0]);
       }
     }
+    bool ds_wild = wild;
+    if (!sure && !wild) ds_wild = score_grads_beyond_planes(dp[0], wscale, [&](int) { return delta; });
     f32x16 dbv[1];
     if constexpr (EXT == 3) {
       ext_scores_sT<1, HB>(a, g, er, s, k0, half, brow, row_in, [&](int kb, int r, float x, float gg) {
@@ -233,7 +243,7 @@ __global__ __launch_bounds__(64 * RS * KG, WPE) void flash_bwd_dq_f32_planes_ker
     }
     if constexpr (DB) store_dbias<1>(ba, g, dbv, k0, half, row_in);
     // dQ^T[d][query] += K^T dS^T
-    if (!wild) {
+    if (!ds_wild) {
 #pragma unroll
       for (int c = 0; c < 2; ++c) {
         const Planes p = planes_step(s[0], c);
@@ -255,7 +265,7 @@ __global__ __launch_bounds__(64 * RS * KG, WPE) void flash_bwd_dq_f32_planes_ker
     }
   };
 
-  if (tid < 2) flags[tid] = 0;
+  if (tid < 4) flags[tid] = 0;
   if (n_stages > 0) {
     load(0);
     __syncthreads();
@@ -329,7 +339,7 @@ __global__ __launch_bounds__(64 * KS * QG, WPE) void flash_bwd_dkdv_f32_planes_k
   __shared__ __attribute__((aligned(1024))) unsigned char smem[2 * T::BYTES];
   __shared__ __attribute__((aligned(1024))) unsigned char kv[(VR ? 1 : 2) * TK::BYTES];  // K, V planes
   __shared__ __attribute__((aligned(16))) float rows[2 * SQ];  // lse*log2e, delta*sm_scale
-  __shared__ int flags[2];
+  __shared__ int flags[4];  // [t % 2], [2 + t % 2] == t + 1: stage t is beyond_sure, beyond_planes
 
   const int tid = threadIdx.x, lane = tid & 63;
   const int w8 = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -387,7 +397,7 @@ __global__ __launch_bounds__(64 * KS * QG, WPE) void flash_bwd_dkdv_f32_planes_k
   PlaneOffsets<D> off;
   off.init(lane);
   Planes vf[VR ? D / 16 : 1];
-  bool k_wild;
+  bool k_wild, k_sure;
   {
     PlaneSpan span;
 #pragma unroll
@@ -409,6 +419,7 @@ __global__ __launch_bounds__(64 * KS * QG, WPE) void flash_bwd_dkdv_f32_planes_k
       if (VR) vf[s] = planes8(y);
     }
     k_wild = wave_any(span.beyond_planes());
+    k_sure = !wave_any(span.beyond_sure()) && !scale_beyond_sure(a.scale);
   }
   auto kfrag = [&](int st) { return TK::rows(kv, 32 * strip, off.row[st]); };
   auto vfrag = [&](int st) { return VR ? vf[VR ? st : 0] : TK::rows(kv + (VR ? 0 : TK::BYTES), 32 * strip, off.row[st]); };
@@ -460,7 +471,10 @@ __global__ __launch_bounds__(64 * KS * QG, WPE) void flash_bwd_dkdv_f32_planes_k
       span.add(reg[i]);
       T::store(smem, loff[i], reg[i]);
     }
-    if (span.beyond_planes()) flags[t & 1] = t + 1;
+    if (span.beyond_sure() | ((tid >= SQ) & !(fabsf(rreg) < kSureScoreGrad))) {
+      flags[t & 1] = t + 1;
+      if (span.beyond_planes()) flags[2 + (t & 1)] = t + 1;
+    }
     if (tid < 2 * SQ) rows[tid] = rreg;
   };
 
@@ -486,7 +500,13 @@ __global__ __launch_bounds__(64 * KS * QG, WPE) void flash_bwd_dkdv_f32_planes_k
     const unsigned char* dt = qt + T::BYTES;
     const float* lsm = rows + 32 * gi;
     const float* dlm = lsm + SQ;
-    const bool wild = k_wild || __builtin_amdgcn_readfirstlane(flags[t & 1]) == t + 1;
+    bool sure = k_sure && __builtin_amdgcn_readfirstlane(flags[t & 1]) != t + 1;
+    float hscale = 1.f;
+    if constexpr (EXT == 3) {
+      hscale = head_mods(a.m, h).hscale;
+      sure = sure && !scale_beyond_sure(a.scale * hscale);
+    }
+    const bool wild = !sure && (k_wild || __builtin_amdgcn_readfirstlane(flags[2 + (t & 1)]) == t + 1);
     const float* Qg = (const float*)a.q + ((size_t)b * a.Lq * a.Hq + h) * rdim;
     const float* Dg = (const float*)ba.dout + ((size_t)b * a.Lq * a.Hq + h) * rdim;
 
@@ -509,6 +529,9 @@ __global__ __launch_bounds__(64 * KS * QG, WPE) void flash_bwd_dkdv_f32_planes_k
         dp = mfma32x32x2f32(in && qin ? Dg[qo + i] : 0.f, in && kin ? vrow[half * (D / 2) + i] : 0.f, dp);
       }
     }
+    bool ds_wild = wild;
+    if (!sure && !wild)  // the rows hold delta * sm_scale
+      ds_wild = score_grads_beyond_planes(dp * a.scale, hscale, [&](int r) { return dlm[8 * (r >> 2) + 4 * half + (r & 3)]; });
     if constexpr (EXT == 3) {
       const float* bbase = nullptr;
       if constexpr (BIAS) bbase = a.bias + (size_t)b * a.bias_bstride + (size_t)h * a.bias_hstride;
@@ -566,6 +589,19 @@ __global__ __launch_bounds__(64 * KS * QG, WPE) void flash_bwd_dkdv_f32_planes_k
           accv[db] = mma_planes(T::cols(dt, 32 * gi + 16 * c, off.tlo[db], off.thi[db]), p, accv[db]);
         __builtin_amdgcn_sched_barrier(0);
       }
+    } else {
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        const int qq = q0 + 8 * (r >> 2) + 4 * half + (r & 3);
+        const bool qin = qq < a.Lq;
+        const size_t qo = (size_t)(qin ? qq : 0) * a.Hq * rdim + col;
+#pragma unroll
+        for (int db = 0; db < D / 32; ++db)
+          accv[db] = mfma32x32x2f32(qin && db * 32 + col < rdim ? Dg[qo + db * 32] : 0.f, s[r], accv[db]);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+    if (!ds_wild) {
 #pragma unroll
       for (int c = 0; c < 2; ++c) {
         const Planes p = planes_step(dp, c);
@@ -581,17 +617,14 @@ __global__ __launch_bounds__(64 * KS * QG, WPE) void flash_bwd_dkdv_f32_planes_k
         const bool qin = qq < a.Lq;
         const size_t qo = (size_t)(qin ? qq : 0) * a.Hq * rdim + col;
 #pragma unroll
-        for (int db = 0; db < D / 32; ++db) {
-          const bool in = qin && db * 32 + col < rdim;
-          accv[db] = mfma32x32x2f32(in ? Dg[qo + db * 32] : 0.f, s[r], accv[db]);
-          acck[db] = mfma32x32x2f32(in ? Qg[qo + db * 32] : 0.f, dp[r], acck[db]);
-        }
+        for (int db = 0; db < D / 32; ++db)
+          acck[db] = mfma32x32x2f32(qin && db * 32 + col < rdim ? Qg[qo + db * 32] : 0.f, dp[r], acck[db]);
         __builtin_amdgcn_sched_barrier(0);
       }
     }
   };
 
-  if (tid < 2) flags[tid] = 0;
+  if (tid < 4) flags[tid] = 0;
   if (n_stages > 0) {
     load(0);
     __syncthreads();

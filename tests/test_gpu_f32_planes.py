@@ -187,3 +187,62 @@ def test_small_values(device, D, H, which):
         # dS of a small V or dO is small itself: its products have a test of their own
         checked = {"v": (0, 3), "do": (0, 3)}.get(which, range(len(errs)))
         assert max(errs[i] for i in checked) <= REL, errs
+
+
+@pytest.mark.parametrize("D,H", [(64, 2), (64, 70), (64, 300), (128, 2), (128, 300)])
+@pytest.mark.parametrize("which", ["v", "do", "both"])
+def test_small_score_gradients(device, D, H, which):
+    """dS is as accurate where V, dO or their product alone make it small."""
+    import torch
+    from probjax_amd.hip_attention import flash_attention_bwd, flash_attention_fwd
+
+    B, L, kw = 1, 100, dict(sm_scale=1 / math.sqrt(D))
+    for e in (-95, -101, -112, -118):
+        q, k, v, do = (to_dev(x, device, torch.float32) for x in rng_normal(95, *[(B, L, H, D)] * 4))
+        a, b = {"v": (e, 0), "do": (0, e), "both": (e // 2, e - e // 2)}[which]
+        v *= 2.0 ** a
+        do *= 2.0 ** b
+        o, lse = flash_attention_fwd(q, k, v, return_lse=True, **kw)
+        grads = flash_attention_bwd(q, k, v, o, do, lse, **kw)
+        x = [t.double().requires_grad_() for t in (q, k, v)]
+        wg = torch.autograd.grad(_attend64(*x, kw["sm_scale"], False), x, do.double())
+        errs = [_rel(g, w) for g, w in zip(grads, wg)]
+        print(f"  2^{e} rel {errs}", flush=True)
+        assert max(errs) <= REL, errs
+
+
+@pytest.mark.parametrize("D,H", [(64, 2), (64, 70), (64, 300), (128, 2), (128, 300)])
+@pytest.mark.parametrize("bias", [False, True])
+def test_large_score_gradients(device, D, H, bias):
+    """A dS of ordinary operands' product that is itself huge: infinite where a
+    gradient lies beyond float32 (one term alone makes it), accurate elsewhere."""
+    import torch
+    from probjax_amd.hip_attention import flash_attention_bwd, flash_attention_fwd
+
+    B, L, kw = 1, 100, dict(sm_scale=1 / math.sqrt(D))
+    q, k, v, do = (to_dev(x, device, torch.float32) for x in rng_normal(96, *[(B, L, H, D)] * 4))
+    # features 3 and 5 are no part of any score
+    for t, i in ((q, 5), (k, 3)):
+        t[..., i] = 0
+        t[0, 41, :, i] = 2.0 ** 34
+    q[..., 3] = 0
+    k[..., 5] = 0
+    v *= 2.0 ** 56
+    do *= 2.0 ** 56
+    if bias:
+        kw["bias"] = torch.zeros(1, 1, L, L, device=device)
+    o, lse = flash_attention_fwd(q, k, v, return_lse=True, **kw)
+    grads = flash_attention_bwd(q, k, v, o, do, lse, bias_grad=bias, **kw)[:3]
+    x = [t.double().requires_grad_() for t in (q, k, v)]
+    wg = torch.autograd.grad(_attend64(*x, kw["sm_scale"], False), x, do.double())
+    big = torch.finfo(torch.float32).max
+    inf = 0
+    for g, w in zip(grads, wg):
+        assert not torch.isnan(g).any()
+        over, under = w.abs() > 1.001 * big, w.abs() < 0.999 * big
+        assert torch.equal(g[over], w[over].sign().float() * float("inf"))
+        assert torch.isfinite(g[under]).all()
+        ordinary = w.abs() < 2.0 ** 120
+        assert float((g.double() - w)[ordinary].norm() / w[ordinary].norm()) <= REL
+        inf += int(over.sum())
+    assert inf > 100
