@@ -89,3 +89,31 @@ def test_level2_equals_general_path(device, dtype, D, B, Lq, Lk, Hq, Hkv, qids, 
         assert np.isfinite(a).all()
         bound = step * (np.abs(b) + np.abs(b).max(initial=0.0))
         assert (np.abs(a - b) <= bound).all(), f"{name}: {np.abs(a - b).max()}"
+
+
+@pytest.mark.parametrize("dtype,D", [("f32", 64), ("f32", 128), ("bf16", 64), ("bf16", 128)])
+@pytest.mark.parametrize("cut", [1, 2, 3, 130, 133])
+def test_documents_start_anywhere(device, dtype, D, cut):
+    """A document whose first position is no multiple of 4, at a length that is:
+    the query range of a key block starts there, and the ids are read from it."""
+    import torch
+    from probjax_amd import hip_attention as hip
+
+    B, L, H = 1, 256, 2
+    tdt = torch.float32 if dtype == "f32" else torch.bfloat16
+    q, k, v, do = (to_dev(x, device, tdt) for x in rng_normal(83, *[(B, L, H, D)] * 4))
+    ids = (torch.arange(L, device=device) >= cut).to(torch.int32)[None]
+    # document by document, without ids, is the same computation
+    got, kw = {}, dict(sm_scale=1 / math.sqrt(D), causal=True)
+    for name, spans in (("ids", [(0, L)]), ("alone", [(0, cut), (cut, L)])):
+        parts = []
+        for a, b in spans:
+            x = [t[:, a:b].contiguous() for t in (q, k, v)]
+            m = hip.ScoreModsArgs(segment_q=ids, segment_k=ids) if name == "ids" else None
+            o, lse = hip.flash_attention_fwd(*x, return_lse=True, mods=m, **kw)
+            parts.append([o, *hip.flash_attention_bwd(*x, o, do[:, a:b].contiguous(), lse, mods=m, **kw)])
+        got[name] = [torch.cat(t, 1).double() for t in zip(*parts)]
+    # float32 sums in another order; one rounding step of bf16
+    tol = 32 * 2.0 ** -24 if dtype == "f32" else 2.0 ** -8
+    for a, b in zip(got["ids"], got["alone"]):
+        assert float((a - b).norm() / b.norm()) <= tol
