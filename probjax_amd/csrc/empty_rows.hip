@@ -63,6 +63,7 @@ struct EmptyArgs {
   void* dst;         // forward: O [B, Lq, Hq, D]; backward: dV [B, Lk, Hkv, D]
   int B, Lq, Lk, Hq, Hkv, D;
   int chunk;         // rows of dst per workgroup
+  int heads;         // (batch, head) pairs: B * Hq, or B * Hkv for the gradient
 };
 
 // A workgroup's columns: 64 bytes of a row in lanes of 16, or 64 single
@@ -114,7 +115,8 @@ __device__ __forceinline__ bool any_empty(const float* lse, long n) {
 }
 
 // Both kernels: one workgroup per (batch and head, chunk of the rows written,
-// 64-byte column group).  Without an empty row they end after reading the lse,
+// 64-byte column group), more heads than a launch's work-items count taken in
+// strides of the grid.  Without an empty row they end after reading the lse,
 // the usual call.  A batch padded on the query side has such rows in every
 // call; then each workgroup sums its columns of V (of the empty rows' dO)
 // itself, from L2 for all but the first, which needs no workspace and no second
@@ -131,33 +133,35 @@ __global__ __launch_bounds__(kEmptyThreads) void fill_empty_rows_kernel(EmptyArg
   using C = Columns<VE>;
   __shared__ float sums[C::N], part[kEmptyWaves][C::N];
   const int tid = threadIdx.x;
-  const int b = blockIdx.x / a.Hq, h = blockIdx.x % a.Hq, hkv = h / (a.Hq / a.Hkv);
-  const float* lse = a.lse + (size_t)blockIdx.x * a.Lq;
   const int r0 = blockIdx.y * a.chunk, r1 = min(r0 + a.chunk, a.Lq);
-  if (!__syncthreads_or(any_empty(lse + r0, r1 - r0) ? 1 : 0)) return;
   const int c = blockIdx.z * C::N + (tid % C::LPR) * VE;
   const bool in = c < a.D;
   const size_t vs = (size_t)a.Hkv * a.D, os = (size_t)a.Hq * a.D;
-  const typename E::T* v = (const typename E::T*)a.src + (size_t)b * a.Lk * vs + (size_t)hkv * a.D + c;
-  float acc[VE] = {};
-  if (in) {
+  for (uint32_t bh = blockIdx.x; bh < (uint32_t)a.heads; bh += gridDim.x) {
+    const int b = bh / a.Hq, h = bh % a.Hq, hkv = h / (a.Hq / a.Hkv);
+    const float* lse = a.lse + (size_t)bh * a.Lq;
+    if (!__syncthreads_or(any_empty(lse + r0, r1 - r0) ? 1 : 0)) continue;
+    const typename E::T* v = (const typename E::T*)a.src + (size_t)b * a.Lk * vs + (size_t)hkv * a.D + c;
+    float acc[VE] = {};
+    if (in) {
 #pragma unroll 8
-    for (int i = tid / C::LPR; i < a.Lk; i += C::ROWS) {
-      float x[VE];
-      E::load(v + i * vs, x);
+      for (int i = tid / C::LPR; i < a.Lk; i += C::ROWS) {
+        float x[VE];
+        E::load(v + i * vs, x);
 #pragma unroll
-      for (int e = 0; e < VE; ++e) acc[e] += x[e];
+        for (int e = 0; e < VE; ++e) acc[e] += x[e];
+      }
     }
-  }
-  add_columns<VE>(acc, part, sums);
-  if (!in) return;
-  const float inv = 1.f / a.Lk;
-  float mean[VE];
+    add_columns<VE>(acc, part, sums);
+    if (!in) continue;
+    const float inv = 1.f / a.Lk;
+    float mean[VE];
 #pragma unroll
-  for (int e = 0; e < VE; ++e) mean[e] = sums[(tid % C::LPR) * VE + e] * inv;
-  typename E::T* o = (typename E::T*)a.dst + (size_t)b * a.Lq * os + (size_t)h * a.D + c;
-  for (int i = r0 + tid / C::LPR; i < r1; i += C::ROWS)
-    if (__float_as_uint(lse[i]) == kPosInfBits) E::store(o + i * os, mean);
+    for (int e = 0; e < VE; ++e) mean[e] = sums[(tid % C::LPR) * VE + e] * inv;
+    typename E::T* o = (typename E::T*)a.dst + (size_t)b * a.Lq * os + (size_t)h * a.D + c;
+    for (int i = r0 + tid / C::LPR; i < r1; i += C::ROWS)
+      if (__float_as_uint(lse[i]) == kPosInfBits) E::store(o + i * os, mean);
+  }
 }
 
 // dV of every key gains the sum over the group's empty rows of dO, divided by
@@ -170,57 +174,60 @@ __global__ __launch_bounds__(kEmptyThreads) void empty_rows_grad_kernel(EmptyArg
   __shared__ float sums[C::N], part[kEmptyWaves][C::N];
   __shared__ int rows[kEmptyWaves][64];
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
-  const int b = blockIdx.x / a.Hkv, hkv = blockIdx.x % a.Hkv, G = a.Hq / a.Hkv;
+  const int G = a.Hq / a.Hkv;
   const long n = (long)G * a.Lq;  // the group's rows, one after the other in the lse
-  const float* lse = a.lse + ((size_t)b * a.Hq + (size_t)hkv * G) * a.Lq;
   const int c = blockIdx.z * C::N + (tid % C::LPR) * VE;
   const bool in = c < a.D;
   const size_t vs = (size_t)a.Hkv * a.D, ds = (size_t)a.Hq * a.D;
-  const typename E::T* d = (const typename E::T*)a.src + (size_t)b * a.Lq * ds + (size_t)hkv * G * a.D + c;
-  if (!__syncthreads_or(any_empty(lse, n) ? 1 : 0)) return;
-  float acc[VE] = {};
-  const int per_head = (a.Lq + 255) / 256;  // blocks of 256 rows of one head
-  for (int t = w; t < G * per_head; t += kEmptyWaves) {
-    const int g = t / per_head, i0 = t % per_head * 256;
-    bool empty[4];
+  for (uint32_t bh = blockIdx.x; bh < (uint32_t)a.heads; bh += gridDim.x) {
+    const int b = bh / a.Hkv, hkv = bh % a.Hkv;
+    const float* lse = a.lse + ((size_t)b * a.Hq + (size_t)hkv * G) * a.Lq;
+    const typename E::T* d = (const typename E::T*)a.src + (size_t)b * a.Lq * ds + (size_t)hkv * G * a.D + c;
+    if (!__syncthreads_or(any_empty(lse, n) ? 1 : 0)) continue;
+    float acc[VE] = {};
+    const int per_head = (a.Lq + 255) / 256;  // blocks of 256 rows of one head
+    for (int t = w; t < G * per_head; t += kEmptyWaves) {
+      const int g = t / per_head, i0 = t % per_head * 256;
+      bool empty[4];
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int i = i0 + 64 * j + lane;
-      empty[j] = i < a.Lq && __float_as_uint(lse[(size_t)g * a.Lq + i]) == kPosInfBits;
-    }
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const uint64_t m = __builtin_amdgcn_ballot_w64(empty[j]);
-      if (m == 0) continue;
-      if (empty[j]) rows[w][__builtin_popcountll(m & ((1ull << lane) - 1))] = i0 + 64 * j + lane;
-      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-      const int count = __builtin_popcountll(m);
-#pragma unroll 4
-      for (int k = lane / C::LPR; k < count; k += 64 / C::LPR) {
-        float x[VE];
-        if (in) {
-          E::load(d + rows[w][k] * ds + (size_t)g * a.D, x);
-#pragma unroll
-          for (int e = 0; e < VE; ++e) acc[e] += x[e];
-        }
+      for (int j = 0; j < 4; ++j) {
+        const int i = i0 + 64 * j + lane;
+        empty[j] = i < a.Lq && __float_as_uint(lse[(size_t)g * a.Lq + i]) == kPosInfBits;
       }
-      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const uint64_t m = __builtin_amdgcn_ballot_w64(empty[j]);
+        if (m == 0) continue;
+        if (empty[j]) rows[w][__builtin_popcountll(m & ((1ull << lane) - 1))] = i0 + 64 * j + lane;
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        const int count = __builtin_popcountll(m);
+#pragma unroll 4
+        for (int k = lane / C::LPR; k < count; k += 64 / C::LPR) {
+          float x[VE];
+          if (in) {
+            E::load(d + rows[w][k] * ds + (size_t)g * a.D, x);
+#pragma unroll
+            for (int e = 0; e < VE; ++e) acc[e] += x[e];
+          }
+        }
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      }
     }
-  }
-  add_columns<VE>(acc, part, sums);
-  if (!in) return;
-  const float inv = 1.f / a.Lk;
-  float total[VE];
+    add_columns<VE>(acc, part, sums);
+    if (!in) continue;
+    const float inv = 1.f / a.Lk;
+    float total[VE];
 #pragma unroll
-  for (int e = 0; e < VE; ++e) total[e] = sums[(tid % C::LPR) * VE + e];
-  typename E::T* dv = (typename E::T*)a.dst + (size_t)b * a.Lk * vs + (size_t)hkv * a.D + c;
-  const int r1 = min((int)(blockIdx.y + 1) * a.chunk, a.Lk);
-  for (int i = blockIdx.y * a.chunk + tid / C::LPR; i < r1; i += C::ROWS) {
-    float x[VE];
-    E::load(dv + i * vs, x);
+    for (int e = 0; e < VE; ++e) total[e] = sums[(tid % C::LPR) * VE + e];
+    typename E::T* dv = (typename E::T*)a.dst + (size_t)b * a.Lk * vs + (size_t)hkv * a.D + c;
+    const int r1 = min((int)(blockIdx.y + 1) * a.chunk, a.Lk);
+    for (int i = blockIdx.y * a.chunk + tid / C::LPR; i < r1; i += C::ROWS) {
+      float x[VE];
+      E::load(dv + i * vs, x);
 #pragma unroll
-    for (int e = 0; e < VE; ++e) x[e] = fmaf(total[e], inv, x[e]);
-    E::store(dv + i * vs, x);
+      for (int e = 0; e < VE; ++e) x[e] = fmaf(total[e], inv, x[e]);
+      E::store(dv + i * vs, x);
+    }
   }
 }
 
@@ -255,7 +262,9 @@ static int launch_empty(EmptyArgs a, bool grad, hipStream_t s) {
   const int groups = (a.D + Columns<VE>::N - 1) / Columns<VE>::N;
   const int64_t chunks = std::min(std::max<int64_t>(512 / (heads * groups), 1), (rows + 63) / 64);
   a.chunk = (int)((rows + chunks - 1) / chunks);
-  const dim3 grid((unsigned)heads, (unsigned)((rows + a.chunk - 1) / a.chunk), groups), block(kEmptyThreads);
+  a.heads = (int)heads;
+  const dim3 grid((unsigned)std::min<int64_t>(heads, 0xffffffffLL / kEmptyThreads),
+                  (unsigned)((rows + a.chunk - 1) / a.chunk), groups), block(kEmptyThreads);
   if (grad)
     launch_kernel<empty_rows_grad_kernel<DT, VE>>(grid, block, 0, s, a);
   else
@@ -284,7 +293,7 @@ extern "C" int pjx_empty_rows(int dtype, int grad, const float* lse, const void*
     return fail(PJX_ERR_INVALID, "pjx_empty_rows: sizes out of range");
   if (batch == 0 || q_len == 0 || kv_len == 0) return PJX_OK;
   if (!lse || !src || !dst) return fail(PJX_ERR_INVALID, "pjx_empty_rows: pointers must be non-null");
-  const EmptyArgs a = {lse, src, dst, (int)batch, (int)q_len, (int)kv_len, (int)q_heads, (int)kv_heads, (int)head_dim, 0};
+  const EmptyArgs a = {lse, src, dst, (int)batch, (int)q_len, (int)kv_len, (int)q_heads, (int)kv_heads, (int)head_dim, 0, 0};
   hipStream_t s = (hipStream_t)stream;
   if (dtype == PJX_DTYPE_F32) return launch_empty_rows<PJX_DTYPE_F32, 4>(a, grad != 0, s);
   return dtype == PJX_DTYPE_F16 ? launch_empty_rows<PJX_DTYPE_F16, 8>(a, grad != 0, s)

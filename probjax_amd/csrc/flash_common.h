@@ -27,6 +27,7 @@ struct FlashArgs {
   int rdim;     // elements per q / k / v / o row in memory: a multiple of 8, at most the kernel's head dim
   int ext;      // 0: none; 1: interval masks in `m`; 2: also segment ids / distance slopes; 3: all of `m`
   int f16;      // 16-bit inputs are fp16 (else bf16); read by the host-side launchers only
+  int block0 = 0;  // first block of this launch (launch_blocks; the kernels launched through it)
   ScoreMods m;
 };
 

@@ -40,7 +40,8 @@ __global__ __launch_bounds__(128 * QS, 2) void flash_dbias_kernel(DbiasArgs da) 
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int col = lane & 31, half = lane >> 5;
   const int nslice = da.bias_b * da.bias_h;
-  const int slice = blockIdx.x % nslice, tile = blockIdx.x / nslice;
+  const int block = a.block0 + blockIdx.x;
+  const int slice = block % nslice, tile = block / nslice;
   const int nkt = (a.Lk + 127) / 128;
   const int qt0 = (tile / nkt) * NQ, kt0 = (tile % nkt) * 128;
   const int strip = w % QS, kh = w / QS;
@@ -188,9 +189,9 @@ static int launch_dbias(const DbiasArgs& da, hipStream_t s) {
   const FlashArgs& a = da.w.f;
   const long blocks = (a.Lq + 32L * QS - 1) / (32 * QS) * ((a.Lk + 127L) / 128) * da.bias_b * da.bias_h;
   if (blocks > 0x7fffffffL) return fail(PJX_ERR_INVALID, "pjx_flash_dbias: grid too large");
-  const dim3 grid((unsigned)blocks), block(128 * QS);
-  if (a.ext) launch_kernel<flash_dbias_kernel<E, D, QS, true>>(grid, block, 0, s, da);
-  else launch_kernel<flash_dbias_kernel<E, D, QS, false>>(grid, block, 0, s, da);
+  auto first = [](DbiasArgs& x) -> int& { return x.w.f.block0; };
+  if (a.ext) launch_blocks<flash_dbias_kernel<E, D, QS, true>>(blocks, 128 * QS, s, da, first);
+  else launch_blocks<flash_dbias_kernel<E, D, QS, false>>(blocks, 128 * QS, s, da, first);
   return check_launch("pjx_flash_dbias");
 }
 

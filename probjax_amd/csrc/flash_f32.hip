@@ -37,7 +37,7 @@ __global__ __launch_bounds__(64 * RS * KG, WPE) void flash_fwd_f32_planes_kernel
   const int w8 = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int strip = w8 % RS, gi = w8 / RS;
   const int col = lane & 31, half = lane >> 5;
-  BlockGeom g = plane_geom(a, blockIdx.x, BQ, strip);
+  BlockGeom g = plane_geom(a, a.block0 + blockIdx.x, BQ, strip);
   if constexpr (EXT > 0) ext_block_range(a, g, 32, BQ);
   const int rdim = a.rdim;
   const uint32_t kv_row = (uint32_t)a.Hkv * rdim * 4;
@@ -309,8 +309,8 @@ static int launch_planes(FlashArgs a, hipStream_t s) {
   a.n_qtiles = (a.Lq + 32 * RS - 1) / (32 * RS);
   const long blocks = (long)a.n_qtiles * a.B * a.Hq;
   if (blocks > 0x7fffffffL) return fail(PJX_ERR_INVALID, "pjx_flash_fwd: grid too large");
-  launch_kernel<flash_fwd_f32_planes_kernel<D, RS, KG, NBUF, WPE, BIAS, EXT>>(dim3((unsigned)blocks), dim3(64 * RS * KG), 0, s,
-                                                                         a);
+  launch_blocks<flash_fwd_f32_planes_kernel<D, RS, KG, NBUF, WPE, BIAS, EXT>>(
+      blocks, 64 * RS * KG, s, a, [](FlashArgs& x) -> int& { return x.block0; });
   return check_launch("pjx_flash_fwd");
 }
 

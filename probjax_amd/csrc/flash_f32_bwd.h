@@ -43,7 +43,7 @@ __global__ __launch_bounds__(64 * RS * KG, WPE) void flash_bwd_dq_f32_planes_ker
   const int w8 = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int strip = w8 % RS, gi = w8 / RS;
   const int col = lane & 31, half = lane >> 5;
-  BlockGeom g = plane_geom(a, blockIdx.x, BQ, strip);
+  BlockGeom g = plane_geom(a, a.block0 + blockIdx.x, BQ, strip);
   if constexpr (EXT > 0) ext_block_range(a, g, 32, BQ);
   const int rdim = a.rdim;
   const uint32_t kv_row = (uint32_t)a.Hkv * rdim * 4;
@@ -347,8 +347,9 @@ __global__ __launch_bounds__(64 * KS * QG, WPE) void flash_bwd_dkdv_f32_planes_k
   const int col = lane & 31, half = lane >> 5;
   const int rdim = a.rdim;
   const int BH = a.B * a.Hkv;
-  const int bh = blockIdx.x % BH;
-  const int k0 = (blockIdx.x / BH) * BK;
+  const int block = a.block0 + blockIdx.x;
+  const int bh = block % BH;
+  const int k0 = (block / BH) * BK;
   const int b = bh / a.Hkv, hkv = bh % a.Hkv;
   const int G = a.Hq / a.Hkv;
   const int kw = k0 + 32 * strip;
@@ -688,8 +689,8 @@ static int launch_dq_planes(FlashBwdArgs a, hipStream_t s) {
   a.f.n_qtiles = (a.f.Lq + 32 * RS - 1) / (32 * RS);
   const long blocks = (long)a.f.n_qtiles * a.f.B * a.f.Hq;
   if (blocks > 0x7fffffffL) return fail(PJX_ERR_INVALID, "pjx_flash_bwd: grid too large");
-  launch_kernel<flash_bwd_dq_f32_planes_kernel<D, RS, KG, NBUF, WPE, BIAS, EXT>>(dim3((unsigned)blocks),
-                                                                                 dim3(64 * RS * KG), 0, s, a);
+  launch_blocks<flash_bwd_dq_f32_planes_kernel<D, RS, KG, NBUF, WPE, BIAS, EXT>>(
+      blocks, 64 * RS * KG, s, a, [](FlashBwdArgs& x) -> int& { return x.f.block0; });
   return check_launch("pjx_flash_bwd (dq)");
 }
 
@@ -697,8 +698,8 @@ template <int D, int KS, int QG, int WPE, bool VR, bool BIAS, int EXT>
 static int launch_dkdv_planes(const FlashBwdArgs& a, hipStream_t s) {
   const long blocks = (long)((a.f.Lk + 32 * KS - 1) / (32 * KS)) * a.f.B * a.f.Hkv;
   if (blocks > 0x7fffffffL) return fail(PJX_ERR_INVALID, "pjx_flash_bwd: grid too large");
-  launch_kernel<flash_bwd_dkdv_f32_planes_kernel<D, KS, QG, WPE, VR, BIAS, EXT>>(dim3((unsigned)blocks),
-                                                                                 dim3(64 * KS * QG), 0, s, a);
+  launch_blocks<flash_bwd_dkdv_f32_planes_kernel<D, KS, QG, WPE, VR, BIAS, EXT>>(
+      blocks, 64 * KS * QG, s, a, [](FlashBwdArgs& x) -> int& { return x.f.block0; });
   return check_launch("pjx_flash_bwd (dk, dv)");
 }
 

@@ -36,6 +36,18 @@ inline void launch_kernel(dim3 grid, dim3 block, size_t lds, hipStream_t stream,
   hipLaunchKernelGGL(K, grid, block, lds, stream, args...);
 }
 
+// Notes and enqueues a one-dimensional grid of `blocks` workgroups, in several
+// launches where its work-items are more than a launch's 32 bits count: the
+// kernel adds `first(args)`, set to each launch's first block, to blockIdx.x.
+template <auto K, typename Args, typename First>
+inline void launch_blocks(int64_t blocks, int threads, hipStream_t stream, Args args, First first) {
+  const int64_t most = 0xffffffffLL / threads;
+  for (int64_t b = 0; b < blocks; b += most) {
+    first(args) = (int)b;
+    launch_kernel<K>(dim3((unsigned)std::min(most, blocks - b)), dim3(threads), 0, stream, args);
+  }
+}
+
 inline int fail(int code, const char* msg) {
   set_error(msg);
   return code;
