@@ -131,7 +131,7 @@ def make_c1(dev, gen):
     nbytes = 4 * B * L * H * D * 4
     fn = lambda: flash_attention_fwd(q, k, v, sm_scale=1 / 8, causal=True)  # noqa: E731
     return dict(name="C1 causal fwd f32 B=1 H=4 L=512 D=64", fn=fn, flop=flop, bytes=nbytes,
-                bound="latency", dtype="f32", kernel="flash_fwd_f32_planes_kernel<64,1,4,1,1,false,0>")
+                bound="latency", dtype="f32", kernel="flash_fwd_f32_planes_kernel<64,1,4,1,1,false,0,false>")
 
 
 def make_c2(dev, gen):

@@ -5,6 +5,12 @@
 
 namespace pjx {
 
+// Whether the rows that one wave loads at once (wave_rows) lie further apart than
+// a buffer's 32-bit offsets reach: a few million heads.
+static bool rows_far(const FlashArgs& a, int head_dim) {
+  return (int64_t)a.Hkv * a.rdim * 4 * (512 / head_dim) > 0xffffffffLL;
+}
+
 // ---------------------------------------------------------------------------
 // One workgroup = RS * KG waves = 32 * RS query rows of one (batch, head);
 // wave (strip, group) owns rows 32 * strip .. and takes key block `group` of
@@ -21,8 +27,10 @@ namespace pjx {
 // MFMA peak of 157.  Not kept: S_{t+1} formed under stage t's softmax inside a
 // wave (needs more than 256 registers, 1.3-1.8x slower), three waves per SIMD
 // (spills, 1.4x slower), fixed wave priorities (1-2%).
+// FAR: rows_far, loads by 64-bit addresses (as a branch here they cost the small
+// causal call of (1, 4, 512, 64) 4%).
 // ---------------------------------------------------------------------------
-template <int D, int RS, int KG, int NBUF, int WPE, bool BIAS, int EXT>
+template <int D, int RS, int KG, int NBUF, int WPE, bool BIAS, int EXT, bool FAR = false>
 __global__ __launch_bounds__(64 * RS * KG, WPE) void flash_fwd_f32_planes_kernel(FlashArgs a) {
   constexpr int SK = 32 * KG, BQ = 32 * RS, NT = 64 * RS * KG;
   using T = PlaneTile<D, SK>;
@@ -40,7 +48,7 @@ __global__ __launch_bounds__(64 * RS * KG, WPE) void flash_fwd_f32_planes_kernel
   BlockGeom g = plane_geom(a, a.block0 + blockIdx.x, BQ, strip);
   if constexpr (EXT > 0) ext_block_range(a, g, 32, BQ);
   const int rdim = a.rdim;
-  const uint32_t kv_row = (uint32_t)a.Hkv * rdim * 4;
+  const typename std::conditional<FAR, size_t, uint32_t>::type kv_row = (size_t)a.Hkv * rdim * 4;
   const unsigned char* Kb = (const unsigned char*)a.k + ((size_t)g.b * a.Lk * a.Hkv + g.hkv) * rdim * 4;
   const unsigned char* Vb = (const unsigned char*)a.v + ((size_t)g.b * a.Lk * a.Hkv + g.hkv) * rdim * 4;
   const bool row_in = g.qi < a.Lq;
@@ -100,6 +108,18 @@ __global__ __launch_bounds__(64 * RS * KG, WPE) void flash_fwd_f32_planes_kernel
 #pragma unroll
     for (int i = 0; i < PER; ++i) {
       const int row = k0 + (64 * w8 + NT * i) % NCH / T::NC;
+      if constexpr (FAR) {
+        const int r = row + lane / T::NC, c = lane % T::NC;
+        f32x4 x = {0.f, 0.f, 0.f, 0.f}, y = x;
+        if (r < g.kv_stop && 8 * c < rdim) {
+          const f32x4* p = (const f32x4*)((is_v(i) ? Vb : Kb) + r * kv_row + 32 * c);
+          x = p[0];
+          y = p[1];
+        }
+        *(f32x4*)reg[i] = x;
+        *(f32x4*)(reg[i] + 4) = y;
+        continue;
+      }
       const rsrc_t r = wave_rows<D>(is_v(i) ? Vb : Kb, row, g.kv_stop, kv_row, rdim);
       *(f32x4*)reg[i] = buffer_load_f32x4(r, goff);
       *(f32x4*)(reg[i] + 4) = buffer_load_f32x4(r, goff + 16);
@@ -304,12 +324,12 @@ __global__ __launch_bounds__(64 * RS * KG, WPE) void flash_fwd_f32_planes_kernel
   }
 }
 
-template <int D, int RS, int KG, int NBUF, int WPE, bool BIAS, int EXT>
+template <int D, int RS, int KG, int NBUF, int WPE, bool BIAS, int EXT, bool FAR = false>
 static int launch_planes(FlashArgs a, hipStream_t s) {
   a.n_qtiles = (a.Lq + 32 * RS - 1) / (32 * RS);
   const long blocks = (long)a.n_qtiles * a.B * a.Hq;
   if (blocks > 0x7fffffffL) return fail(PJX_ERR_INVALID, "pjx_flash_fwd: grid too large");
-  launch_blocks<flash_fwd_f32_planes_kernel<D, RS, KG, NBUF, WPE, BIAS, EXT>>(
+  launch_blocks<flash_fwd_f32_planes_kernel<D, RS, KG, NBUF, WPE, BIAS, EXT, FAR>>(
       blocks, 64 * RS * KG, s, a, [](FlashArgs& x) -> int& { return x.block0; });
   return check_launch("pjx_flash_fwd");
 }
@@ -347,6 +367,8 @@ static int launch_f32(const FlashArgs& a, hipStream_t s) {
 
 template <int D, bool BIAS>
 static int launch_f32_ext(const FlashArgs& a, hipStream_t s) {
+  // the general level covers the others
+  if (rows_far(a, D)) return launch_planes<D, 2, D == 64 ? 4 : 2, 1, D == 64 ? 2 : 1, BIAS, 3, true>(a, s);
   switch (a.ext) {
     case 0: return launch_f32<D, BIAS, 0>(a, s);
     case 1: return launch_f32<D, BIAS, 1>(a, s);

@@ -87,3 +87,20 @@ def test_rows_without_a_key(device):
     hip.empty_rows(lse, out, dv, grad=True)
     want = (v.float() + out.float() / 2).bfloat16()
     assert torch.equal(dv[empty], want[empty]) and torch.equal(dv[~empty], v[~empty])
+
+
+def test_float32_row_of_many_heads(device):
+    """Rows of all heads so long that 8 of them are more than 32-bit offsets hold."""
+    import torch
+    from probjax_amd.hip_attention import flash_attention_fwd
+
+    D, L, H = 64, 10, (1 << 21) + (1 << 19)
+    q, k, v = _randn(device, torch.float32, (1, 1, H, D), (1, L, H, D), (1, L, H, D))
+    kw = dict(sm_scale=D ** -0.5)
+    print("float32, 2.6 million heads", flush=True)
+    lengths = torch.tensor([L - 1], dtype=torch.int32, device=device)
+    o = flash_attention_fwd(q, k, v, kv_lengths=lengths, **kw)
+    for e in (slice(0, 500), slice(H // 2, H // 2 + 500), slice(H - 500, H)):
+        x = [t[0, :L - 1, e].transpose(0, 1).double() for t in (q, k, v)]
+        s = torch.matmul(x[1], x[0].transpose(1, 2)) * D ** -0.5
+        assert _rel(o[0, 0, e], (torch.softmax(s, 1) * x[2]).sum(1)) <= 32 * 2.0 ** -24
