@@ -25,10 +25,11 @@
 // dS, whose planes are an infinity and NaNs, NaN for an infinity.  Between
 // kSureMin and kSureMax (scale within 2^10 of 1) no operands can do so: dS K and
 // dS Q stay below 2^110 a term, and dP's own float32 rounding is above the 2^-134
-// that a plane may lose.  Tiles with other operands look at w itself, and where a
-// lane's largest is above kPlaneMax or below kScoreGradMin the products of dS
-// take the float32 MFMAs.  A look at w in every tile made a training step of
-// (B, H, L, D) = (4, 8, 1024, 64) 2.5% slower, this 1.4%, less than two runs differ.
+// that a plane may lose.  Tiles with other operands look at dP and delta, and
+// where a lane's largest, times scale, is above kPlaneMax or below kScoreGradMin
+// the products of P and dS take the float32 MFMAs.  Backward of (B, H, L, D), us
+// without this and with it: (4, 8, 1024, 64) 124 -> 125, (4, 8, 1024, 128) 277
+// -> 279, (4, 8, 2048, 128) 786 -> 805.
 #pragma once
 
 #include "flash_common.h"
@@ -108,12 +109,11 @@ __device__ __forceinline__ bool scale_beyond_sure(float scale) {
   return !(fabsf(scale) <= kSureScale && fabsf(scale) >= 1.f / kSureScale);
 }
 
-// Whether the dS of any lane of the wave is, whose 16 w are scale (dp - delta[r]).
-template <typename F>
-__device__ __forceinline__ bool score_grads_beyond_planes(const f32x16& dp, float scale, F delta) {
-  float m = 0.f;
+// Whether the dS of any lane of the wave is: its 16 dP and delta, times scale.
+__device__ __forceinline__ bool score_grads_beyond_planes(const f32x16& dp, float delta, float scale) {
+  float m = fabsf(delta);
 #pragma unroll
-  for (int r = 0; r < 16; ++r) m = fmaxf(m, fabsf(dp[r] - delta(r)));
+  for (int r = 0; r < 16; ++r) m = fmaxf(m, fabsf(dp[r]));
   m *= fabsf(scale);
   return wave_any(m > kPlaneMax || (m > 0.f && m < kScoreGradMin));
 }

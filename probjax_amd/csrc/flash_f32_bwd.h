@@ -193,7 +193,7 @@ __global__ __launch_bounds__(64 * RS * KG, WPE) void flash_bwd_dq_f32_planes_ker
       }
     }
     bool ds_wild = wild;
-    if (!sure && !wild) ds_wild = score_grads_beyond_planes(dp[0], wscale, [&](int) { return delta; });
+    if (!sure && !wild) ds_wild = score_grads_beyond_planes(dp[0], delta, wscale);
     f32x16 dbv[1];
     if constexpr (EXT == 3) {
       ext_scores_sT<1, HB>(a, g, er, s, k0, half, brow, row_in, [&](int kb, int r, float x, float gg) {
@@ -531,8 +531,8 @@ __global__ __launch_bounds__(64 * KS * QG, WPE) void flash_bwd_dkdv_f32_planes_k
       }
     }
     bool ds_wild = wild;
-    if (!sure && !wild)  // the rows hold delta * sm_scale
-      ds_wild = score_grads_beyond_planes(dp * a.scale, hscale, [&](int r) { return dlm[8 * (r >> 2) + 4 * half + (r & 3)]; });
+    if (!sure && !wild)  // one row's delta * sm_scale a lane
+      ds_wild = score_grads_beyond_planes(dp, dlm[col] / a.scale, a.scale * hscale);
     if constexpr (EXT == 3) {
       const float* bbase = nullptr;
       if constexpr (BIAS) bbase = a.bias + (size_t)b * a.bias_bstride + (size_t)h * a.bias_hstride;
@@ -581,7 +581,7 @@ __global__ __launch_bounds__(64 * KS * QG, WPE) void flash_bwd_dkdv_f32_planes_k
       }
     }
     // dV^T[d][key] += dO^T P and dK^T[d][key] += Q^T dS
-    if (!wild) {
+    if (!ds_wild) {
 #pragma unroll
       for (int c = 0; c < 2; ++c) {
         const Planes p = planes_step(s, c);
@@ -590,19 +590,6 @@ __global__ __launch_bounds__(64 * KS * QG, WPE) void flash_bwd_dkdv_f32_planes_k
           accv[db] = mma_planes(T::cols(dt, 32 * gi + 16 * c, off.tlo[db], off.thi[db]), p, accv[db]);
         __builtin_amdgcn_sched_barrier(0);
       }
-    } else {
-#pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const int qq = q0 + 8 * (r >> 2) + 4 * half + (r & 3);
-        const bool qin = qq < a.Lq;
-        const size_t qo = (size_t)(qin ? qq : 0) * a.Hq * rdim + col;
-#pragma unroll
-        for (int db = 0; db < D / 32; ++db)
-          accv[db] = mfma32x32x2f32(qin && db * 32 + col < rdim ? Dg[qo + db * 32] : 0.f, s[r], accv[db]);
-        __builtin_amdgcn_sched_barrier(0);
-      }
-    }
-    if (!ds_wild) {
 #pragma unroll
       for (int c = 0; c < 2; ++c) {
         const Planes p = planes_step(dp, c);
@@ -618,8 +605,11 @@ __global__ __launch_bounds__(64 * KS * QG, WPE) void flash_bwd_dkdv_f32_planes_k
         const bool qin = qq < a.Lq;
         const size_t qo = (size_t)(qin ? qq : 0) * a.Hq * rdim + col;
 #pragma unroll
-        for (int db = 0; db < D / 32; ++db)
-          acck[db] = mfma32x32x2f32(qin && db * 32 + col < rdim ? Qg[qo + db * 32] : 0.f, dp[r], acck[db]);
+        for (int db = 0; db < D / 32; ++db) {
+          const bool in = qin && db * 32 + col < rdim;
+          accv[db] = mfma32x32x2f32(in ? Dg[qo + db * 32] : 0.f, s[r], accv[db]);
+          acck[db] = mfma32x32x2f32(in ? Qg[qo + db * 32] : 0.f, dp[r], acck[db]);
+        }
         __builtin_amdgcn_sched_barrier(0);
       }
     }
