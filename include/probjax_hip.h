@@ -227,8 +227,10 @@ size_t pjx_flash_bwd_split_workspace_size(int dtype, int64_t batch, int64_t q_he
  * forward's (pjx_score_mods) or NULL.  A workspace of at least
  * pjx_flash_bwd_ds_workspace_size() bytes selects the dS route where it applies,
  * one of pjx_flash_bwd_split_workspace_size() bytes the split key blocks.
- * dtype: PJX_DTYPE_BF16, PJX_DTYPE_F16 or PJX_DTYPE_F32 (all fp32 products, no
- * roundings).  head_dim in {64, 128, 256}.
+ * dtype: PJX_DTYPE_BF16, PJX_DTYPE_F16 or PJX_DTYPE_F32 (nothing is rounded
+ * below fp32: at head_dim 64 and 128 a value is the sum of three bf16 values and
+ * a product their six largest products, at 256 an fp32 product).  head_dim in
+ * {64, 128, 256}.
  */
 int pjx_flash_bwd(int dtype, const void* q, const void* k, const void* v, const void* o,
                   const void* dout, const float* lse, void* dq, void* dk, void* dv,

@@ -127,6 +127,8 @@ __device__ __forceinline__ bool any_empty(const float* lse, long n) {
 //                                      gradient 2.6 / 125 / 180 -> 2.7 / 7.7 / 9.8
 //   bf16 B=1 L=4096 H=32 Hkv=1 D=128:  fill 3.5 / 418 / 791 -> 2.3 / 9.3 / 16.5
 //                                      gradient 57 / 8910 / 33306 -> 6.4 / 148 / 478
+// (Calls after one another; between a training step's other kernels the first
+// shape's 2.2 and 2.7 without an empty row are 3.9 and 4.6.)
 template <int DT, int VE>
 __global__ __launch_bounds__(kEmptyThreads) void fill_empty_rows_kernel(EmptyArgs a) {
   typedef Elems<DT, VE> E;
@@ -235,7 +237,9 @@ __global__ __launch_bounds__(kEmptyThreads) void empty_rows_grad_kernel(EmptyArg
 // rows, blockIdx.z 0 and 1.  One pass over memory, 16 bytes a lane (a row of any
 // kernel's head dim is whole 16-byte chunks), indexed in 32 bits within a batch
 // entry.  A step over 2x2048x8x64 in bf16 with a learned bias: 350 us with torch
-// operations (compare, two selects by row) here, 319 with this kernel.
+// operations (compare, two selects by row) here, 319 with this kernel.  The
+// copies are made in every backward after a fill, whether or not such a row
+// exists: 5.4 us of that step.
 struct ZeroArgs {
   const float* lse;     // [B, Hq, Lq]
   const u32x4* src[2];  // [B, Lq, Hq, per]

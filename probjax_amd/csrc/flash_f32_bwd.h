@@ -6,9 +6,9 @@
 // units in turn.  The workgroup shapes follow the forward's: by the number of
 // 128-row tiles (128-key blocks), at most one per CU or more.  us per backward,
 // float32 MFMA kernels before -> chosen, other shapes (B, H, L, D causal):
-//   (1,4,512,64)   138 -> 1x4 50, 2x4 57       (4,8,1024,64) 272 -> 2x4 130, 4x2 148
+//   (1,4,512,64)   138 -> 1x4 50, 2x4 57       (4,8,1024,64) 272 -> 2x4 125, 4x2 148
 //   (4,8,2048,64)  743 -> 4x2 345, 2x4 409     (4,16,2048,64 full) 1870 -> 4x2 1220
-//   (4,8,1024,128) 540 -> 2x2 283, 4x1 370     (4,8,2048,128) 1092 -> 4x1 785, 2x2 984
+//   (4,8,1024,128) 540 -> 2x2 279, 4x1 370     (4,8,2048,128) 1092 -> 4x1 805, 2x2 984
 // Relative errors against float64 at (4,8,1024,64): dq, dk 4.8e-7 -> 3.6e-7,
 // dv 4.0e-7 -> 3.1e-7.
 #pragma once

@@ -641,12 +641,11 @@ __global__ __launch_bounds__(G * kThreads, WPC) void flash_fwd_bf16_pipe_kernel(
 // contiguous half row of K, and the step of P.V pairs key (r, half 0) with key
 // (r, half 1) of the S^T layout, so V is read in its natural layout.
 // ---------------------------------------------------------------------------
-template <int D>
-constexpr int split_waves() { return 4; }
+constexpr int kSplitWaves = 4;
 
 template <int D, bool BIAS>
-__global__ __launch_bounds__(64 * split_waves<D>(), 1) void flash_fwd_f32_split_kernel(FlashArgs a) {
-  constexpr int NW = split_waves<D>();
+__global__ __launch_bounds__(64 * kSplitWaves, 1) void flash_fwd_f32_split_kernel(FlashArgs a) {
+  constexpr int NW = kSplitWaves;
   constexpr int DH = D / 2;          // floats per half row
   constexpr int OS = D + 4;          // combine row stride (floats)
   __shared__ __attribute__((aligned(16))) float red_o[NW * 32 * OS];
@@ -883,7 +882,7 @@ template <int D, auto K>
 static int launch_split(const FlashArgs& a, hipStream_t stream) {
   const long blocks = (long)((a.Lq + 31) / 32) * a.B * a.Hq;
   if (blocks > 0x7fffffffL) return fail(PJX_ERR_INVALID, "pjx_flash_fwd: grid too large");
-  launch_kernel<K>(dim3((unsigned)blocks), dim3(64 * split_waves<D>()), 0, stream, a);
+  launch_kernel<K>(dim3((unsigned)blocks), dim3(64 * kSplitWaves), 0, stream, a);
   return check_launch("pjx_flash_fwd");
 }
 
