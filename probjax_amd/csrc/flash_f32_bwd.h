@@ -516,7 +516,7 @@ __global__ __launch_bounds__(64 * KS * QG, WPE) void flash_bwd_dkdv_f32_planes_k
     if (!wild) {
 #pragma unroll
       for (int st = 0; st < D / 16; ++st) {
-        s = mma_planes(T::rows(qt, 32 * gi, off.row[st]), kfrag(st), s);
+        s = mma_planes<true>(T::rows(qt, 32 * gi, off.row[st]), kfrag(st), s);
         dp = mma_planes(T::rows(dt, 32 * gi, off.row[st]), vfrag(st), dp);
         __builtin_amdgcn_sched_barrier(0);
       }

@@ -246,3 +246,27 @@ def test_large_score_gradients(device, D, H, bias):
         assert float((g.double() - w)[ordinary].norm() / w[ordinary].norm()) <= REL
         inf += int(over.sum())
     assert inf > 100
+
+
+@pytest.mark.parametrize("D,H", [(64, 2), (64, 70), (64, 300), (128, 2), (128, 300)])
+def test_one_p_in_both_kernels(device, D, H):
+    """The dK/dV kernel's P is the dQ kernel's, bit for bit, also where scores of
+    a hundred leave a P fewer digits: with dP = 1, no delta and dO in one
+    row, the bias gradient is the one and dV the other."""
+    import torch
+    from probjax_amd.hip_attention import flash_attention_bwd, flash_attention_fwd
+
+    L, row = 129, 77
+    q, k = (to_dev(x, device, torch.float32) for x in rng_normal(98, *[(1, L, H, D)] * 2))
+    q *= 20
+    v, do = torch.zeros_like(k), torch.zeros_like(q)
+    v[..., 0] = 1
+    do[0, row, :, 0] = 1
+    kw = dict(sm_scale=1 / math.sqrt(D), bias=torch.zeros(1, 1, L, L, device=device))
+    _, lse = flash_attention_fwd(q, k, v, return_lse=True, **kw)
+    grads = flash_attention_bwd(q, k, v, torch.zeros_like(q), do, lse, bias_grad=True, **kw)
+    p = grads[2][0, :, :, 0].t()
+    kw["bias"] = kw["bias"].expand(1, H, L, L).contiguous()  # a gradient for every head
+    db = flash_attention_bwd(q, k, v, torch.zeros_like(q), do, lse, bias_grad=True, **kw)[3][0, :, row]
+    seen = db > 2.0 ** -100  # below, a P is no sum of three planes
+    assert seen.sum() > 40 * H and torch.equal(p[seen], db[seen])
